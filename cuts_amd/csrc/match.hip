@@ -47,16 +47,30 @@
 
 #include "batch.hpp"
 
+// The library builds this file as four objects side by side, since the
+// chain level's unrolled closed form takes the compiler as long as all else
+// together: parts 1 to 3 hold that level's kernels, part 0 the rest and the
+// host code.  Without CUTS_MATCH_PART the file is one object.
+#if !defined(CUTS_MATCH_PART) || CUTS_MATCH_PART == 0
+#define CUTS_MATCH_HOST 1
+#else
+#define CUTS_MATCH_HOST 0
+#endif
+
 // Scratch of the no-allocation entry point (run_match_noalloc): every
 // buffer of such a run -- trie levels, scans, counters, degree tables the
 // graph has not cached -- is carved from this array.  Each device holds its
 // own copy for the life of the process.  Host code never passes this name
 // to a kernel: it is a host-side stand-in; the device address comes from
 // hipGetSymbolAddress (scratch_address below).
+#if CUTS_MATCH_HOST
 constexpr uint64_t kScratchBytes = 256ull << 20;
 static __device__ __align__(256) unsigned char scratch[kScratchBytes];
+#endif
 
 namespace cuts {
+
+#if CUTS_MATCH_HOST
 
 // The device address of this device's scratch array, looked up once per
 // device with that device current (context_init calls it).
@@ -77,8 +91,13 @@ char* scratch_address(int device) {
 void hip_check(hipError_t e, const char* what) {
   if (e != hipSuccess) throw Error(-4, std::string(what) + ": " + hipGetErrorString(e));
 }
+#endif
 
+#ifdef CUTS_MATCH_PART
+inline namespace kernels {  // with linkage: instantiated in one part, launched from another
+#else
 namespace {
+#endif
 
 constexpr int BLOCK = 256;  // 4 wave64s
 constexpr int IPT = 4;      // work items per thread per tile
@@ -101,10 +120,10 @@ constexpr int LDS_OFF = 2048;      // staged work offsets per tile
 #endif
 constexpr int SCAN_IPT = 8;
 constexpr int SCAN_TILE = BLOCK * SCAN_IPT;
-constexpr uint64_t MAX_CHUNK = 1ull << 31;  // work items per launch sequence (written rows stay below 2^32)
+[[maybe_unused]] constexpr uint64_t MAX_CHUNK = 1ull << 31;  // work items per launch sequence (written rows stay below 2^32)
 // work items of one speculative counting launch (counts, offsets and tile
 // numbers are 64-bit; the tile index of such a level is at most 1 GiB)
-constexpr uint64_t MAX_SPEC_ITEMS = 1ull << 38;
+[[maybe_unused]] constexpr uint64_t MAX_SPEC_ITEMS = 1ull << 38;
 
 struct GView {
   const uint32_t *off_out, *adj_out, *off_in, *adj_in, *sig;
@@ -122,7 +141,7 @@ struct GView {
   const uint16_t* hr;      // hub rows: row r = |N(hub_r) & N(v)| for every v (V uint16)
 };
 
-GView view_of(const DeviceGraph& dg) {
+inline GView view_of(const DeviceGraph& dg) {
   return GView{dg.off_out, dg.adj_out, dg.off_in, dg.adj_in, dg.sig, dg.V, dg.hub_id, dg.nsig_out, dg.nsig_in, dg.bits,
                dg.words, dg.h2_off, dg.h2_v, dg.h2_c, dg.h2_did, dg.h2_dense, dg.arc_cn, dg.hr_id, dg.hr};
 }
@@ -225,7 +244,7 @@ __device__ __forceinline__ uint32_t arc_common(const GView& g, uint32_t u, uint3
 // membership test in the longer one (a bit test when it belongs to a hub),
 // stored at (u, w) and at the mirror arc (w, u).  One thread per arc; the
 // arc's source is found by an upper-bound search of the offsets.
-__global__ __launch_bounds__(256) void k_arc_common(GView g, uint64_t A, uint32_t* __restrict__ cn) {
+static __global__ __launch_bounds__(256) void k_arc_common(GView g, uint64_t A, uint32_t* __restrict__ cn) {
   for (uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x; i < A; i += (uint64_t)gridDim.x * 256) {
     uint32_t lo = 0, hi = g.V;  // largest u with off[u] <= i
     while (lo < hi) {
@@ -252,7 +271,7 @@ __global__ __launch_bounds__(256) void k_arc_common(GView g, uint64_t A, uint32_
 }
 
 // One block per hub: sets the bits of its neighbours.
-__global__ __launch_bounds__(256) void k_hub_bits(const uint32_t* __restrict__ off, const uint32_t* __restrict__ adj,
+static __global__ __launch_bounds__(256) void k_hub_bits(const uint32_t* __restrict__ off, const uint32_t* __restrict__ adj,
                                                   const uint32_t* __restrict__ hubs, uint32_t nh, uint32_t words,
                                                   uint64_t* __restrict__ bits) {
   for (uint32_t h = blockIdx.x; h < nh; h += gridDim.x) {
@@ -284,7 +303,7 @@ __device__ __forceinline__ void add_wave(unsigned long long* dst, uint64_t v) {
 // Level 0 in ascending vertex order: a 0/1 flag per candidate vertex, an
 // exclusive scan of the flags, and a scatter.  A deterministic level 0 makes
 // a run stopped between trunks correspond to an exact root range.
-__global__ __launch_bounds__(BLOCK) void k_level0_flags(const uint32_t* __restrict__ sig, uint32_t tin,
+static __global__ __launch_bounds__(BLOCK) void k_level0_flags(const uint32_t* __restrict__ sig, uint32_t tin,
                                                        uint32_t tout, uint32_t rb, uint32_t re, uint32_t rs,
                                                        uint32_t n, uint32_t* __restrict__ flags) {
   for (uint64_t i = (uint64_t)blockIdx.x * BLOCK + threadIdx.x; i < n; i += (uint64_t)gridDim.x * BLOCK) {
@@ -293,7 +312,7 @@ __global__ __launch_bounds__(BLOCK) void k_level0_flags(const uint32_t* __restri
   }
 }
 
-__global__ __launch_bounds__(BLOCK) void k_level0_scatter(const uint32_t* __restrict__ flags,
+static __global__ __launch_bounds__(BLOCK) void k_level0_scatter(const uint32_t* __restrict__ flags,
                                                          const uint64_t* __restrict__ pos, uint32_t rb, uint32_t rs,
                                                          uint32_t n, uint32_t* __restrict__ out) {
   for (uint64_t i = (uint64_t)blockIdx.x * BLOCK + threadIdx.x; i < n; i += (uint64_t)gridDim.x * BLOCK)
@@ -308,7 +327,7 @@ __global__ __launch_bounds__(BLOCK) void k_level0_scatter(const uint32_t* __rest
 // the same order.  The total goes to *total in host memory (a system-scope
 // store).
 constexpr uint32_t L0_THREADS = 1024;
-__global__ __launch_bounds__(L0_THREADS) void k_level0_small(const uint32_t* __restrict__ sig, uint32_t tin,
+static __global__ __launch_bounds__(L0_THREADS) void k_level0_small(const uint32_t* __restrict__ sig, uint32_t tin,
                                                             uint32_t tout, uint32_t rb, uint32_t re, uint32_t rs,
                                                             uint32_t n, uint32_t* __restrict__ out, uint64_t* total,
                                                             unsigned long long* __restrict__ dev_total) {
@@ -354,7 +373,7 @@ __global__ __launch_bounds__(L0_THREADS) void k_level0_small(const uint32_t* __r
 // rows0[lvcnt[0] - 1] when level 0's size stayed on the device), and the
 // device-side level counts (16 words, to pub[48..]), written to host memory
 // (system-scope stores) for one synchronisation with no copy.
-__global__ void k_publish_end(const unsigned long long* __restrict__ ctr, const uint32_t* __restrict__ last,
+static __global__ void k_publish_end(const unsigned long long* __restrict__ ctr, const uint32_t* __restrict__ last,
                               const uint32_t* __restrict__ rows0, const unsigned long long* __restrict__ lvcnt,
                               uint64_t* pub) {
   const uint32_t t = threadIdx.x;
@@ -549,7 +568,7 @@ __device__ __forceinline__ uint64_t block_excl_scan(uint64_t v, uint64_t* s_tmp,
   return wpre + inc - v;
 }
 
-__global__ __launch_bounds__(BLOCK) void k_scan_reduce(const uint32_t* __restrict__ in, uint64_t n,
+static __global__ __launch_bounds__(BLOCK) void k_scan_reduce(const uint32_t* __restrict__ in, uint64_t n,
                                                       uint64_t* __restrict__ bsum) {
   __shared__ uint64_t s_tmp[BLOCK / 64];
   const uint64_t base = (uint64_t)blockIdx.x * SCAN_TILE;
@@ -565,7 +584,7 @@ __global__ __launch_bounds__(BLOCK) void k_scan_reduce(const uint32_t* __restric
 }
 
 // single block: exclusive scan of bsum[0..nb) in place; bsum[nb] = total
-__global__ __launch_bounds__(BLOCK) void k_scan_partials(uint64_t* __restrict__ bsum, uint64_t nb) {
+static __global__ __launch_bounds__(BLOCK) void k_scan_partials(uint64_t* __restrict__ bsum, uint64_t nb) {
   __shared__ uint64_t s_tmp[BLOCK / 64];
   uint64_t carry = 0;
   for (uint64_t b0 = 0; b0 < nb; b0 += BLOCK) {
@@ -579,7 +598,7 @@ __global__ __launch_bounds__(BLOCK) void k_scan_partials(uint64_t* __restrict__ 
   if (threadIdx.x == 0) bsum[nb] = carry;
 }
 
-__global__ __launch_bounds__(BLOCK) void k_scan_down(const uint32_t* __restrict__ in, uint64_t n,
+static __global__ __launch_bounds__(BLOCK) void k_scan_down(const uint32_t* __restrict__ in, uint64_t n,
                                                     const uint64_t* __restrict__ bsum, uint64_t nb,
                                                     uint64_t* __restrict__ out) {
   __shared__ uint64_t s_tmp[BLOCK / 64];
@@ -608,8 +627,8 @@ __global__ __launch_bounds__(BLOCK) void k_scan_down(const uint32_t* __restrict_
 // tiles: each block sums the tile totals before it itself (a block-wide
 // reduction of at most that many words), and the last block writes the
 // total.
-constexpr uint64_t SCAN_FUSE_BLOCKS = 1024;
-__global__ __launch_bounds__(BLOCK) void k_scan_down_fused(const uint32_t* __restrict__ in, uint64_t n,
+[[maybe_unused]] constexpr uint64_t SCAN_FUSE_BLOCKS = 1024;
+static __global__ __launch_bounds__(BLOCK) void k_scan_down_fused(const uint32_t* __restrict__ in, uint64_t n,
                                                           const uint64_t* __restrict__ bsum, uint64_t nb,
                                                           uint64_t* __restrict__ out) {
   __shared__ uint64_t s_tmp[BLOCK / 64];
@@ -640,7 +659,7 @@ __global__ __launch_bounds__(BLOCK) void k_scan_down_fused(const uint32_t* __res
 
 // Levels of at most SCAN_TILE rows: the whole exclusive scan in one block
 // (out[0..n] with out[n] the total), one launch instead of three.
-__global__ __launch_bounds__(BLOCK) void k_scan_single(const uint32_t* __restrict__ in, uint64_t n,
+static __global__ __launch_bounds__(BLOCK) void k_scan_single(const uint32_t* __restrict__ in, uint64_t n,
                                                       uint64_t* __restrict__ out) {
   __shared__ uint64_t s_tmp[BLOCK / 64];
   uint32_t v[SCAN_IPT];
@@ -666,7 +685,7 @@ __global__ __launch_bounds__(BLOCK) void k_scan_single(const uint32_t* __restric
 // tile_p[ntiles] = prefix owning item w_end-1.  Block 0 also clears the
 // counters the expansion that follows starts from (its eight tile counters
 // and, when given, its output row counter), which saves a fill launch each.
-__global__ __launch_bounds__(BLOCK) void k_tile_index(const uint64_t* __restrict__ off, uint64_t n, uint64_t w_begin,
+static __global__ __launch_bounds__(BLOCK) void k_tile_index(const uint64_t* __restrict__ off, uint64_t n, uint64_t w_begin,
                                                      uint64_t w_end, uint64_t ntiles, uint32_t* __restrict__ tile_p,
                                                      unsigned int* __restrict__ tilectr,
                                                      unsigned int* __restrict__ outctr) {
@@ -701,7 +720,7 @@ __device__ __forceinline__ void publish_rows(uint64_t* publish, uint32_t rows, u
 // expansion that reads dyn does nothing -- and bit 0 of *status is set, for
 // the host to redo the level with the work it then reads back.  Block 0 also
 // clears the expansion's counters, as k_tile_index does.
-__global__ __launch_bounds__(BLOCK) void k_tile_index_dyn(const uint64_t* __restrict__ off, uint64_t n,
+static __global__ __launch_bounds__(BLOCK) void k_tile_index_dyn(const uint64_t* __restrict__ off, uint64_t n,
                                                          uint64_t max_items, uint64_t tile_cap, uint64_t row_cap,
                                                          uint32_t* __restrict__ tile_p,
                                                          unsigned int* __restrict__ tilectr,
@@ -969,7 +988,7 @@ __global__ __launch_bounds__(BLOCK) void k_closed_form(GView g, KPlan P, const u
 }
 
 // Degree-threshold table: tbl[u] = |{x in N(u) : deg(x) >= thr}|, one wave per vertex.
-__global__ __launch_bounds__(BLOCK) void k_cnt_table(GView g, uint32_t thr, uint32_t* __restrict__ tbl) {
+static __global__ __launch_bounds__(BLOCK) void k_cnt_table(GView g, uint32_t thr, uint32_t* __restrict__ tbl) {
   const uint32_t lane = threadIdx.x & 63;
   const uint64_t nw = (uint64_t)gridDim.x * (BLOCK / 64);
   for (uint64_t u = (uint64_t)blockIdx.x * (BLOCK / 64) + (threadIdx.x >> 6); u < g.V; u += nw) {
@@ -2128,7 +2147,7 @@ __global__ __launch_bounds__(BLOCK) void k_chain_shared_h2(GView g, KPlan P, con
 // Chain tables for thresholds (ta, tb): H[u] = sum over x in N(u) with
 // deg(x) >= ta of |{y in N(x) : deg(y) >= tb}|, H[V + u] = sum of those
 // deg(x).  One wave per vertex.
-__global__ __launch_bounds__(BLOCK) void k_chain_table(GView g, uint32_t ta, const uint32_t* __restrict__ tb_tbl,
+static __global__ __launch_bounds__(BLOCK) void k_chain_table(GView g, uint32_t ta, const uint32_t* __restrict__ tb_tbl,
                                                       uint64_t* __restrict__ H) {
   const uint32_t lane = threadIdx.x & 63;
   const uint64_t nw = (uint64_t)gridDim.x * (BLOCK / 64);
@@ -2204,6 +2223,36 @@ __global__ __launch_bounds__(BLOCK) void k_chain_row(GView g, KPlan P, const uin
     add_wave(&counters[3], bytes);
   }
 }
+
+#ifdef CUTS_MATCH_PART
+#define CUTS_L13(X) X(1) X(2) X(3) X(4) X(5) X(6) X(7) X(8) X(9) X(10) X(11) X(12) X(13)
+#define CUTS_I_CHAIN(L) CUTS_EXTERN template __global__ void k_expand<L, M_CHAIN>(GView, KPlan, ExpandArgs);
+#define CUTS_I_SIB(L) CUTS_EXTERN template __global__ void k_chain_sib<L>(GView, KPlan, SibArgs, ChainTables);
+#define CUTS_I_ROW(L)                                                                                               \
+  CUTS_EXTERN template __global__ void k_chain_row<L>(GView, KPlan, const uint32_t*, uint64_t, const uint32_t*,      \
+                                                      const uint32_t*, ChainTables, uint32_t*, uint8_t*,            \
+                                                      unsigned long long*, int);
+#if CUTS_MATCH_PART == 0
+#define CUTS_EXTERN extern
+CUTS_L13(CUTS_I_CHAIN)
+CUTS_L13(CUTS_I_SIB)
+CUTS_L13(CUTS_I_ROW) CUTS_I_ROW(14) CUTS_I_ROW(15)
+#else
+#define CUTS_EXTERN
+#if CUTS_MATCH_PART == 1
+CUTS_L13(CUTS_I_CHAIN)
+#elif CUTS_MATCH_PART == 2
+CUTS_L13(CUTS_I_SIB)
+#else
+CUTS_L13(CUTS_I_ROW) CUTS_I_ROW(14) CUTS_I_ROW(15)
+#endif
+#endif
+#endif
+
+}  // namespace
+
+#if CUTS_MATCH_HOST
+namespace {
 
 // ---------------------------------------------------------- dispatch
 #define CUTS_DISPATCH_L(L, CALL) \
@@ -3992,5 +4041,7 @@ void run_match_noalloc(Context& c, DeviceGraph& dg, const Plan& p, const MatchOp
   m.arena = &a;
   m.run();
 }
+
+#endif  // CUTS_MATCH_HOST
 
 }  // namespace cuts
