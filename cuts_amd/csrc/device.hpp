@@ -57,6 +57,14 @@ struct KPlan {
   // pr_a and pr_b adjacent in the query: |A & B|'s base is the per-arc
   // common-neighbour count of the arc (row[pr_a], row[pr_b])
   uint32_t pr_adj;
+  // last two positions counted from the whole prefix of positions 0..k-3 (the
+  // pr_* fields describe them): 1: a pair with an owner at position k-3, so
+  // that |A| * |B| - |A & B| depends on every prefix vertex; 2: position k-2
+  // joined to exactly pr_a and pr_b and k-1 to one of them (pr_c), thresholds
+  // <= 2, so that every vertex of A & B is in k-1's list and the prefix has
+  // |A & B| * (|C| - 1) completions
+  uint32_t tl_kind;
+  uint32_t pr_c;
   // last two positions as a chain (symmetric graphs): k-1's one backward
   // neighbour is k-2, whose one backward neighbour ch_u is older than k-3.
   // A prefix P of positions 0..k-3 with u = row[ch_u] and

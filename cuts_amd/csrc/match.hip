@@ -435,6 +435,29 @@ __device__ __forceinline__ void pair_bases(const GView& g, const KPlan& P, const
   }
 }
 
+// Completions of the prefix r[0..N) of positions 0..k-3 (N = k-2) whose last
+// two positions are counted together (tl_kind); |A & B| without its
+// intersection N(u) & N(w) where pair_bases has no index for it.  na gets the
+// prefix's children at position k-2; with stats, mb the merge-model bytes of
+// the prefix's and its children's expansions.
+template <int N>
+__device__ __forceinline__ uint64_t tail_count(const GView& g, const KPlan& P, const uint32_t (&r)[N],
+                                               const PairTables& pt, bool stats, uint64_t& na, uint64_t& mb,
+                                               uint64_t& bytes) {
+  uint32_t u, w;
+  int64_t ca, cb, cab;
+  pair_bases<N>(g, P, r, pt, u, w, ca, cb, cab, bytes);
+  const bool one = P.tl_kind == 1;
+  const int64_t n = one ? ca : cab;
+  na += (uint64_t)n;
+  if (stats) {
+    const uint64_t du = g.off_out[u + 1] - g.off_out[u], dw = g.off_out[w + 1] - g.off_out[w];
+    const uint64_t dc = (one || P.pr_c == P.pr_b) ? dw : du;
+    mb += (one ? 8 + 4 * du : 16 + 4 * (du + dw)) + (uint64_t)n * (24 + 4 * dc);
+  }
+  return (uint64_t)(one ? ca * cb - cab : cab * ((P.pr_c == P.pr_a ? ca : cb) - 1));
+}
+
 // Per prefix: the constraint whose list is shortest (upper bound on the
 // prefix's children).  Ties keep the lowest constraint index.
 // With merge (profiling) it adds the merge-model bytes of expanding the
@@ -1102,7 +1125,7 @@ __device__ __forceinline__ void add_runs(uint32_t* __restrict__ cnt, uint64_t p,
   if (head && mine) atomicAdd(&cnt[p], (uint32_t)__popcll(mine));
 }
 
-enum { M_WRITE = 0, M_COUNT = 1, M_FUSED = 2, M_PAIR = 3, M_CHAIN = 4, M_COLLAPSE = 5, M_GWRITE = 6 };
+enum { M_WRITE = 0, M_COUNT = 1, M_FUSED = 2, M_PAIR = 3, M_CHAIN = 4, M_COLLAPSE = 5, M_GWRITE = 6, M_TAIL = 7 };
 
 struct ExpandArgs {
   const uint32_t* rows;      // n rows of L words
@@ -1120,7 +1143,7 @@ struct ExpandArgs {
   uint32_t* out_parent;      // M_WRITE: parent prefix of every row written (or null)
   const uint32_t* shared;    // M_CHAIN: per prefix, its older positions' intersections with u
   ChainTables ctab;          // M_CHAIN
-  PairTables ptab;           // M_COLLAPSE
+  PairTables ptab;           // M_COLLAPSE, M_TAIL
   const uint64_t* coff;      // M_GWRITE: start of every prefix's block in cand
   uint32_t* cand;            // M_GWRITE: candidates grouped by prefix
   uint32_t xcd;              // 1: XCD-contiguous tile mapping
@@ -1477,6 +1500,20 @@ __global__ __launch_bounds__(BLOCK) void k_expand(GView g, KPlan P, ExpandArgs a
               mb += 16 + 16 + 4 * (du + dw) + (uint64_t)cab * (24 + 4 * du + (uint64_t)(ca - 1) * (24 + 4 * dw));
             }
           }
+        } else if (MODE == M_TAIL) {
+          // a survivor v completes the prefix of positions 0..k-3, whose last
+          // two positions are counted from it (tail_count)
+#pragma unroll
+          for (int j = 0; j < G; ++j) {
+            if (!ok[j]) continue;
+            ++valid;
+            uint32_t r[L + 1];
+#pragma unroll
+            for (int l = 0; l < L; ++l) r[l] = row[j][l];
+            r[L] = v[j];
+            acc += tail_count<L + 1>(g, P, r, a.ptab, a.stats != 0, pairs, mb, bytes);
+            if (a.stats) mb += 16;  // the survivor's node, written and read back
+          }
         } else if (MODE == M_CHAIN) {
           // a survivor v completes the prefix of positions 0..k-3, whose
           // chain of the last two positions is counted in closed form
@@ -1649,13 +1686,15 @@ __global__ __launch_bounds__(BLOCK) void k_expand(GView g, KPlan P, ExpandArgs a
   }
   if (MODE != M_WRITE) {
     add_wave(&a.counters[0], acc);
-    if (MODE == M_FUSED || MODE == M_PAIR || MODE == M_CHAIN || MODE == M_COLLAPSE) add_wave(&a.counters[1], valid);
-    if (MODE == M_PAIR || MODE == M_CHAIN || MODE == M_COLLAPSE) add_wave(&a.counters[2], pairs);
+    if (MODE == M_FUSED || MODE == M_PAIR || MODE == M_CHAIN || MODE == M_COLLAPSE || MODE == M_TAIL)
+      add_wave(&a.counters[1], valid);
+    if (MODE == M_PAIR || MODE == M_CHAIN || MODE == M_COLLAPSE || MODE == M_TAIL) add_wave(&a.counters[2], pairs);
     if (MODE == M_COLLAPSE) add_wave(&a.counters[9], trips);
   }
   if (a.stats) {
     add_wave(&a.counters[3], bytes);
-    if (MODE == M_FUSED || MODE == M_PAIR || MODE == M_CHAIN || MODE == M_COLLAPSE) add_wave(&a.counters[8], mb);
+    if (MODE == M_FUSED || MODE == M_PAIR || MODE == M_CHAIN || MODE == M_COLLAPSE || MODE == M_TAIL)
+      add_wave(&a.counters[8], mb);
   }
 }
 
@@ -1937,6 +1976,47 @@ __global__ __launch_bounds__(BLOCK) void k_chain_prep(GView g, KPlan P, const ui
     }
     minlen[p] = need ? min(du, dw) : 0u;
     minsel[p] = (uint8_t)(du <= dw ? 0u : 1u);
+  }
+}
+
+// Last two positions counted from the stored rows of level k-3 (L = k-2
+// words): tail_count per row; |N(u) & N(w)| of a pair without an index from a
+// hub row, or left to k_common (minlen, minsel and desc set here).
+template <int L>
+__global__ __launch_bounds__(BLOCK) void k_tail_row(GView g, KPlan P, const uint32_t* __restrict__ rows, uint64_t n,
+                                                   PairTables pt, bool known, uint32_t* __restrict__ minlen,
+                                                   uint8_t* __restrict__ minsel, uint4* __restrict__ desc,
+                                                   unsigned long long* __restrict__ counters, int stats) {
+  uint64_t acc = 0, na = 0, mb = 0, bytes = 0;
+  const bool hub = g.hr_id && P.pr_tab <= 2;
+  for (uint64_t p = (uint64_t)blockIdx.x * BLOCK + threadIdx.x; p < n; p += (uint64_t)gridDim.x * BLOCK) {
+    uint32_t r[L];
+#pragma unroll
+    for (int l = 0; l < L; ++l) r[l] = rows[p * L + l];
+    bytes += 4 * L;
+    acc += tail_count<L>(g, P, r, pt, stats != 0, na, mb, bytes);
+    if (known) continue;
+    const uint32_t u = rows[p * L + P.pr_a], w = rows[p * L + P.pr_b];
+    const uint32_t hc = hub ? hub_common(g, u, w) : ~0u;
+    uint32_t len = 0, sel = 0;
+    if (hc != ~0u) {
+      acc -= hc;
+    } else {
+      const uint32_t ul = g.off_out[u], uh = g.off_out[u + 1], wl = g.off_out[w], wh = g.off_out[w + 1];
+      sel = uh - ul <= wh - wl ? 0u : 1u;
+      len = min(uh - ul, wh - wl);
+      // walk the shorter list, test membership in the other
+      const int32_t h = g.hub_id ? g.hub_id[sel ? u : w] : -1;
+      desc[p] = make_uint4(sel ? wl : ul, h >= 0 ? (uint32_t)h : ~0u, sel ? ul : wl, sel ? uh : wh);
+    }
+    minlen[p] = len;
+    minsel[p] = (uint8_t)sel;
+  }
+  add_wave(&counters[0], acc);
+  add_wave(&counters[1], na);
+  if (stats) {
+    add_wave(&counters[8], mb);
+    add_wave(&counters[3], bytes);
   }
 }
 
@@ -2379,6 +2459,7 @@ struct Matcher {
   uint32_t k;
   bool closed_last = false, fuse = false, write = false, pair = false, chain = false, chain_fused = false;
   bool collapse_fused = false, sib = false;
+  bool tail = false, tail_fused = false;  // last two positions from whole prefixes; in the expansion of k-3
   bool sib_live = false;      // candidates of the current level-(k-4) input are built
   uint64_t cand_limit = 0;    // most candidates one build may hold
   const uint32_t* tbl = nullptr;
@@ -2416,6 +2497,7 @@ struct Matcher {
   bool pair_cab_known() const {
     return kp.pr_tab <= 2 && (g.h2_off || (g.arc_cn && kp.pr_adj));
   }
+  bool tail_known() const { return kp.pr_a == kp.pr_b || pair_cab_known(); }
   bool past_deadline() {
     if (has_deadline && !aborted && std::chrono::steady_clock::now() >= deadline) aborted = true;
     return aborted;
@@ -2510,6 +2592,7 @@ struct Matcher {
   // closed form, written embeddings, the pair level's intersection pass)
   bool chainable(uint32_t L) const {
     if (L >= k || !speculate() || o.trunks > 1) return false;
+    if (tail && !tail_fused && L == k - 2) return false;
     if (chain && !chain_fused && L == k - 2) return false;
     if (chain && L == k - 3) return false;
     if (sib && L == k - 4) return false;
@@ -2558,6 +2641,10 @@ struct Matcher {
       chain_rows(L, rows, n);
       return;
     }
+    if (tail && !tail_fused && L == k - 2) {
+      tail_rows(L, rows, n, in);
+      return;
+    }
     if (chain && L == k - 3) {
       chain_shared(L, rows, n, in);
       if (aborted) return;
@@ -2587,9 +2674,10 @@ struct Matcher {
     if (collapse_fused && L == k - 4) mode = M_COLLAPSE;
     else if (pair && L == k - 3) mode = M_PAIR;
     else if (chain_fused && L == k - 3) mode = M_CHAIN;
+    else if (tail_fused && L == k - 3) mode = M_TAIL;
     else if (L == k - 1 && !write) mode = M_COUNT;
     else if (L == k - 2 && fuse) mode = M_FUSED;
-    const int mclass = mode == M_WRITE ? 4 : mode == M_COUNT ? 5 : mode == M_FUSED ? 6 : (mode == M_PAIR || mode == M_COLLAPSE) ? 8 : 10;
+    const int mclass = mode == M_WRITE ? 4 : mode == M_COUNT ? 5 : (mode == M_FUSED || mode == M_TAIL) ? 6 : (mode == M_PAIR || mode == M_COLLAPSE) ? 8 : 10;
     if (mode == M_PAIR) ensure_aux(arena, in.pbase, in.pbase_cap, n);
     const bool spec = speculate() && !(mode == M_WRITE && L == k - 1);
     // a speculative level of at most SCAN_TILE rows plans, scans and indexes
@@ -2737,6 +2825,13 @@ struct Matcher {
 #undef EC2
         HIPCHECK(hipGetLastError());
         pend(10, 0, true);
+      } else if (mode == M_TAIL) {
+        pbegin(true);
+#define ET(LL) hipLaunchKernelGGL((k_expand<LL, M_TAIL>), dim3(grid * cgrow), dim3(nthr), 0, c.stream, g, kp, a)
+        CUTS_DISPATCH_PAIR(L, ET)
+#undef ET
+        HIPCHECK(hipGetLastError());
+        pend(6, 0, true);
       } else if (mode == M_FUSED) {
         pbegin(true);
 #define EF(LL) hipLaunchKernelGGL((k_expand<LL, M_FUSED>), dim3(grid * cgrow), dim3(nthr), 0, c.stream, g, kp, a)
@@ -2819,7 +2914,7 @@ struct Matcher {
     a.xcd = (o.flags & 8u) ? 0 : 1;
     a.tilectr = (unsigned int*)(ctr + 4);
     a.stats = 0;
-    const int mclass = mode == M_WRITE ? 4 : mode == M_COUNT ? 5 : mode == M_FUSED ? 6 : (mode == M_PAIR || mode == M_COLLAPSE) ? 8 : 10;
+    const int mclass = mode == M_WRITE ? 4 : mode == M_COUNT ? 5 : (mode == M_FUSED || mode == M_TAIL) ? 6 : (mode == M_PAIR || mode == M_COLLAPSE) ? 8 : 10;
     const uint32_t grid = grid_for(tmax, 1, gcap(mclass));
     const uint32_t nthr = o.expand_threads ? o.expand_threads : (uint32_t)BLOCK;
     const uint32_t cgrow = (uint32_t)(BLOCK / nthr);
@@ -2873,6 +2968,7 @@ struct Matcher {
 #define ESK(LL) EXS(LL, M_COLLAPSE)
 #define ESH(LL) EXS(LL, M_CHAIN)
 #define ESP(LL) EXS(LL, M_PAIR)
+#define EST(LL) EXS(LL, M_TAIL)
     if (mode == M_COUNT) {
       CUTS_DISPATCH_L(L, ESC)
     } else if (mode == M_FUSED) {
@@ -2881,9 +2977,12 @@ struct Matcher {
       CUTS_DISPATCH_PAIR(L, ESK)
     } else if (mode == M_CHAIN) {
       CUTS_DISPATCH_PAIR(L, ESH)
+    } else if (mode == M_TAIL) {
+      CUTS_DISPATCH_PAIR(L, EST)
     } else {
       CUTS_DISPATCH_PAIR(L, ESP)
     }
+#undef EST
 #undef ESP
 #undef ESH
 #undef ESK
@@ -2910,6 +3009,21 @@ struct Matcher {
     // the pair level's bases (in.pbase) were read by the expansion that has
     // run; the same per-prefix slots now take the walk's descriptors
     common_pass(L, rows, n, in, CommonArgs{kp.pr_a, kp.pr_b, kp.pr_tab, 0u, in.pbase}, in.nsurv, spec);
+  }
+
+  // Last two positions over the rows of level k-3 (L = k-2 words): k_tail_row,
+  // then the intersections that no index holds.
+  void tail_rows(uint32_t L, const uint32_t* rows, uint64_t n, LevelBuf& in) {
+    const bool known = tail_known();
+    if (!known) ensure_aux(arena, in.pbase, in.pbase_cap, n);
+    const uint32_t grid = grid_for(n, BLOCK, grid_cap);
+    pbegin(true);
+#define TR(LL) hipLaunchKernelGGL((k_tail_row<LL>), dim3(grid), dim3(BLOCK), 0, c.stream, g, kp, rows, n, ptbl, known, in.minlen, in.minsel, in.pbase, ctr, (int)prof)
+    CUTS_DISPATCH_L(L, TR)
+#undef TR
+    HIPCHECK(hipGetLastError());
+    pend(7, 0, true);
+    if (!known) common_pass(L, rows, n, in, CommonArgs{kp.pr_a, kp.pr_b, kp.pr_tab, 1u, in.pbase}, nullptr, speculate());
   }
 
   // Counts common neighbours over the work planned in in.minlen / in.minsel
@@ -3189,6 +3303,11 @@ struct Matcher {
     fuse = closed_last && !(o.flags & 2u) && k >= 3;
     pair = fuse && kp.pr_ok && !(o.flags & 128u);
     chain = fuse && !pair && kp.ch_ok && !(o.flags & 256u);
+    // the last two positions from whole prefixes: inside the expansion of
+    // position k-3 where an index holds the intersection, else over stored
+    // rows (a pair only: its intersections can be subtracted afterwards)
+    tail = fuse && !pair && !chain && !(o.flags & 128u) && (kp.tl_kind == 1 || (kp.tl_kind == 2 && tail_known()));
+    tail_fused = tail && tail_known() && k >= 4;
     // 6 blocks of 4 waves per CU: measured best on the power-law workloads
     // (the tiles are taken dynamically, so the grid only sets residency)
     if (o.expand_threads != 0 && o.expand_threads != 64 && o.expand_threads != 128 && o.expand_threads != 256)
@@ -3228,10 +3347,10 @@ struct Matcher {
       ctab.tb = kp.ch_tb > 1 ? cnt_table(c, dg, arena, kp.ch_tb) : nullptr;
       ctab.H = chain_table(c, dg, arena, kp.ch_ta, kp.ch_tb);
     }
-    if (pair) {
+    if (pair || tail) {
       ptbl.a = kp.pr_ta > 1 ? cnt_table(c, dg, arena, kp.pr_ta) : nullptr;
       ptbl.b = kp.pr_tb > 1 ? cnt_table(c, dg, arena, kp.pr_tb) : nullptr;
-      ptbl.ab = kp.pr_tab > 1 ? cnt_table(c, dg, arena, kp.pr_tab) : nullptr;
+      ptbl.ab = kp.pr_a == kp.pr_b && kp.pr_tab > 1 ? cnt_table(c, dg, arena, kp.pr_tab) : nullptr;
     }
     // level sizes of this query's last complete run (a hint only: a level
     // that outgrows it repeats the run)
@@ -3362,7 +3481,7 @@ struct Matcher {
           r.level[k - 4] = hp[1];
           r.level[k - 3] = hp[2];
           r.level[k - 2] = hp[9];
-        } else if (pair || chain_fused) {
+        } else if (pair || chain_fused || tail_fused) {
           r.level[k - 3] = hp[1];
           r.level[k - 2] = hp[2];
         } else if (fuse) {
@@ -3613,15 +3732,24 @@ KPlan make_kplan(const Plan& p, bool symmetric, bool loop_free) {
   // the last two positions together: a = k-2 and b = k-1 not adjacent, one
   // backward neighbour each, both older than k-3 (so |A & B| depends on the
   // rows of level k-4 only)
-  if (kp.sc_ok && loop_free && p.k >= 4 && kp.nj[last - 1] == 1) {
-    const uint32_t pa = kp.jc[last - 1][0] & 31, pb = kp.sc_pos;
-    if (pb != last - 1 && pa + 3 < p.k && pb + 3 < p.k) {
-      kp.pr_ok = 1;
+  if (kp.sc_ok && loop_free && p.k >= 3 && kp.sc_pos != last - 1 &&
+      (kp.nj[last - 1] == 1 || (kp.nj[last - 1] == 2 && p.k >= 4))) {
+    const bool dbl = kp.nj[last - 1] == 2;
+    const uint32_t pa = kp.jc[last - 1][0] & 31, pb = dbl ? kp.jc[last - 1][1] & 31 : kp.sc_pos;
+    kp.pr_ok = !dbl && pa + 3 < p.k && pb + 3 < p.k;
+    if (!kp.pr_ok && !dbl) kp.tl_kind = 1;
+    if (dbl && (kp.sc_pos == pa || kp.sc_pos == pb) && kp.sc_thr <= 2 &&
+        std::max(p.sig_in[last - 1], p.sig_out[last - 1]) <= 2) {
+      kp.tl_kind = 2;
+      kp.pr_c = kp.sc_pos;
+    }
+    if (kp.pr_ok || kp.tl_kind) {
       kp.pr_a = pa;
       kp.pr_b = pb;
-      kp.pr_ta = std::max(p.sig_in[last - 1], p.sig_out[last - 1]);
+      // (kind 2: A & B's vertices have degree >= 2; A and B serve as C only)
+      kp.pr_ta = dbl ? kp.sc_thr : std::max(p.sig_in[last - 1], p.sig_out[last - 1]);
       kp.pr_tb = kp.sc_thr;
-      kp.pr_tab = std::max(kp.pr_ta, kp.pr_tb);
+      kp.pr_tab = dbl ? 2 : std::max(kp.pr_ta, kp.pr_tb);
       auto adjacent = [&](uint32_t i, uint32_t j) {
         const uint32_t a = std::max(i, j), b = std::min(i, j);
         return i != j && (((p.pmask[a] | p.cmask[a]) >> b) & 1);
@@ -3632,7 +3760,7 @@ KPlan make_kplan(const Plan& p, bool symmetric, bool loop_free) {
       }
       kp.pr_adj = adjacent(pa, pb);
       const uint32_t c = last - 2;
-      if (pa != pb && kp.nj[c] == 2 && std::max(p.sig_in[c], p.sig_out[c]) <= 2 && kp.pr_tab <= 2) {
+      if (kp.pr_ok && pa != pb && kp.nj[c] == 2 && std::max(p.sig_in[c], p.sig_out[c]) <= 2 && kp.pr_tab <= 2) {
         const uint32_t j0 = kp.jc[c][0] & 31, j1 = kp.jc[c][1] & 31;
         kp.pr_collapse = (j0 == pa && j1 == pb) || (j0 == pb && j1 == pa);
       }
