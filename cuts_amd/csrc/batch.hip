@@ -760,9 +760,7 @@ namespace {
 template <typename T>
 T* balloc(Batch& b, int slot, uint64_t n) {
   void* p = nullptr;
-  hipError_t e = hipMalloc(&p, std::max<uint64_t>(n, 1) * sizeof(T));
-  if (e != hipSuccess) {
-    (void)hipGetLastError();
+  if (device_malloc(&p, std::max<uint64_t>(n, 1) * sizeof(T)) != hipSuccess) {
     throw Error(-5, "batch: device allocation of " + std::to_string(n * sizeof(T)) + " bytes failed");
   }
   b.allocs[slot] = p;

@@ -7,6 +7,7 @@
 #include <hip/hip_runtime_api.h>
 
 #include <cstdint>
+#include <functional>
 #include <map>
 #include <mutex>
 #include <stdexcept>
@@ -25,6 +26,18 @@ struct Error : std::runtime_error {
 
 void hip_check(hipError_t e, const char* what);
 #define HIPCHECK(x) ::cuts::hip_check((x), #x)
+
+// Device memory (pool.cpp).  device_malloc: hipMalloc on the current device
+// that gives the pool's blocks back before it fails.  pool_take / pool_give:
+// blocks kept between graphs; null when there is no memory; a block is given
+// back once the device has finished with it.  pool_context: a context of the
+// device begins (+1) or ends (-1).  device_free_bytes: free memory, kept
+// blocks included.
+hipError_t device_malloc(void** out, uint64_t bytes);
+void* pool_take(int device, uint64_t bytes);
+void pool_give(int device, void* b);
+void pool_context(int device, int change);
+uint64_t device_free_bytes(int device);
 
 // Plan in the form the kernels read: per position the list of constraints
 // (earlier position | direction<<7) and the signature thresholds, plus the
@@ -125,7 +138,7 @@ struct DeviceGraph {
   uint16_t* h2_dense = nullptr;
   uint32_t h2_dense_rows = 0;
   double h2_build_s = 0;
-  bool h2_on_gpu = false;  // built by k_two_hop (V <= 2^17) rather than on the host
+  bool h2_on_gpu = false;  // built on the device (V <= 2^17) rather than on the host
   // per-arc common-neighbour counts (symmetric loop-free graphs): arc_cn[i]
   // = |N(u) & N(w)| for the arc (u, w) at adj_out[i]; built on the device at
   // upload
@@ -215,6 +228,7 @@ struct Context {
   unsigned long long* lvcnt = nullptr;
   std::unordered_map<std::string, std::array<uint64_t, kMaxQuery>> level_hints;
   char* scratch = nullptr;                // this device's no-allocation scratch array
+  bool counted = false;                   // known to the device's pool (pool_context)
   ~Context();
 };
 
@@ -250,6 +264,14 @@ struct MatchResult {
 
 void context_init(Context& c, int device);
 void upload_graph(Context& c, const Graph& g, DeviceGraph& dg);
+// Upload's common-neighbour rows (index.hip), built on c.stream from the
+// uploaded lists; both return once they are built.  build_hub_rows fills dg.hr
+// (one row of V counts per hub); build_two_hop_device the two-hop index: off
+// (V + 1 zeros) receives the lists' offsets, dense_rows picks the dense rows'
+// vertices from them.
+void build_hub_rows(Context& c, DeviceGraph& dg, const std::vector<uint32_t>& hubs);
+void build_two_hop_device(Context& c, DeviceGraph& dg, std::vector<uint64_t>& off,
+                          const std::function<std::vector<uint32_t>(const std::vector<uint64_t>&)>& dense_rows);
 void run_match(Context& c, DeviceGraph& dg, const Plan& p, const MatchOpts& o, MatchResult& r);
 // Bytes of the static scratch array behind run_match_noalloc.
 uint64_t noalloc_scratch_bytes();

@@ -240,10 +240,13 @@ __device__ __forceinline__ uint32_t arc_common(const GView& g, uint32_t u, uint3
 }
 
 // Per-arc common-neighbour counts of a symmetric loop-free graph: for every
-// arc (u, w) with u < w, |N(u) & N(w)| by walking the shorter list with a
-// membership test in the longer one (a bit test when it belongs to a hub),
-// stored at (u, w) and at the mirror arc (w, u).  One thread per arc; the
-// arc's source is found by an upper-bound search of the offsets.
+// arc (u, w), |N(u) & N(w)| from the two-hop index or a hub row of u or w (one
+// load); the rest (both lists short) once per pair u < w, by walking the
+// shorter list with a membership test in the longer one (a bit test when it
+// belongs to a hub), stored at (u, w) and at the mirror arc (w, u).  One
+// thread per arc; the arc's source is found by an upper-bound search of the
+// offsets.  The walks of long lists were the kernel's time (R-MAT 18: 12.2 ms,
+// 1.3 ms with the rows).
 static __global__ __launch_bounds__(256) void k_arc_common(GView g, uint64_t A, uint32_t* __restrict__ cn) {
   for (uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x; i < A; i += (uint64_t)gridDim.x * 256) {
     uint32_t lo = 0, hi = g.V;  // largest u with off[u] <= i
@@ -253,11 +256,16 @@ static __global__ __launch_bounds__(256) void k_arc_common(GView g, uint64_t A, 
       else hi = mid - 1;
     }
     const uint32_t u = lo, w = g.adj_out[i];
+    uint64_t dummy = 0;
+    const uint32_t known = g.h2_off ? two_hop(g, u, w, dummy) : hub_common(g, u, w);
+    if (g.h2_off || known != ~0u) {
+      cn[i] = known;
+      continue;
+    }
     if (u >= w) continue;
     const uint32_t du = g.off_out[u + 1] - g.off_out[u], dw = g.off_out[w + 1] - g.off_out[w];
     const uint32_t s = du <= dw ? u : w, o = du <= dw ? w : u;
     uint32_t c = 0;
-    uint64_t dummy = 0;
     for (uint32_t j = g.off_out[s]; j < g.off_out[s + 1]; ++j) c += adj_has(g, o, g.adj_out[j], dummy);
     cn[i] = c;
     uint32_t a = g.off_out[w], b = g.off_out[w + 1];
@@ -267,6 +275,38 @@ static __global__ __launch_bounds__(256) void k_arc_common(GView g, uint64_t A, 
       else b = mid;
     }
     cn[a] = c;
+  }
+}
+
+// The signature of every list entry's vertex.
+static __global__ __launch_bounds__(256) void k_entry_sigs(const uint32_t* __restrict__ adj, uint64_t A,
+                                                          const uint2* __restrict__ sig, uint2* __restrict__ out) {
+  for (uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x; i < A; i += (uint64_t)gridDim.x * 256) out[i] = sig[adj[i]];
+}
+
+// What upload asks of the out-lists: {largest length, vertices in their own
+// list, ordered neighbour pairs}.
+static __global__ __launch_bounds__(256) void k_list_stats(const uint32_t* __restrict__ off,
+                                                          const uint32_t* __restrict__ adj, uint32_t V,
+                                                          unsigned long long* __restrict__ out) {
+  unsigned long long most = 0, loops = 0, pairs = 0;
+  for (uint64_t v = (uint64_t)blockIdx.x * 256 + threadIdx.x; v < V; v += (uint64_t)gridDim.x * 256) {
+    const uint32_t lo = off[v], hi = off[v + 1];
+    const uint64_t d = hi - lo;
+    most = most > d ? most : d;
+    loops += member_safe(adj, lo, hi, (uint32_t)v);
+    if (d) pairs += d * (d - 1);
+  }
+  for (int o = 32; o > 0; o >>= 1) {
+    const uint32_t m = __shfl_xor((uint32_t)most, o);  // lengths are 32-bit
+    most = most > m ? most : m;
+    loops += __shfl_xor((uint32_t)loops, o);
+    pairs += ((uint64_t)__shfl_xor((uint32_t)(pairs >> 32), o) << 32) | __shfl_xor((uint32_t)pairs, o);
+  }
+  if ((threadIdx.x & 63) == 0) {
+    atomicMax(&out[0], most);
+    if (loops) atomicAdd(&out[1], loops);
+    if (pairs) atomicAdd(&out[2], pairs);
   }
 }
 
@@ -2384,11 +2424,15 @@ template <typename T>
 void dev_alloc(T*& p, uint64_t n) {
   if (p) HIPCHECK(hipFree(p));
   p = nullptr;
-  hipError_t e = hipMalloc(&p, std::max<uint64_t>(n, 1) * sizeof(T));
-  if (e != hipSuccess) {
-    (void)hipGetLastError();
+  if (device_malloc((void**)&p, std::max<uint64_t>(n, 1) * sizeof(T)) != hipSuccess)
     throw Error(-5, "device allocation of " + std::to_string(n * sizeof(T)) + " bytes failed");
-  }
+}
+
+// An array of the device graph's own, from the pool.
+template <typename T>
+void graph_alloc(const DeviceGraph& dg, T*& p, uint64_t n) {
+  p = (T*)pool_take(dg.device, std::max<uint64_t>(n, 1) * sizeof(T));
+  if (!p) throw Error(-5, "device allocation of " + std::to_string(n * sizeof(T)) + " bytes failed");
 }
 
 // Device buffer of n elements: hipMalloc'd (the old one freed), or carved
@@ -3518,108 +3562,6 @@ struct Matcher {
   }
 };
 
-// Two-hop index on the GPU (symmetric graphs): for every vertex u, the
-// vertices v != u that share a neighbour with u, ascending, with
-// |N(u) & N(v)|.  Each block owns a V-word counter row, zero between
-// vertices.  For its vertex u the block counts every wedge u-x-v with an
-// atomic (a wave per x, its lanes over N(x)), then reads the row in vertex
-// order -- each wave a contiguous quarter, so no barrier inside the sweeps:
-// pass 1 counts the distinct v (u's entries), pass 2 writes them at u's
-// offset (and into u's dense uint16 row when u has one) -- and clears it.
-// Counter reads are agent-scope atomic loads, so they see the atomics'
-// results at L2 rather than a stale L1 line.
-__global__ __launch_bounds__(BLOCK) void k_two_hop(const uint32_t* __restrict__ off, const uint32_t* __restrict__ adj,
-                                                  uint32_t V, uint32_t* __restrict__ rows, int pass,
-                                                  unsigned long long* __restrict__ entries,
-                                                  const uint64_t* __restrict__ h2_off, uint32_t* __restrict__ hv,
-                                                  uint32_t* __restrict__ hc, const int32_t* __restrict__ did,
-                                                  uint16_t* __restrict__ dense) {
-  __shared__ uint32_t s_cnt[BLOCK / 64];
-  uint32_t* cnt = rows + (uint64_t)blockIdx.x * V;
-  const uint32_t tid = threadIdx.x, lane = tid & 63, wave = uni(tid >> 6);
-  constexpr uint32_t NW = BLOCK / 64;
-  const uint32_t q0 = (uint32_t)((uint64_t)V * wave / NW), q1 = (uint32_t)((uint64_t)V * (wave + 1) / NW);
-  for (uint32_t u = blockIdx.x; u < V; u += gridDim.x) {
-    const uint32_t a0 = off[u], a1 = off[u + 1];
-    for (uint32_t i = a0 + wave; i < a1; i += NW) {
-      const uint32_t x = adj[i];
-      const uint32_t b1 = off[x + 1];
-      for (uint32_t j = off[x] + lane; j < b1; j += 64) {
-        const uint32_t v = adj[j];
-        if (v != u) atomicAdd(&cnt[v], 1u);
-      }
-    }
-    __syncthreads();
-    // sweep A: nonzero entries of this wave's quarter
-    uint32_t mine = 0;
-    for (uint32_t v0 = q0; v0 < q1; v0 += 64) {
-      const uint32_t v = v0 + lane;
-      const uint32_t c = v < q1 ? __hip_atomic_load(&cnt[v], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0u;
-      mine += (uint32_t)__popcll(__ballot(c != 0));
-      if (pass == 1 && c) __hip_atomic_store(&cnt[v], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
-    if (lane == 0) s_cnt[wave] = mine;
-    __syncthreads();
-    uint32_t before = 0, total = 0;
-#pragma unroll
-    for (uint32_t w = 0; w < NW; ++w) {
-      const uint32_t t = s_cnt[w];
-      if (w < wave) before += t;
-      total += t;
-    }
-    if (pass == 1) {
-      if (wave == 0) entries[u] = total;  // the same value from every lane of wave 0
-    } else {
-      // sweep B: write the entries in vertex order, clear the row
-      const int32_t dr = did ? did[u] : -1;
-      uint64_t o = h2_off[u] + before;
-      for (uint32_t v0 = q0; v0 < q1; v0 += 64) {
-        const uint32_t v = v0 + lane;
-        const uint32_t c = v < q1 ? __hip_atomic_load(&cnt[v], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0u;
-        const uint64_t m = __ballot(c != 0);
-        if (c) {
-          const uint64_t at = o + lane_rank(m);
-          hv[at] = v;
-          hc[at] = c;
-          if (dr >= 0) dense[(uint64_t)dr * V + v] = (uint16_t)c;
-          __hip_atomic_store(&cnt[v], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
-        o += (uint64_t)__popcll(m);
-      }
-    }
-    __syncthreads();
-  }
-}
-
-// Hub rows (graphs without the two-hop index): row r holds |N(u) & N(v)|
-// for u = hubs[r] and every v != u as uint16 (a count stays below the
-// largest degree, < 2^16).  One block per job (row, first of up to HR_JOB
-// consecutive entries x of u's list): each wave takes an x, its lanes add
-// one to the count of every v in N(x).  Two counts share a 32-bit word, so
-// an add is a 32-bit atomic of 1 or 1 << 16 into its half, which never
-// carries (its count ends below 2^16).
-constexpr uint32_t HR_JOB = 64;
-__global__ __launch_bounds__(BLOCK) void k_hub_rows(const uint32_t* __restrict__ off, const uint32_t* __restrict__ adj,
-                                                   uint32_t V, const uint32_t* __restrict__ hubs,
-                                                   const uint2* __restrict__ jobs, uint32_t* __restrict__ words) {
-  const uint2 jb = jobs[blockIdx.x];
-  const uint32_t u = hubs[jb.x];
-  const uint32_t a1 = min(jb.y + HR_JOB, off[u + 1]);
-  const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const uint64_t base = (uint64_t)jb.x * V;
-  for (uint32_t i = jb.y + wave; i < a1; i += BLOCK / 64) {
-    const uint32_t x = adj[i];
-    const uint32_t b1 = off[x + 1];
-    for (uint32_t j = off[x] + lane; j < b1; j += 64) {
-      const uint32_t v = adj[j];
-      if (v != u) {
-        const uint64_t gi = base + v;
-        atomicAdd(&words[gi >> 1], 1u << ((uint32_t)(gi & 1) * 16));
-      }
-    }
-  }
-}
-
 // Plain streaming copy of n 16-byte words: the calibration kernel for HBM
 // byte counters (it moves exactly 16n bytes each way).
 __global__ __launch_bounds__(BLOCK) void k_copy_probe(const uint4* __restrict__ src, uint4* __restrict__ dst,
@@ -3792,20 +3734,18 @@ DeviceGraph::~DeviceGraph() {
   int prev = 0;
   (void)hipGetDevice(&prev);
   (void)hipSetDevice(device);
-  for (uint32_t* p : {off_out, adj_out, sig}) (void)hipFree(p);
-  if (nsig_out) (void)hipFree(nsig_out);
-  if (!symmetric) {
-    (void)hipFree(off_in);
-    (void)hipFree(adj_in);
-    if (nsig_in) (void)hipFree(nsig_in);
+  // the next owner of these blocks may use them on any stream
+  (void)hipDeviceSynchronize();
+  if (symmetric) {
+    off_in = adj_in = nullptr;  // the out-side's
+    nsig_in = nullptr;
   }
+  for (void* p : {(void*)off_out, (void*)adj_out, (void*)sig, (void*)nsig_out, (void*)off_in, (void*)adj_in,
+                  (void*)nsig_in, (void*)hub_id, (void*)bits, (void*)arc_cn, (void*)h2_off, (void*)h2_v, (void*)h2_c,
+                  (void*)h2_did, (void*)h2_dense, (void*)hr_id, (void*)hr})
+    pool_give(device, p);
   for (auto& kv : cnt_tables) (void)hipFree(kv.second);
   for (auto& kv : chain_tables) (void)hipFree(kv.second);
-  if (hub_id) (void)hipFree(hub_id);
-  if (bits) (void)hipFree(bits);
-  if (arc_cn) (void)hipFree(arc_cn);
-  for (void* p : {(void*)h2_off, (void*)h2_v, (void*)h2_c, (void*)h2_did, (void*)h2_dense, (void*)hr_id, (void*)hr})
-    if (p) (void)hipFree(p);
   (void)hipSetDevice(prev);
 }
 
@@ -3829,6 +3769,7 @@ Context::~Context() {
     if (e) (void)hipEventDestroy(e);
   if (copy_stream) (void)hipStreamDestroy(copy_stream);
   if (stream) (void)hipStreamDestroy(stream);
+  if (counted) pool_context(device, -1);
 }
 
 void context_init(Context& c, int device) {
@@ -3853,10 +3794,10 @@ void context_init(Context& c, int device) {
   HIPCHECK(hipHostMalloc(&c.host_res, 1024, hipHostMallocCoherent | hipHostMallocMapped));
   HIPCHECK(hipMalloc(&c.lvcnt, kMaxQuery * sizeof(unsigned long long)));
   HIPCHECK(hipHostGetDevicePointer((void**)&c.host_res_dev, c.host_res, 0));
-  size_t fr = 0, tot = 0;
-  HIPCHECK(hipMemGetInfo(&fr, &tot));
+  pool_context(device, 1);
+  c.counted = true;
   // trie tables may take 40% of the free HBM by default
-  c.default_budget = (uint64_t)(fr * 0.4);
+  c.default_budget = (uint64_t)((double)device_free_bytes(device) * 0.4);
   c.scratch = scratch_address(device);
 }
 
@@ -3866,16 +3807,8 @@ void upload_graph(Context& c, const Graph& g, DeviceGraph& dg) {
   dg.V = g.V;
   dg.A = g.arcs();
   dg.symmetric = g.symmetric;
-  uint32_t md = 0;
-  uint64_t loops = 0;
-  for (uint32_t v = 0; v < g.V; ++v) {
-    md = std::max(md, g.out_off[v + 1] - g.out_off[v]);
-    loops += std::binary_search(g.out_adj.begin() + g.out_off[v], g.out_adj.begin() + g.out_off[v + 1], v);
-  }
-  dg.max_deg = md;
-  dg.loops = loops;
   auto up = [&](uint32_t*& d, const std::vector<uint32_t>& h) {
-    dev_alloc(d, h.size());
+    graph_alloc(dg, d, h.size());
     HIPCHECK(hipMemcpy(d, h.data(), h.size() * 4, hipMemcpyHostToDevice));
   };
   up(dg.off_out, g.out_off);
@@ -3888,21 +3821,33 @@ void upload_graph(Context& c, const Graph& g, DeviceGraph& dg) {
     up(dg.off_in, g.in_off);
     up(dg.adj_in, g.in_adj);
   }
-  auto up_nsig = [&](uint2*& d, const std::vector<uint32_t>& adj) {
-    std::vector<uint2> h(adj.size());
-#pragma omp parallel for schedule(static)
-    for (int64_t i = 0; i < (int64_t)adj.size(); ++i) h[i] = make_uint2(g.sig[2 * (uint64_t)adj[i]], g.sig[2 * (uint64_t)adj[i] + 1]);
-    dev_alloc(d, std::max<size_t>(h.size(), 1));
-    if (!h.empty()) HIPCHECK(hipMemcpy(d, h.data(), h.size() * sizeof(uint2), hipMemcpyHostToDevice));
+  auto entry_sigs = [&](uint2*& d, const uint32_t* adj, uint64_t A) {
+    graph_alloc(dg, d, A);
+    if (!A) return;
+    hipLaunchKernelGGL(k_entry_sigs, dim3(grid_for(A, 256, (uint32_t)c.cus * 32)), dim3(256), 0, c.stream, adj, A,
+                       (const uint2*)dg.sig, d);
+    HIPCHECK(hipGetLastError());
   };
-  up_nsig(dg.nsig_out, g.out_adj);
+  entry_sigs(dg.nsig_out, dg.adj_out, g.out_adj.size());
   if (g.symmetric) dg.nsig_in = dg.nsig_out;
-  else up_nsig(dg.nsig_in, g.in_adj);
+  else entry_sigs(dg.nsig_in, dg.adj_in, g.in_adj.size());
+  // longest out-list, self-loops and wedges
+  unsigned long long *d_stats = nullptr, stats[3];
+  dev_alloc(d_stats, 3);
+  HIPCHECK(hipMemsetAsync(d_stats, 0, sizeof(stats), c.stream));
+  hipLaunchKernelGGL(k_list_stats, dim3(grid_for(g.V, 256, (uint32_t)c.cus * 8)), dim3(256), 0, c.stream, dg.off_out,
+                     dg.adj_out, g.V, d_stats);
+  HIPCHECK(hipGetLastError());
+  HIPCHECK(hipMemcpyAsync(stats, d_stats, sizeof(stats), hipMemcpyDeviceToHost, c.stream));
+  HIPCHECK(hipStreamSynchronize(c.stream));
+  (void)hipFree(d_stats);
+  dg.max_deg = (uint32_t)stats[0];
+  dg.loops = stats[1];
+  const uint64_t wedges = stats[2];
   // Hub bitmaps: the lowest power-of-two degree threshold (>= 32) whose
   // bitmaps fit the budget (1/32 of free HBM, at most 4 GiB).
   if (g.symmetric && g.V >= 64) {
-    size_t fr = 0, tot = 0;
-    HIPCHECK(hipMemGetInfo(&fr, &tot));
+    const uint64_t fr = device_free_bytes(c.device);
     uint64_t cap = std::min<uint64_t>(fr / 32, 4ull << 30);
     // CUTS_HUB_BITMAP_MB replaces the cap (at most half of free HBM)
     if (const char* e = std::getenv("CUTS_HUB_BITMAP_MB"))
@@ -3930,9 +3875,9 @@ void upload_graph(Context& c, const Graph& g, DeviceGraph& dg) {
       dg.words = words;
       dg.hubs = (uint32_t)hubs.size();
       dg.hub_min_deg = t;
-      dev_alloc(dg.hub_id, g.V);
+      graph_alloc(dg, dg.hub_id, g.V);
       HIPCHECK(hipMemcpy(dg.hub_id, hid.data(), g.V * 4, hipMemcpyHostToDevice));
-      dev_alloc(dg.bits, (uint64_t)hubs.size() * words);
+      graph_alloc(dg, dg.bits, (uint64_t)hubs.size() * words);
       HIPCHECK(hipMemset(dg.bits, 0, (uint64_t)hubs.size() * words * 8));
       uint32_t* dh = nullptr;
       dev_alloc(dh, hubs.size());
@@ -3944,23 +3889,12 @@ void upload_graph(Context& c, const Graph& g, DeviceGraph& dg) {
       (void)hipFree(dh);
     }
   }
-  // Per-arc common-neighbour counts (symmetric loop-free graphs), built on
-  // the device with the hub bitmaps above: 4 bytes per arc while they fit
-  // 1/16 of free HBM.
+  // Per-arc common-neighbour counts (symmetric loop-free graphs): 4 bytes
+  // per arc while they fit 1/16 of free HBM, filled below from the index or
+  // the hub rows.
   if (g.symmetric && dg.loops == 0 && dg.A > 0) {
-    size_t fr = 0, tot = 0;
-    HIPCHECK(hipMemGetInfo(&fr, &tot));
-    if (dg.A * 4 <= fr / 16) {
-      const auto t0 = std::chrono::steady_clock::now();
-      dev_alloc(dg.arc_cn, dg.A);
-      GView gv = view_of(dg);
-      gv.arc_cn = nullptr;
-      const uint32_t grid = (uint32_t)std::min<uint64_t>((dg.A + 255) / 256, (uint64_t)c.cus * 32);
-      hipLaunchKernelGGL(k_arc_common, dim3(grid), dim3(256), 0, c.stream, gv, dg.A, dg.arc_cn);
-      HIPCHECK(hipGetLastError());
-      HIPCHECK(hipStreamSynchronize(c.stream));
-      dg.arc_cn_build_s = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
-    }
+    const uint64_t fr = device_free_bytes(c.device);
+    if (dg.A * 4 <= fr / 16) graph_alloc(dg, dg.arc_cn, dg.A);
   }
   // Two-hop index: built on the host when the wedges (ordered neighbour
   // pairs of every vertex, an upper bound on the entries) fit 1/16 of free
@@ -3968,13 +3902,7 @@ void upload_graph(Context& c, const Graph& g, DeviceGraph& dg) {
   // vertices.
   if (g.symmetric && g.V >= 2) {
     const auto t0 = std::chrono::steady_clock::now();
-    uint64_t wedges = 0;
-    for (uint32_t v = 0; v < g.V; ++v) {
-      const uint64_t d = g.out_off[v + 1] - g.out_off[v];
-      wedges += d * (d ? d - 1 : 0);
-    }
-    size_t fr = 0, tot = 0;
-    HIPCHECK(hipMemGetInfo(&fr, &tot));
+    const uint64_t fr = device_free_bytes(c.device);
     // the host build keeps two V-word arrays per thread: bounded V.
     // CUTS_H2_MAX_WEDGES lowers the wedge cap (0: no index, hub rows instead)
     uint64_t wcap = std::min<uint64_t>(fr / 16 / 8, 1ull << 28);
@@ -4007,45 +3935,8 @@ void upload_graph(Context& c, const Graph& g, DeviceGraph& dg) {
       };
       std::vector<uint64_t> off((size_t)V + 1, 0);
       if (V <= (1u << 17)) {
-        // on the GPU (k_two_hop): pass 1 counts every vertex's entries, the
-        // host sums them into offsets and picks the dense rows, pass 2 writes
-        // the lists and the rows; one V-word counter row per block
         dg.h2_on_gpu = true;
-        const uint32_t G = std::min<uint32_t>(V, 128);
-        uint32_t* cnt_rows = nullptr;
-        unsigned long long* ent = nullptr;
-        dev_alloc(cnt_rows, (uint64_t)G * V);
-        dev_alloc(ent, V);
-        HIPCHECK(hipMemsetAsync(cnt_rows, 0, (uint64_t)G * V * 4, c.stream));
-        hipLaunchKernelGGL(k_two_hop, dim3(G), dim3(BLOCK), 0, c.stream, dg.off_out, dg.adj_out, V, cnt_rows, 1, ent,
-                           (const uint64_t*)nullptr, (uint32_t*)nullptr, (uint32_t*)nullptr, (const int32_t*)nullptr,
-                           (uint16_t*)nullptr);
-        HIPCHECK(hipGetLastError());
-        std::vector<unsigned long long> T(V);
-        HIPCHECK(hipMemcpyAsync(T.data(), ent, (uint64_t)V * 8, hipMemcpyDeviceToHost, c.stream));
-        HIPCHECK(hipStreamSynchronize(c.stream));
-        for (uint32_t u = 0; u < V; ++u) off[u + 1] = off[u] + T[u];
-        dg.h2_entries = off[V];
-        const std::vector<uint32_t> cand = dense_rows(off);
-        dev_alloc(dg.h2_off, V + 1);
-        HIPCHECK(hipMemcpy(dg.h2_off, off.data(), (V + 1) * 8, hipMemcpyHostToDevice));
-        dev_alloc(dg.h2_v, std::max<uint64_t>(off[V], 1));
-        dev_alloc(dg.h2_c, std::max<uint64_t>(off[V], 1));
-        if (!cand.empty()) {
-          std::vector<int32_t> did(V, -1);
-          for (uint64_t r = 0; r < cand.size(); ++r) did[cand[r]] = (int32_t)r;
-          dev_alloc(dg.h2_did, V);
-          HIPCHECK(hipMemcpy(dg.h2_did, did.data(), (uint64_t)V * 4, hipMemcpyHostToDevice));
-          dev_alloc(dg.h2_dense, cand.size() * V);
-          HIPCHECK(hipMemset(dg.h2_dense, 0, cand.size() * 2ull * V));
-          dg.h2_dense_rows = (uint32_t)cand.size();
-        }
-        hipLaunchKernelGGL(k_two_hop, dim3(G), dim3(BLOCK), 0, c.stream, dg.off_out, dg.adj_out, V, cnt_rows, 2, ent,
-                           (const uint64_t*)dg.h2_off, dg.h2_v, dg.h2_c, (const int32_t*)dg.h2_did, dg.h2_dense);
-        HIPCHECK(hipGetLastError());
-        HIPCHECK(hipStreamSynchronize(c.stream));
-        (void)hipFree(cnt_rows);
-        (void)hipFree(ent);
+        build_two_hop_device(c, dg, off, dense_rows);
       } else {
         std::vector<uint32_t> hv, hc;
         build_two_hop(g, off, hv, hc);
@@ -4062,17 +3953,17 @@ void upload_graph(Context& c, const Graph& g, DeviceGraph& dg) {
             for (uint64_t i = off[u]; i < off[u + 1]; ++i) row[hv[i]] = (uint16_t)hc[i];
           }
           for (uint64_t r = 0; r < rows; ++r) did[cand[r]] = (int32_t)r;
-          dev_alloc(dg.h2_did, V);
+          graph_alloc(dg, dg.h2_did, V);
           HIPCHECK(hipMemcpy(dg.h2_did, did.data(), (uint64_t)V * 4, hipMemcpyHostToDevice));
-          dev_alloc(dg.h2_dense, rows * V);
+          graph_alloc(dg, dg.h2_dense, rows * V);
           HIPCHECK(hipMemcpy(dg.h2_dense, dense.data(), rows * 2ull * V, hipMemcpyHostToDevice));
           dg.h2_dense_rows = (uint32_t)rows;
         }
-        dev_alloc(dg.h2_off, V + 1);
+        graph_alloc(dg, dg.h2_off, V + 1);
         HIPCHECK(hipMemcpy(dg.h2_off, off.data(), (V + 1) * 8, hipMemcpyHostToDevice));
-        dev_alloc(dg.h2_v, hv.size());
+        graph_alloc(dg, dg.h2_v, hv.size());
         HIPCHECK(hipMemcpy(dg.h2_v, hv.data(), hv.size() * 4, hipMemcpyHostToDevice));
-        dev_alloc(dg.h2_c, hc.size());
+        graph_alloc(dg, dg.h2_c, hc.size());
         HIPCHECK(hipMemcpy(dg.h2_c, hc.data(), hc.size() * 4, hipMemcpyHostToDevice));
       }
       dg.h2_build_s = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
@@ -4095,33 +3986,26 @@ void upload_graph(Context& c, const Graph& g, DeviceGraph& dg) {
       hubs.resize(std::min<uint64_t>(hubs.size(), cap_rows));
       if (!hubs.empty()) {
         const uint64_t H = hubs.size();
-        std::vector<uint2> jobs;
         std::vector<int32_t> id(V, -1);
-        for (uint64_t r = 0; r < H; ++r) {
-          const uint32_t u = hubs[r];
-          id[u] = (int32_t)r;
-          for (uint32_t i = g.out_off[u]; i < g.out_off[u + 1]; i += HR_JOB) jobs.push_back(make_uint2((uint32_t)r, i));
-        }
-        uint32_t* d_hubs = nullptr;
-        uint2* d_jobs = nullptr;
-        dev_alloc(d_hubs, H);
-        dev_alloc(d_jobs, jobs.size());
-        dev_alloc(dg.hr_id, V);
-        dev_alloc(dg.hr, (H * V + 1) & ~1ull);
-        HIPCHECK(hipMemcpy(d_hubs, hubs.data(), H * 4, hipMemcpyHostToDevice));
-        HIPCHECK(hipMemcpy(d_jobs, jobs.data(), jobs.size() * sizeof(uint2), hipMemcpyHostToDevice));
+        for (uint64_t r = 0; r < H; ++r) id[hubs[r]] = (int32_t)r;
+        graph_alloc(dg, dg.hr_id, V);
+        graph_alloc(dg, dg.hr, H * V);
         HIPCHECK(hipMemcpy(dg.hr_id, id.data(), (uint64_t)V * 4, hipMemcpyHostToDevice));
-        HIPCHECK(hipMemsetAsync(dg.hr, 0, ((H * V + 1) & ~1ull) * 2, c.stream));
-        hipLaunchKernelGGL(k_hub_rows, dim3((uint32_t)jobs.size()), dim3(BLOCK), 0, c.stream, dg.off_out, dg.adj_out, V,
-                           d_hubs, d_jobs, (uint32_t*)dg.hr);
-        HIPCHECK(hipGetLastError());
-        HIPCHECK(hipStreamSynchronize(c.stream));
-        (void)hipFree(d_hubs);
-        (void)hipFree(d_jobs);
+        build_hub_rows(c, dg, hubs);
         dg.hr_rows = (uint32_t)H;
         dg.hr_build_s = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
       }
     }
+  }
+  if (dg.arc_cn) {
+    const auto t0 = std::chrono::steady_clock::now();
+    GView gv = view_of(dg);
+    gv.arc_cn = nullptr;
+    hipLaunchKernelGGL(k_arc_common, dim3(grid_for(dg.A, 256, (uint32_t)c.cus * 32)), dim3(256), 0, c.stream, gv, dg.A,
+                       dg.arc_cn);
+    HIPCHECK(hipGetLastError());
+    HIPCHECK(hipStreamSynchronize(c.stream));
+    dg.arc_cn_build_s = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
   }
 }
 

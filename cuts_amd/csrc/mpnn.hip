@@ -535,11 +535,8 @@ namespace {
 template <typename T>
 T* malloc_dev(uint64_t n) {
   void* p = nullptr;
-  hipError_t e = hipMalloc(&p, std::max<uint64_t>(n, 1) * sizeof(T));
-  if (e != hipSuccess) {
-    (void)hipGetLastError();
+  if (device_malloc(&p, std::max<uint64_t>(n, 1) * sizeof(T)) != hipSuccess)
     throw Error(-5, "mpnn: device allocation failed");
-  }
   return (T*)p;
 }
 }  // namespace
