@@ -44,6 +44,10 @@ namespace {
 constexpr int BB = 256;      // threads per block (4 wave64)
 constexpr int NW = BB / 64;  // waves per block
 constexpr int RMAX = 256;    // rows per item (one per thread in the scan)
+constexpr int CU = 4;        // candidates of a thread in flight together
+// Roots of a level-0 item: each 256 take a stage append with its barriers, so
+// items of 4,096 kept one block busy for 250 us while the others waited.
+constexpr uint32_t L0_ROOTS = 512;
 // LDS words per row (input and staged): a template parameter of at least
 // kmax-1, odd so that rows of different lanes fall in different banks.
 
@@ -172,6 +176,33 @@ __device__ uint64_t closed_form_rt(const GV& g, const KPlan& P, const uint32_t* 
   return (uint64_t)c;
 }
 
+// Last two positions counted from the whole prefix row[0..L) + v of positions
+// 0..k-3 (tl_kind 1 and 2, tail_count of the single-query kernels), |N(u) &
+// N(w)| from the two-hop index.  dv: v's degree; na gets the prefix's
+// children at position k-2.
+__device__ uint64_t tail_count_rt(const GV& g, const KPlan& P, const uint32_t* row, uint32_t L, uint32_t v, uint32_t dv,
+                                  const uint32_t* __restrict__ ta_tbl, const uint32_t* __restrict__ tb_tbl,
+                                  const uint32_t* __restrict__ tab_tbl, int64_t& na) {
+  const uint32_t pa = P.pr_a, pb = P.pr_b;
+  const uint32_t u = pa == L ? v : row[pa], w = pb == L ? v : row[pb];
+  const uint32_t du = pa == L ? dv : g.off_out[u + 1] - g.off_out[u];
+  const uint32_t dw = pb == L ? dv : g.off_out[w + 1] - g.off_out[w];
+  int64_t ca = ta_tbl ? ta_tbl[u] : du, cb = tb_tbl ? tb_tbl[w] : dw;
+  int64_t cab = pa != pb ? (int64_t)two_hop(g, u, w) : (int64_t)(tab_tbl ? tab_tbl[u] : du);
+  for (uint32_t l = 0; l <= L; ++l) {
+    const uint32_t x = l == L ? v : row[l];
+    // a vertex below every threshold counts nowhere
+    const uint32_t d = l == L ? dv : g.sig[2 * (uint64_t)x];
+    const bool ina = ((P.pr_ma >> l) & 1) || (l != pa && has_arc(g, pa == L ? x : u, pa == L ? u : x));
+    const bool inb = pa == pb ? ina : ((P.pr_mb >> l) & 1) || (l != pb && has_arc(g, pb == L ? x : w, pb == L ? w : x));
+    ca -= ina && d >= P.pr_ta;
+    cb -= inb && d >= P.pr_tb;
+    cab -= ina && inb && d >= P.pr_tab;
+  }
+  na = P.tl_kind == 1 ? ca : cab;
+  return (uint64_t)(P.tl_kind == 1 ? ca * cb - cab : cab * ((P.pr_c == pa ? ca : cb) - 1));
+}
+
 // Candidate work of the row row[0..L) + v at its next position L+1: the
 // length of its shortest constraint list (what the consumer will scan), or
 // the closed form's membership tests when L+1 is a closed-form last position.
@@ -199,9 +230,11 @@ struct Shared {
   uint64_t base;
   uint32_t wcnt[NW];
   uint64_t wwork[NW];
+  uint64_t acc[NW][4];            // per wave, sums of the query's items so far: count, sizes of levels L .. L+2
   uint64_t off[RMAX + 1];         // exclusive scan of the rows' shortest list lengths
   uint8_t minsel[RMAX];
-  uint32_t cbase[RMAX];           // fused level: prefix part of the closed form
+  uint32_t cbase[RMAX];           // fused level: prefix part of the closed form; writing level: the staged
+                                  // rows' candidate work
   uint32_t rows[RMAX * WROW];     // input rows of the item
   uint32_t stage[RMAX * WROW];    // output rows waiting for a flush
 };
@@ -227,26 +260,125 @@ __device__ uint64_t wave_incl_scan(uint64_t x) {
   return x;
 }
 
-// One atomic per wave (operand masked to lane 0; the wave total is uniform).
-__device__ void add_block(unsigned long long* dst, uint64_t v) {
-  const uint64_t s = uni64(wave_sum(v));
-  if (s) atomicAdd(dst, lane_id() == 0 ? (unsigned long long)s : 0ull);
+// Adds an item's sums to the wave's slots; the block adds them to the query's
+// words in memory when its next item is another query's (add_query).
+template <int WROW>
+__device__ void add_item(Shared<WROW>& s, uint64_t cnt, uint64_t l0, uint64_t l1, uint64_t l2) {
+  uint64_t* acc = s.acc[wave_id()];
+  const uint64_t t[4] = {uni64(wave_sum(cnt)), uni64(wave_sum(l0)), uni64(wave_sum(l1)), uni64(wave_sum(l2))};
+#pragma unroll
+  for (int i = 0; i < 4; ++i) acc[i] += t[i];  // the same value from every lane
 }
 
-// Called by all 64 lanes of one wave.
-__device__ void push_item(const BatchArgs& a, uint32_t level, const Item& it) {
+// The block's sums for query q and n of its items retired: one atomic per
+// word and run of items of one query.  (One per wave and item before, all on
+// the few words of the queries that fill a level: with items of 1,024
+// candidates they took most of the launch.)  Wave 0, while no wave adds.
+template <int WROW>
+__device__ void add_query(const BatchArgs& a, Shared<WROW>& s, uint32_t q, uint32_t L, uint64_t n) {
   const bool l0 = lane_id() == 0;
-  const unsigned long long slot = uni64(atomicAdd(&a.st->tail[level].v, l0 ? 1ull : 0ull));
-  if (slot >= a.qcap) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    uint64_t t = 0;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) {
+      t += s.acc[w][i];
+      s.acc[w][i] = 0;
+    }
+    t = uni64(t);
+    unsigned long long* dst = i == 0 ? &a.counts[q] : &a.levels[q * kMaxQuery + L + i - 1];
+    if (t) atomicAdd(dst, l0 ? (unsigned long long)t : 0ull);
+  }
+  const unsigned long long left = uni64(atomicSub(&a.qpend[q], l0 ? (unsigned long long)n : 0ull));
+  if (left == n) a.done[q] = wall_clock64();
+}
+
+// Publishes the n (at most RMAX) staged rows at arena offset `off` as items of
+// query q and level `level`, cut where the rows' candidate work (`work`, in
+// row order) passes a multiple of item_split: a group of 256 hub rows is
+// hundreds of thousands of candidates, which one block would walk alone while
+// the others idle.  One item, as the queue's capacity counts it, when the
+// extra slots are used up.  Called by all 64 lanes of one wave.
+__device__ void push_items(const BatchArgs& a, uint32_t q, uint32_t level, uint32_t n, uint64_t off,
+                           const uint32_t* work) {
+  const uint32_t lane = lane_id();
+  const bool l0 = lane == 0;
+  const unsigned long long f = uni64(atomicAdd(&a.st->flushed[level].v, l0 ? 1ull : 0ull));
+  if (f >= a.qcap) {
     atomicOr(&a.st->abort.v, l0 ? 1ull : 0ull);
     return;
   }
-  atomicAdd(&a.qpend[it.qL >> 8], l0 ? 1ull : 0ull);
-  a.items[(uint64_t)(level & 1) * a.qcap + slot] = it;  // same 16 bytes from every lane
+  // lane t holds rows 4t .. 4t+3; a row starts an item when it is the first
+  // or its work's exclusive prefix is in another multiple than the row before
+  constexpr uint32_t RL = RMAX / 64;
+  uint32_t w[RL];
+  uint64_t sum = 0;
+#pragma unroll
+  for (uint32_t i = 0; i < RL; ++i) {
+    w[i] = lane * RL + i < n ? work[lane * RL + i] : 0u;
+    sum += w[i];
+  }
+  uint64_t incl = sum;
+  for (int o = 1; o < 64; o <<= 1) {
+    const uint32_t lo = __shfl_up((uint32_t)incl, o), hi = __shfl_up((uint32_t)(incl >> 32), o);
+    if (lane >= (uint32_t)o) incl += ((uint64_t)hi << 32) | lo;
+  }
+  uint64_t ex = incl - sum;
+  uint64_t prev = lane == 0 ? ~0ull : 0ull;  // the multiple of the row before this lane's first
+  {
+    // exclusive prefix of the previous lane's last row
+    const uint64_t last = incl - w[RL - 1];
+    const uint32_t lo = __shfl_up((uint32_t)last, 1), hi = __shfl_up((uint32_t)(last >> 32), 1);
+    if (lane) prev = ((((uint64_t)hi) << 32) | lo) / a.item_split;
+  }
+  uint32_t starts = 0;
+#pragma unroll
+  for (uint32_t i = 0; i < RL; ++i) {
+    const uint64_t b = ex / a.item_split;
+    if (lane * RL + i < n && b != prev) starts |= 1u << i;
+    prev = b;
+    ex += w[i];
+  }
+  uint32_t cnt = __popc(starts), cincl = cnt;
+  for (int o = 1; o < 64; o <<= 1) {
+    const uint32_t t = __shfl_up(cincl, o);
+    if (lane >= (uint32_t)o) cincl += t;
+  }
+  uint32_t m = uni(__shfl(cincl, 63));
+  if (m > 1) {
+    const unsigned long long e = uni64(atomicAdd(&a.st->extra[level].v, l0 ? (unsigned long long)(m - 1) : 0ull));
+    if (e + (m - 1) > kExtraItems) {
+      m = 1;
+      starts = l0 ? 1u : 0u;
+      cnt = starts;
+      cincl = 1;
+    }
+  }
+  const unsigned long long slot = uni64(atomicAdd(&a.st->tail[level].v, l0 ? (unsigned long long)m : 0ull));
+  atomicAdd(&a.qpend[q], l0 ? (unsigned long long)m : 0ull);
+  Item* dst = a.items + (uint64_t)(level & 1) * (a.qcap + kExtraItems) + slot + (cincl - cnt);
+  // an item ends where the next one starts: the first start after it in this
+  // lane, else the first one of a later lane, else n
+  const uint64_t has = __ballot(starts != 0);
+  const uint32_t first = lane * RL + (starts ? (uint32_t)__builtin_ctz(starts) : 0u);
+  const uint64_t later = lane == 63 ? 0ull : has & (~0ull << (lane + 1));
+  const uint32_t nl = later ? (uint32_t)__builtin_ctzll(later) : 0u;
+  const uint32_t next_first = __shfl(first, nl);
+  uint32_t end_after = later ? next_first : n;
+  while (starts) {
+    const uint32_t i = (uint32_t)__builtin_ctz(starts);
+    starts &= starts - 1;
+    const uint32_t r0 = lane * RL + i, r1 = starts ? lane * RL + (uint32_t)__builtin_ctz(starts) : end_after;
+    Item it;
+    it.qL = (q << 8) | level;
+    it.n = r1 - r0;
+    it.off = off + (uint64_t)r0 * level;
+    *dst++ = it;
+  }
 }
 
 // Writes the staged rows (length `words`, i.e. level `words`) to that
-// level's arena half and publishes them as one item.  Whole block.
+// level's arena half and publishes them (push_items).  Whole block.
 template <int WROW>
 __device__ void flush_stage(const BatchArgs& a, Shared<WROW>& s, uint32_t q, uint32_t words) {
   __syncthreads();
@@ -267,14 +399,10 @@ __device__ void flush_stage(const BatchArgs& a, Shared<WROW>& s, uint32_t q, uin
   const uint64_t base = uni64(s.base);
   if (base != ~0ull) {
     uint32_t* dst = a.arena + (uint64_t)(words & 1) * a.half_words + base;
-    for (uint32_t i = threadIdx.x; i < n * words; i += BB) dst[i] = s.stage[(i / words) * WROW + i % words];
-    if (wave_id() == 0) {
-      Item it;
-      it.qL = (q << 8) | words;
-      it.n = n;
-      it.off = base;
-      push_item(a, words, it);
-    }
+    // a row per thread: neighbouring rows share lines, and no division
+    if (threadIdx.x < n)
+      for (uint32_t l = 0; l < words; ++l) dst[threadIdx.x * words + l] = s.stage[threadIdx.x * WROW + l];
+    if (wave_id() == 0) push_items(a, q, words, n, base, s.cbase);
   }
   s.nstage = 0;  // every thread read nstage before the barrier above
   s.wstage = 0;
@@ -308,7 +436,9 @@ __device__ void stage_append(const BatchArgs& a, Shared<WROW>& s, uint32_t q, bo
       wst = 0;
     }
     if (ok) {
-      uint32_t* dst = &s.stage[(nst + pre + lane_rank64(m)) * WROW];
+      const uint32_t at = nst + pre + lane_rank64(m);
+      s.cbase[at] = (uint32_t)work;
+      uint32_t* dst = &s.stage[at * WROW];
       for (uint32_t l = 0; l < L; ++l) dst[l] = row[l];
       dst[L] = v;
     }
@@ -357,6 +487,9 @@ __device__ void process(const BatchArgs& a, Shared<WROW>& s, uint32_t L) {
   const bool pair = fuse && uni(P.pr_ok) && (a.flags & 8u) == 0;
   // the chain level needs the two-hop index (threshold of A at most 2)
   const bool chain = fuse && !pair && uni(P.ch_ok) && (a.flags & 16u) == 0 && g.h2_off != nullptr && uni(P.ch_ta) <= 2;
+  // the last two positions from whole prefixes, inside the expansion of k-3
+  const bool tail = fuse && !pair && uni(P.tl_kind) && (a.flags & 8u) == 0 && k >= 4 &&
+                    (uni(P.pr_a) == uni(P.pr_b) || (g.h2_off != nullptr && uni(P.pr_tab) <= 2));
   uint64_t cnt = 0, surv = 0, sna = 0;
 
   if (L == 0) {
@@ -371,20 +504,19 @@ __device__ void process(const BatchArgs& a, Shared<WROW>& s, uint32_t L) {
       if (k > 1) stage_append(a, s, q, ok, nullptr, 0, u, ok ? next_work(g, P, nullptr, 0, u, closed) : 0);
     }
     if (k > 1) flush_stage(a, s, q, 1);
-    add_block(&a.levels[q * kMaxQuery + 0], surv);
-    if (k == 1) add_block(&a.counts[q], surv);
+    add_item(s, k == 1 ? surv : 0, surv, 0, 0);
     return;
   }
 
   const uint32_t n = it.n;
   const uint32_t* src = a.arena + (uint64_t)(L & 1) * a.half_words + it.off;
-  for (uint32_t i = tid; i < n * L; i += BB) s.rows[(i / L) * WROW + i % L] = src[i];
+  if (tid < n)
+    for (uint32_t l = 0; l < L; ++l) s.rows[tid * WROW + l] = src[tid * L + l];
   __syncthreads();
 
   if (L == k - 1 && closed) {
     if (tid < n) cnt = closed_form_rt(g, P, &s.rows[tid * WROW], L, false, 0, tbl);
-    add_block(&a.counts[q], cnt);
-    add_block(&a.levels[q * kMaxQuery + L], cnt);
+    add_item(s, cnt, cnt, 0, 0);
     return;
   }
 
@@ -393,6 +525,7 @@ __device__ void process(const BatchArgs& a, Shared<WROW>& s, uint32_t L) {
   const int mode = (L == k - 1) ? 1
                    : (pair && L == k - 3)  ? 3
                    : (chain && L == k - 3) ? 4
+                   : (tail && L == k - 3)  ? 5
                    : (L == k - 2 && fuse)  ? 2
                                            : 0;
   // fused level with an older closed-form vertex u: the closed form splits
@@ -486,80 +619,116 @@ __device__ void process(const BatchArgs& a, Shared<WROW>& s, uint32_t L) {
   const uint64_t W = block_scan(s, n, len);
 
   const uint32_t tin = P.sig_in[L], tout = P.sig_out[L];
-  for (uint64_t w0 = 0; w0 < W; w0 += BB) {
-    const uint64_t w = w0 + tid;
-    bool ok = false;
-    uint32_t v = 0, r = 0;
-    uint64_t fc = 0;  // fused: closed-form count of the survivor
-    if (w < W) {
-      uint32_t lo = 0, hi = n + 1;
-      while (lo < hi) {
-        const uint32_t mid = (lo + hi) >> 1;
-        if (s.off[mid] <= w) lo = mid + 1;
-        else hi = mid;
+  // CU candidates of a thread go through the list word, the signature and the
+  // hub tests together, so that their loads are in flight at once
+  for (uint64_t w0 = 0; w0 < W; w0 += (uint64_t)CU * BB) {
+    bool ok[CU];
+    uint32_t v[CU], r[CU], jcs[CU];
+    uint2 sg[CU];
+#pragma unroll
+    for (int j = 0; j < CU; ++j) {
+      const uint64_t w = w0 + (uint64_t)j * BB + tid;
+      ok[j] = w < W;
+      const uint64_t wc = ok[j] ? w : W - 1;  // the last candidate in place of none
+      uint32_t lo = 0;                       // largest row with off(row) <= wc
+      for (uint32_t m = n; m > 1;) {
+        const uint32_t half = m >> 1;
+        lo = s.off[lo + half] <= wc ? lo + half : lo;
+        m -= half;
       }
-      r = lo - 1;
-      const uint32_t idx = (uint32_t)(w - s.off[r]);
-      const uint32_t* row = &s.rows[r * WROW];
-      const uint32_t sel = s.minsel[r];
-      const uint32_t jc = P.jc[L][sel];
-      const uint32_t u = row[jc & 31];
-      const uint32_t* off = (jc >> 7) ? g.off_in : g.off_out;
-      const uint32_t* adj = (jc >> 7) ? g.adj_in : g.adj_out;
-      const uint32_t li = off[u] + idx;
-      v = adj[li];
-      const uint2 sgv = ((jc >> 7) ? g.nsig_in : g.nsig_out)[li];
-      ok = sgv.x >= tin && sgv.y >= tout;
-      for (uint32_t l = 0; l < L && ok; ++l) ok = v != row[l];
-      for (uint32_t c = 0; c < nj && ok; ++c) {
-        if (c == sel) continue;
-        const uint32_t jc2 = P.jc[L][c];
-        const uint32_t u2 = row[jc2 & 31];
-        if (g.hub_id) {
-          ok = has_arc(g, u2, v);
-        } else {
-          const uint32_t* off2 = (jc2 >> 7) ? g.off_in : g.off_out;
-          const uint32_t* adj2 = (jc2 >> 7) ? g.adj_in : g.adj_out;
-          ok = bmember(adj2, off2[u2], off2[u2 + 1], v);
+      r[j] = lo;
+      const uint32_t jc = P.jc[L][s.minsel[lo]];
+      jcs[j] = jc;
+      const uint32_t u = s.rows[lo * WROW + (jc & 31)];
+      const uint32_t li = ((jc >> 7) ? g.off_in : g.off_out)[u] + (uint32_t)(wc - s.off[lo]);
+      v[j] = ((jc >> 7) ? g.adj_in : g.adj_out)[li];
+      sg[j] = ((jc >> 7) ? g.nsig_in : g.nsig_out)[li];
+    }
+#pragma unroll
+    for (int j = 0; j < CU; ++j) {
+      ok[j] = ok[j] && sg[j].x >= tin && sg[j].y >= tout;
+      const uint32_t* row = &s.rows[r[j] * WROW];
+      for (uint32_t l = 0; l < L; ++l) ok[j] = ok[j] && v[j] != row[l];
+    }
+    for (uint32_t c = 0; c < nj; ++c) {
+      const uint32_t jc2 = P.jc[L][c];
+      if (g.hub_id) {
+        int32_t h[CU];
+        uint64_t bw[CU];
+#pragma unroll
+        for (int j = 0; j < CU; ++j) h[j] = g.hub_id[s.rows[r[j] * WROW + (jc2 & 31)]];
+#pragma unroll
+        for (int j = 0; j < CU; ++j)
+          bw[j] = (ok[j] && jcs[j] != jc2 && h[j] >= 0) ? g.bits[(uint64_t)h[j] * g.words + (v[j] >> 6)] : 0ull;
+#pragma unroll
+        for (int j = 0; j < CU; ++j) {
+          if (!ok[j] || jcs[j] == jc2) continue;
+          const uint32_t u2 = s.rows[r[j] * WROW + (jc2 & 31)];
+          ok[j] = h[j] >= 0 ? (bool)((bw[j] >> (v[j] & 63)) & 1ull)
+                            : bmember(g.adj_out, g.off_out[u2], g.off_out[u2 + 1], v[j]);
         }
-      }
-      if (mode == 3 && ok) {
-        const bool ina = ((P.pr_ma >> L) & 1) || has_arc(g, row[pa], v);
-        const bool inb = ((P.pr_mb >> L) & 1) || has_arc(g, row[pb], v);
-        const uint64_t na = pxa[r] - (uint32_t)(ina && sgv.x >= P.pr_ta);
-        const uint64_t nb = pxb[r] - (uint32_t)(inb && sgv.x >= P.pr_tb);
-        const int64_t nab = (int64_t)(int32_t)pxz[r] - (int64_t)(ina && inb && sgv.x >= P.pr_tab);
-        fc = na * nb - (uint64_t)nab;  // modulo-2^64 sums are exact
-        sna += na;
-        if (pa != pb && !h2) atomicAdd(&pns[r], 1u);
-      }
-      if (mode == 4 && ok) {
-        int64_t na = 0;
-        fc = (uint64_t)chain_closed_rt(g, P, row, L, v, a.chH[q], a.tbls[3 * q + 1], tbl, pxa[r], na);
-        sna += (uint64_t)na;
-      }
-      if (mode == 2 && ok) {
-        if (use_cbase) {
-          // v is certainly in N(u) when it was drawn from u's own list
-          const uint32_t us = row[sc_pos];
-          const bool in = (jc & 31) == sc_pos || has_arc(g, us, v);
-          fc = (uint64_t)s.cbase[r] - ((in && (sc_thr <= 1 || g.sig[2 * (uint64_t)v] >= sc_thr)) ? 1 : 0);
-        } else {
-          fc = closed_form_rt(g, P, row, L, true, v, tbl);
+      } else {
+        const uint32_t* off2 = (jc2 >> 7) ? g.off_in : g.off_out;
+        const uint32_t* adj2 = (jc2 >> 7) ? g.adj_in : g.adj_out;
+#pragma unroll
+        for (int j = 0; j < CU; ++j) {
+          const uint32_t u2 = s.rows[r[j] * WROW + (jc2 & 31)];
+          if (ok[j] && jcs[j] != jc2) ok[j] = bmember(adj2, off2[u2], off2[u2 + 1], v[j]);
         }
       }
     }
-    const uint32_t* row = &s.rows[r * WROW];
-    if (mode == 1) {
-      cnt += ok;
-    } else if (mode >= 2) {
-      if (ok) {
-        ++surv;
-        cnt += fc;
+    // the outcomes one candidate after another: one copy of the code, the
+    // next candidate moved to the front
+#pragma unroll 1
+    for (int it = 0; it < CU; ++it) {
+      const bool o = ok[0];
+      const uint32_t vv = v[0], rr = r[0], dv = sg[0].x, jc = jcs[0];
+#pragma unroll
+      for (int j = 0; j + 1 < CU; ++j) {
+        ok[j] = ok[j + 1];
+        v[j] = v[j + 1];
+        r[j] = r[j + 1];
+        sg[j] = sg[j + 1];
+        jcs[j] = jcs[j + 1];
       }
-    } else {
-      surv += ok;
-      stage_append(a, s, q, ok, row, L, v, ok ? next_work(g, P, row, L, v, closed) : 0);
+      const uint32_t* row = &s.rows[rr * WROW];
+      if (mode == 0) {
+        surv += o;
+        stage_append(a, s, q, o, row, L, vv, o ? next_work(g, P, row, L, vv, closed) : 0);
+        continue;
+      }
+      if (!o) continue;
+      if (mode == 1) {
+        ++cnt;
+        continue;
+      }
+      uint64_t fc;  // completions of the survivor
+      if (mode == 3) {
+        const bool ina = ((P.pr_ma >> L) & 1) || has_arc(g, row[pa], vv);
+        const bool inb = ((P.pr_mb >> L) & 1) || has_arc(g, row[pb], vv);
+        const uint64_t na = pxa[rr] - (uint32_t)(ina && dv >= P.pr_ta);
+        const uint64_t nb = pxb[rr] - (uint32_t)(inb && dv >= P.pr_tb);
+        const int64_t nab = (int64_t)(int32_t)pxz[rr] - (int64_t)(ina && inb && dv >= P.pr_tab);
+        fc = na * nb - (uint64_t)nab;  // modulo-2^64 sums are exact
+        sna += na;
+        if (pa != pb && !h2) atomicAdd(&pns[rr], 1u);
+      } else if (mode == 4) {
+        int64_t na = 0;
+        fc = (uint64_t)chain_closed_rt(g, P, row, L, vv, a.chH[q], a.tbls[3 * q + 1], tbl, pxa[rr], na);
+        sna += (uint64_t)na;
+      } else if (mode == 5) {
+        int64_t na = 0;
+        fc = tail_count_rt(g, P, row, L, vv, dv, a.tbls[3 * q + 1], tbl, a.tbls[3 * q + 2], na);
+        sna += (uint64_t)na;
+      } else if (use_cbase) {
+        // v is certainly in N(u) when it was drawn from u's own list
+        const bool in = (jc & 31) == sc_pos || has_arc(g, row[sc_pos], vv);
+        fc = (uint64_t)s.cbase[rr] - ((in && (sc_thr <= 1 || dv >= sc_thr)) ? 1 : 0);
+      } else {
+        fc = closed_form_rt(g, P, row, L, true, vv, tbl);
+      }
+      ++surv;
+      cnt += fc;
     }
   }
   if (mode == 0) flush_stage(a, s, q, L + 1);
@@ -595,21 +764,9 @@ __device__ void process(const BatchArgs& a, Shared<WROW>& s, uint32_t L) {
       }
     }
   }
-  if (mode == 3 || mode == 4) {
-    add_block(&a.counts[q], cnt);
-    add_block(&a.levels[q * kMaxQuery + L], surv);
-    add_block(&a.levels[q * kMaxQuery + L + 1], sna);
-    add_block(&a.levels[q * kMaxQuery + L + 2], cnt);
-  } else if (mode == 1) {
-    add_block(&a.counts[q], cnt);
-    add_block(&a.levels[q * kMaxQuery + L], cnt);
-  } else if (mode == 2) {
-    add_block(&a.counts[q], cnt);
-    add_block(&a.levels[q * kMaxQuery + L], surv);
-    add_block(&a.levels[q * kMaxQuery + L + 1], cnt);
-  } else {
-    add_block(&a.levels[q * kMaxQuery + L], surv);
-  }
+  if (mode >= 3) add_item(s, cnt, surv, sna, cnt);
+  else if (mode == 2) add_item(s, cnt, surv, cnt, 0);
+  else add_item(s, cnt, mode == 1 ? cnt : surv, 0, 0);
 }
 
 // Processes every item of level L: published by the earlier launches, or by
@@ -618,45 +775,54 @@ template <int WROW>
 __device__ __forceinline__ void level_items(const BatchArgs& a, Shared<WROW>& s, uint32_t L) {
   const bool l0 = lane_id() == 0;
   const unsigned long long n_items = uni64(std::min<unsigned long long>(
-      __hip_atomic_load(&a.st->tail[L].v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT), a.qcap));
+      __hip_atomic_load(&a.st->tail[L].v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT), a.qcap + kExtraItems));
+  // items per ticket: one while they are few, so that every block gets some,
+  // up to eight (all blocks draw from one word)
+  const uint32_t take = (uint32_t)std::min<unsigned long long>(8, 1 + n_items / (16ull * gridDim.x));
   s.nstage = 0;  // same value from every thread
   s.wstage = 0;
-  uint32_t prev_q = 0xFFFFFFFFu;  // query of the item finished in the last round
+  if (threadIdx.x < NW * 4) s.acc[threadIdx.x / 4][threadIdx.x % 4] = 0;
+  uint32_t cur_q = 0xFFFFFFFFu;  // query of the last items (wave 0's, as the next three)
+  unsigned long long t_next = 0, t_end = 0, retired = 0;
   while (true) {
     if (wave_id() == 0) {
-      // retire the previous item, then take the next ticket
-      if (prev_q != 0xFFFFFFFFu) {
-        const unsigned long long left = uni64(atomicSub(&a.qpend[prev_q], l0 ? 1ull : 0ull));
-        if (left == 1ull) a.done[prev_q] = wall_clock64();
+      uint32_t cmd = 1, q = 0xFFFFFFFFu;
+      if (t_next >= t_end &&
+          uni64(__hip_atomic_load(&a.st->abort.v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) == 0) {
+        t_next = uni64(atomicAdd(&a.st->head[L].v, l0 ? (unsigned long long)take : 0ull));
+        t_end = std::min<unsigned long long>(t_next + take, n_items);
       }
-      uint32_t cmd = 1;
-      if (uni64(__hip_atomic_load(&a.st->abort.v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) == 0) {
-        const unsigned long long t = uni64(atomicAdd(&a.st->head[L].v, l0 ? 1ull : 0ull));
-        if (t < n_items) {
-          const Item* ip = &a.items[(uint64_t)(L & 1) * a.qcap + t];
-          Item it;
-          it.qL = uni(ip->qL);
-          it.n = uni(ip->n);
-          it.off = uni64(ip->off);
-          // an item outside the shapes the kernels write means corrupt
-          // memory: stop instead of reading out of bounds
-          const bool sane = (it.qL >> 8) < a.nq && (it.qL & 0xFF) == L &&
-                            (L == 0 ? (it.off + it.n <= a.roots[3 * (it.qL >> 8) + 2])
-                                    : (it.n >= 1 && it.n <= (uint32_t)RMAX &&
-                                       it.off + (uint64_t)it.n * L <= a.half_words));
-          if (sane) {
-            s.item = it;
-            cmd = 0;
-          } else {
-            atomicOr(&a.st->abort.v, l0 ? 4ull : 0ull);
-          }
+      if (t_next < t_end) {
+        const Item* ip = &a.items[(uint64_t)(L & 1) * (a.qcap + kExtraItems) + t_next];
+        Item it;
+        it.qL = uni(ip->qL);
+        it.n = uni(ip->n);
+        it.off = uni64(ip->off);
+        // an item outside the shapes the kernels write means corrupt
+        // memory: stop instead of reading out of bounds
+        const bool sane = (it.qL >> 8) < a.nq && (it.qL & 0xFF) == L &&
+                          (L == 0 ? (it.off + it.n <= a.roots[3 * (it.qL >> 8) + 2])
+                                  : (it.n >= 1 && it.n <= (uint32_t)RMAX &&
+                                     it.off + (uint64_t)it.n * L <= a.half_words));
+        if (sane) {
+          s.item = it;
+          cmd = 0;
+          q = it.qL >> 8;
+          ++t_next;
+        } else {
+          atomicOr(&a.st->abort.v, l0 ? 4ull : 0ull);
         }
       }
+      if (q != cur_q && retired) {
+        add_query(a, s, cur_q, L, retired);
+        retired = 0;
+      }
+      cur_q = q;
+      ++retired;
       s.cmd = cmd;
     }
     __syncthreads();
     if (uni(s.cmd)) break;
-    prev_q = uni(s.item.qL) >> 8;
     process(a, s, L);
     __syncthreads();
   }
@@ -720,6 +886,8 @@ __global__ __launch_bounds__(BB) void k_batch_init(BatchArgs a) {
     for (uint32_t l = 0; l <= kMaxQuery; ++l) {
       a.st->head[l].v = 0;
       a.st->tail[l].v = 0;
+      a.st->flushed[l].v = 0;
+      a.st->extra[l].v = 0;
       a.st->arena[l].v = 0;
     }
     a.st->tail[0].v = a.n_init;
@@ -796,6 +964,8 @@ void batch_create(Context& c, DeviceGraph& dg, const std::vector<const Plan*>& p
   std::vector<uint32_t> roots(3 * (size_t)b.nq);
   std::vector<unsigned long long> qinit(b.nq);
   std::vector<Item> init;
+  uint64_t coarse = 0, fine = 0;  // items of vchunk roots, and of at most L0_ROOTS
+  const uint32_t small = std::min<uint32_t>(b.vchunk, L0_ROOTS);
   for (uint32_t q = 0; q < b.nq; ++q) {
     uint32_t first = 0, end = dg.V, stride = 1;
     if (o.roots) {
@@ -808,16 +978,23 @@ void batch_create(Context& c, DeviceGraph& dg, const std::vector<const Plan*>& p
     roots[3 * q] = first;
     roots[3 * q + 1] = stride;
     roots[3 * q + 2] = cnt;
-    for (uint64_t off = 0; off < cnt; off += b.vchunk) {
+    coarse += ((uint64_t)cnt + b.vchunk - 1) / b.vchunk;
+    fine += ((uint64_t)cnt + small - 1) / small;
+  }
+  if (coarse > qcap) throw Error(-1, "batch: queue too small for the level-0 items");
+  // the queue's extra slots take the finer items
+  const uint32_t chunk = fine <= kExtraItems ? small : b.vchunk;
+  for (uint32_t q = 0; q < b.nq; ++q) {
+    const uint32_t cnt = roots[3 * q + 2];
+    for (uint64_t off = 0; off < cnt; off += chunk) {
       Item it;
       it.qL = q << 8;
-      it.n = (uint32_t)std::min<uint64_t>(b.vchunk, cnt - off);
+      it.n = (uint32_t)std::min<uint64_t>(chunk, cnt - off);
       it.off = off;
       init.push_back(it);
       ++qinit[q];
     }
   }
-  if (init.size() > qcap) throw Error(-1, "batch: queue too small for the level-0 items");
   const uint64_t half_words = (o.arena_bytes ? o.arena_bytes : (8ull << 30)) / 8;
   if (half_words < 16) throw Error(-1, "batch: arena too small");
   std::vector<KPlan> kp(b.nq);
@@ -830,7 +1007,7 @@ void batch_create(Context& c, DeviceGraph& dg, const std::vector<const Plan*>& p
     b.k.push_back(plans[q]->k);
     b.kmax = std::max(b.kmax, plans[q]->k);
     if (kp[q].sc_ok && kp[q].sc_thr > 1 && !(o.flags & 1u)) tb[3 * q] = cnt_table(c, dg, kp[q].sc_thr);
-    if (kp[q].pr_ok && !(o.flags & (1u | 2u | 128u))) {
+    if ((kp[q].pr_ok || kp[q].tl_kind) && !(o.flags & (1u | 2u | 128u))) {
       if (kp[q].pr_ta > 1) tb[3 * q + 1] = cnt_table(c, dg, kp[q].pr_ta);
       if (kp[q].pr_tab > 1) tb[3 * q + 2] = cnt_table(c, dg, kp[q].pr_tab);
     }
@@ -868,7 +1045,7 @@ void batch_create(Context& c, DeviceGraph& dg, const std::vector<const Plan*>& p
   a.chH = dchh;
   a.st = balloc<BState>(b, 2, 1);
   HIPCHECK(hipMemset(a.st, 0, sizeof(BState)));
-  a.items = balloc<Item>(b, 3, 2 * qcap);
+  a.items = balloc<Item>(b, 3, 2 * (qcap + kExtraItems));
   a.qcap = qcap;
   a.arena = balloc<uint32_t>(b, 5, 2 * half_words);
   a.half_words = half_words;
@@ -907,6 +1084,12 @@ void batch_create(Context& c, DeviceGraph& dg, const std::vector<const Plan*>& p
     b.grid = (uint32_t)c.cus * bpc;
   }
   a.item_work = o.item_work ? o.item_work : 16384;
+  // a flush's items: an eighth of that, at least 2,048 candidates -- an item's
+  // planning costs about as much as 500 candidates, and larger items leave
+  // blocks idle (39 and 36 walk queries on the 36,692-vertex Chung-Lu graph:
+  // 5.4 / 5.4 ms with items of 1,024, 4.9 / 5.2 of 2,048, 4.8 / 5.9 of 4,096,
+  // 6.7 / 7.8 of 8,192)
+  a.item_split = std::max<uint64_t>(std::min<uint64_t>(a.item_work, 2048), a.item_work / 8);
   a.flags = (o.flags & 3u) | ((o.flags & 64u) ? 4u : 0u) | ((o.flags & 128u) ? 8u : 0u) | ((o.flags & 256u) ? 16u : 0u);
   a.nq = b.nq;
 }

@@ -17,9 +17,15 @@ struct alignas(256) PadCtr {
   unsigned long long v;
 };
 
+// Slots of an item half beyond the queue's capacity, for flushes split into
+// several items.
+constexpr uint64_t kExtraItems = 1ull << 20;
+
 struct BState {
   PadCtr head[kMaxQuery + 1];   // items of level L taken
   PadCtr tail[kMaxQuery + 1];   // items of level L published
+  PadCtr flushed[kMaxQuery + 1];  // flushes of level L (at most qcap)
+  PadCtr extra[kMaxQuery + 1];    // items asked for beyond one per flush (granted up to kExtraItems)
   PadCtr arena[kMaxQuery + 1];  // arena words of level L allocated (in half L & 1)
   PadCtr abort;                 // 1 item queue full, 2 arena full, 4 corrupt item, 8 barrier wait too long
   PadCtr t_start;
@@ -42,7 +48,7 @@ struct BatchArgs {
                                 // (= B's of the pair level), A's and A & B's (A's of the chain level)
   const uint64_t* const* chH;   // per query: chain-level vertex tables or null
   BState* st;
-  Item* items;                  // 2 halves of qcap items; level L uses half L & 1
+  Item* items;                  // 2 halves of qcap + kExtraItems items; level L uses half L & 1
   uint64_t qcap;
   uint32_t* arena;              // 2 halves of half_words; level L rows in half L & 1
   uint64_t half_words;
@@ -51,7 +57,8 @@ struct BatchArgs {
   const unsigned long long* qinit;  // per query: level-0 items
   const Item* init_items;       // level-0 items, copied into the queue by every replay
   uint64_t n_init;
-  uint64_t item_work;           // candidate work at which a staged item is flushed
+  uint64_t item_work;           // candidate work at which staged rows are flushed
+  uint64_t item_split;          // candidate work at which a flush starts a new item
   uint32_t flags;               // 1: no closed form, 2: no fusion, 4: no per-prefix base, 8: no pair level,
                                 // 16: no chain level
   uint32_t nq;                  // queries in the batch

@@ -106,3 +106,27 @@ def test_thresholds_above_two_and_a_deadline(ctx):
         for flags in FLAGS:
             assert ctx.match(dg, p, flags=flags).count == want, (loops, flags)
             assert ctx.match(dg, p, flags=flags, time_limit_ms=1e6, trunks=9).count == want
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("queue", ["level", "persistent"])
+def test_batch_counts_them_too(ctx, queue):
+    """The batched queue, with its flushes cut into items of one candidate, of
+    a few, and not at all."""
+    g = F.Graph.chung_lu(160, 700, 2.2, 0, 12)
+    og = oracle.OGraph.from_view(g.view())
+    plans, want = [], []
+    for edges, order in CASES.values():
+        k = len(order)
+        plans.append(F.Plan(F.Graph.from_edges(k, edges), order))
+        want.append(oracle.count(og, oracle.qmatrix(k, oracle.undirected(edges))))
+    dg = ctx.upload(g)
+    single = [ctx.match(dg, p) for p in plans]
+    assert [r.count for r in single] == want
+    for kw in (dict(), dict(item_work=1), dict(item_work=50, vchunk=9), dict(item_work=1 << 20)):
+        for flags in (0, F.FLAG_NO_TWO_HOP, F.FLAG_NO_PAIR, F.FLAG_NO_BITMAP):
+            b = F.Batch(ctx, dg, plans, queue=queue, flags=flags, arena_bytes=1 << 28, **kw)
+            for _ in range(2):
+                r = b.run()
+                assert r.counts == want, (kw, flags)
+                assert r.level_sizes == [s.level_sizes for s in single], (kw, flags)
