@@ -239,6 +239,33 @@ __device__ __forceinline__ uint32_t arc_common(const GView& g, uint32_t u, uint3
   return g.arc_cn[lo];
 }
 
+// |N(u) & N(w)| for u != w, thresholds up to 2, from the two-hop index (a
+// dense row of either vertex is one load) or, adjacent in the data graph, from
+// a hub row or the per-arc table, searched in the shorter list; call it where
+// one of them is known to hold it.
+__device__ __forceinline__ uint32_t index_common(const GView& g, uint32_t u, uint32_t w, uint64_t& bytes) {
+  if (g.h2_off) {
+    if (g.h2_did) {
+      const int32_t du = g.h2_did[u];
+      if (du < 0) {
+        const int32_t dw = g.h2_did[w];
+        if (dw >= 0) {
+          bytes += 10;
+          return g.h2_dense[(uint64_t)dw * g.V + u];
+        }
+      }
+    }
+    return two_hop(g, u, w, bytes);
+  }
+  const uint32_t hc = hub_common(g, u, w);
+  if (hc != ~0u) {
+    bytes += 10;
+    return hc;
+  }
+  const bool swap = g.off_out[u + 1] - g.off_out[u] > g.off_out[w + 1] - g.off_out[w];
+  return arc_common(g, swap ? w : u, swap ? u : w, bytes);
+}
+
 // Per-arc common-neighbour counts of a symmetric loop-free graph: for every
 // arc (u, w), |N(u) & N(w)| from the two-hop index or a hub row of u or w (one
 // load); the rest (both lists short) once per pair u < w, by walking the
@@ -446,10 +473,13 @@ __device__ __forceinline__ uint32_t tbl_or_deg(const GView& g, const uint32_t* t
 // for |A & B| the prefix vertices inside both, negated, plus the filtered
 // size of N(u) when u = w, else |N(u) & N(w)| from the two-hop index (0
 // without it).
+// dn: the degree of r[N-1], where the caller has it from its list entry (else
+// ~0u), which saves that vertex's gathers: with one prefix per lane every load
+// at a vertex of its own is 64 lines.
 template <int N>
 __device__ __forceinline__ void pair_bases(const GView& g, const KPlan& P, const uint32_t (&r)[N], const PairTables& pt,
-                                           uint32_t& u, uint32_t& w, int64_t& ca, int64_t& cb, int64_t& cab,
-                                           uint64_t& bytes) {
+                                           uint32_t dn, uint32_t& u, uint32_t& w, int64_t& ca, int64_t& cb,
+                                           int64_t& cab, uint64_t& bytes) {
   u = 0;
   w = 0;
 #pragma unroll
@@ -457,18 +487,25 @@ __device__ __forceinline__ void pair_bases(const GView& g, const KPlan& P, const
     if (l == (int)P.pr_a) u = r[l];
     if (l == (int)P.pr_b) w = r[l];
   }
-  ca = tbl_or_deg(g, pt.a, u);
-  cb = tbl_or_deg(g, pt.b, w);
+  if (dn == ~0u) dn = g.sig[2 * (uint64_t)r[N - 1]];
+  const bool na = P.pr_a == (uint32_t)(N - 1), nb = P.pr_b == (uint32_t)(N - 1);  // an owner is the newest vertex
+  ca = pt.a ? pt.a[u] : na ? dn : g.off_out[u + 1] - g.off_out[u];
+  cb = pt.b ? pt.b[w] : nb ? dn : g.off_out[w + 1] - g.off_out[w];
   cab = 0;
   if (P.pr_a == P.pr_b) cab = (int64_t)tbl_or_deg(g, pt.ab, u);
-  else if (g.h2_off && P.pr_tab <= 2) cab = (int64_t)two_hop(g, u, w, bytes);
-  else if (g.arc_cn && P.pr_adj && P.pr_tab <= 2) cab = (int64_t)arc_common(g, u, w, bytes);
+  else if (P.pr_tab <= 2 && (g.h2_off || (g.arc_cn && P.pr_adj)))
+    cab = (int64_t)(nb ? index_common(g, u, w, bytes) : index_common(g, w, u, bytes));
   bytes += 16 + 4 * N;
 #pragma unroll
   for (int l = 0; l < N; ++l) {
-    const bool ina = ((P.pr_ma >> l) & 1) || adj_has(g, u, r[l], bytes);
-    const bool inb = ((P.pr_mb >> l) & 1) || adj_has(g, w, r[l], bytes);
-    const uint32_t d = g.sig[2 * (uint64_t)r[l]];
+    // no vertex is in its own list; the test runs in the list of the older
+    // vertex, which the lanes of a prefix share
+    const bool ina = ((P.pr_ma >> l) & 1) || (l != (int)P.pr_a && adj_has(g, na ? r[l] : u, na ? u : r[l], bytes));
+    const bool inb = P.pr_a == P.pr_b ? ina
+                                      : ((P.pr_mb >> l) & 1) ||
+                                            (l != (int)P.pr_b && adj_has(g, nb ? r[l] : w, nb ? w : r[l], bytes));
+    if (!ina && !inb) continue;
+    const uint32_t d = l == N - 1 ? dn : g.sig[2 * (uint64_t)r[l]];
     ca -= ina && d >= P.pr_ta;
     cb -= inb && d >= P.pr_tb;
     cab -= ina && inb && d >= P.pr_tab;
@@ -482,11 +519,11 @@ __device__ __forceinline__ void pair_bases(const GView& g, const KPlan& P, const
 // the prefix's and its children's expansions.
 template <int N>
 __device__ __forceinline__ uint64_t tail_count(const GView& g, const KPlan& P, const uint32_t (&r)[N],
-                                               const PairTables& pt, bool stats, uint64_t& na, uint64_t& mb,
-                                               uint64_t& bytes) {
+                                               const PairTables& pt, uint32_t dn, bool stats, uint64_t& na,
+                                               uint64_t& mb, uint64_t& bytes) {
   uint32_t u, w;
   int64_t ca, cb, cab;
-  pair_bases<N>(g, P, r, pt, u, w, ca, cb, cab, bytes);
+  pair_bases<N>(g, P, r, pt, dn, u, w, ca, cb, cab, bytes);
   const bool one = P.tl_kind == 1;
   const int64_t n = one ? ca : cab;
   na += (uint64_t)n;
@@ -562,7 +599,7 @@ __device__ __forceinline__ uint32_t plan_row(const GView& g, const KPlan& P, con
     uint32_t u = 0, w = 0;
     int64_t ca = 0, cb = 0, cab = 0;
     uint64_t dummy = 0;
-    pair_bases<L>(g, P, row, pt, u, w, ca, cb, cab, dummy);
+    pair_bases<L>(g, P, row, pt, ~0u, u, w, ca, cb, cab, dummy);
     pbase[p] = make_uint4((uint32_t)ca, (uint32_t)cb, (uint32_t)(int32_t)cab, 0u);
     if (collapse) {
       // position k-3's survivors are N(u) & N(w) minus the prefix (cab of
@@ -1082,17 +1119,21 @@ struct ChainTables {
 // each of its |A| children by its own list.
 template <int N>
 __device__ __forceinline__ int64_t chain_closed(const GView& g, const KPlan& P, const uint32_t (&r)[N],
-                                                const ChainTables& t, uint32_t shared, bool h2, int64_t& na,
-                                                bool stats, uint64_t& mb, uint64_t& bytes) {
+                                                const ChainTables& t, uint32_t shared, bool h2, uint32_t dn,
+                                                int64_t& na, bool stats, uint64_t& mb, uint64_t& bytes) {
   uint64_t& dummy = bytes;
   bytes += 4 * N + 8 + 8 + (t.ta ? 4 : 0);  // degrees of the row, u's offsets, H(u), cnt_ta(u)
   uint32_t u = 0, d[N];
 #pragma unroll
   for (int l = 0; l < N; ++l) {
     if (l == (int)P.ch_u) u = r[l];
-    d[l] = g.sig[2 * (uint64_t)r[l]];
+    d[l] = l == N - 1 && dn != ~0u ? dn : g.sig[2 * (uint64_t)r[l]];
   }
-  const uint32_t du = g.off_out[u + 1] - g.off_out[u];
+  // (loop-free symmetric graphs: the signature is the degree)
+  uint32_t du = d[0];
+#pragma unroll
+  for (int l = 1; l < N; ++l)
+    if (l == (int)P.ch_u) du = d[l];
   // prefix vertices inside N(u) that meet ta
   uint32_t inu = 0;
 #pragma unroll
@@ -1106,8 +1147,8 @@ __device__ __forceinline__ int64_t chain_closed(const GView& g, const KPlan& P, 
 #pragma unroll
   for (int l = 0; l < N; ++l)
     if ((inu >> l) & 1) {
-      c -= t.tb ? t.tb[r[l]] : g.off_out[r[l] + 1] - g.off_out[r[l]];
-      dsum += g.off_out[r[l] + 1] - g.off_out[r[l]];
+      c -= t.tb ? t.tb[r[l]] : d[l];
+      dsum += d[l];
       bytes += t.tb ? 4 : 8;
     }
   if (P.ch_tb <= 1 || du >= P.ch_tb) c -= na;
@@ -1117,11 +1158,12 @@ __device__ __forceinline__ int64_t chain_closed(const GView& g, const KPlan& P, 
 #pragma unroll
     for (int j = 0; j < N; ++j) {
       if (j == i || !((inu >> j) & 1)) continue;
-      if (((P.qadj[i] >> j) & 1) || adj_has(g, r[i], r[j], dummy)) ++c;
+      // (in the list of the older vertex, which the lanes of a prefix share)
+      if (((P.qadj[i] >> j) & 1) || adj_has(g, i < j ? r[i] : r[j], i < j ? r[j] : r[i], dummy)) ++c;
     }
   }
   c -= (int64_t)shared;
-  if (h2 && (P.ch_tb <= 1 || d[N - 1] >= P.ch_tb)) c -= two_hop(g, u, r[N - 1], dummy);
+  if (h2 && (P.ch_tb <= 1 || d[N - 1] >= P.ch_tb)) c -= index_common(g, u, r[N - 1], dummy);
   if (stats) mb += 8 + 4ull * du + 24ull * (uint64_t)na + 4ull * (t.H[g.V + u] - dsum);
   return c;
 }
@@ -1297,6 +1339,38 @@ __global__ __launch_bounds__(BLOCK) void k_expand(GView g, KPlan P, ExpandArgs a
   const uint32_t nj = P.nj[L];
   const uint32_t tin = P.sig_in[L], tout = P.sig_out[L];
   uint64_t acc = 0, valid = 0, pairs = 0, trips = 0, bytes = 0, mb = 0;
+  // modes whose survivors wait in a queue of their wave: prefix, vertex,
+  // degree (at most 63 left over and 64 new)
+  constexpr bool QUEUED = MODE == M_TAIL || MODE == M_CHAIN;
+  __shared__ uint32_t s_q[QUEUED ? BLOCK / 64 : 1][3][QUEUED ? 128 : 1];
+  uint32_t nq = 0;
+  // counts the queue's entry i, a survivor v that completes the prefix of
+  // positions 0..k-3, whose last two positions are counted together
+  auto count_queued = [&](uint32_t i, bool on) {
+    // the wave's queue writes come before these reads (its LDS accesses
+    // execute in order)
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    if (on) {
+      const uint64_t p = s_q[wave][0][i];
+      const uint32_t dv = s_q[wave][2][i];
+      uint32_t r[L + 1];
+#pragma unroll
+      for (int l = 0; l < L; ++l) r[l] = a.rows[p * L + l];
+      r[L] = s_q[wave][1][i];
+      ++valid;
+      if constexpr (MODE == M_TAIL) {
+        acc += tail_count<L + 1>(g, P, r, a.ptab, dv, a.stats != 0, pairs, mb, bytes);
+      } else if constexpr (MODE == M_CHAIN) {
+        int64_t na = 0;
+        acc += (uint64_t)chain_closed<L + 1>(g, P, r, a.ctab, a.shared[p], true, dv, na, a.stats != 0, mb, bytes);
+        pairs += (uint64_t)na;
+      }
+      if (a.stats) mb += 16;  // the survivor's node, written and read back
+    }
+    __builtin_amdgcn_wave_barrier();
+  };
   // Tiles (next_tile): static for a launch with no more tiles than blocks,
   // else dynamic and XCD-aware.  The fetch runs in wave 0 under a
   // wave-uniform branch, so the branches at the edges of this barrier loop
@@ -1527,7 +1601,7 @@ __global__ __launch_bounds__(BLOCK) void k_expand(GView g, KPlan P, ExpandArgs a
             r[L] = v[j];
             uint32_t u, w;
             int64_t ca, cb, cab;
-            pair_bases<L + 1>(g, P, r, a.ptab, u, w, ca, cb, cab, bytes);
+            pair_bases<L + 1>(g, P, r, a.ptab, sg[j].x, u, w, ca, cb, cab, bytes);
             acc += (uint64_t)(cab * ((ca - 1) * (cb - 1) - (cab - 1)));
             pairs += (uint64_t)cab;
             trips += (uint64_t)(cab * (ca - 1));
@@ -1540,36 +1614,32 @@ __global__ __launch_bounds__(BLOCK) void k_expand(GView g, KPlan P, ExpandArgs a
               mb += 16 + 16 + 4 * (du + dw) + (uint64_t)cab * (24 + 4 * du + (uint64_t)(ca - 1) * (24 + 4 * dw));
             }
           }
-        } else if (MODE == M_TAIL) {
-          // a survivor v completes the prefix of positions 0..k-3, whose last
-          // two positions are counted from it (tail_count)
+        } else if (QUEUED) {
+          // survivors queue up in LDS and are counted 64 at a time: where few
+          // items survive (4% of the R-MAT 20 5-cycle query's), counting them
+          // where they are found runs the closed form for a few lanes of
+          // every wave
+#pragma unroll 1
+          for (int it = 0; it < G; ++it) {
+            const uint64_t m = __ballot(ok[0]);
+            if (ok[0]) {
+              const uint32_t at = nq + lane_rank(m);
+              s_q[wave][0][at] = plo + min(pi[0], span - 1);
+              s_q[wave][1][at] = v[0];
+              s_q[wave][2][at] = sg[0].x;
+            }
+            nq += (uint32_t)__popcll(m);
 #pragma unroll
-          for (int j = 0; j < G; ++j) {
-            if (!ok[j]) continue;
-            ++valid;
-            uint32_t r[L + 1];
-#pragma unroll
-            for (int l = 0; l < L; ++l) r[l] = row[j][l];
-            r[L] = v[j];
-            acc += tail_count<L + 1>(g, P, r, a.ptab, a.stats != 0, pairs, mb, bytes);
-            if (a.stats) mb += 16;  // the survivor's node, written and read back
-          }
-        } else if (MODE == M_CHAIN) {
-          // a survivor v completes the prefix of positions 0..k-3, whose
-          // chain of the last two positions is counted in closed form
-#pragma unroll
-          for (int j = 0; j < G; ++j) {
-            if (!ok[j]) continue;
-            ++valid;
-            uint32_t r[L + 1];
-#pragma unroll
-            for (int l = 0; l < L; ++l) r[l] = row[j][l];
-            r[L] = v[j];
-            const uint32_t sh = a.shared[plo + min(pi[j], span - 1)];
-            int64_t na = 0;
-            acc += (uint64_t)chain_closed<L + 1>(g, P, r, a.ctab, sh, true, na, a.stats != 0, mb, bytes);
-            pairs += (uint64_t)na;
-            if (a.stats) mb += 16;  // the survivor's node, written and read back
+            for (int j = 0; j + 1 < G; ++j) {
+              ok[j] = ok[j + 1];
+              pi[j] = pi[j + 1];
+              v[j] = v[j + 1];
+              sg[j] = sg[j + 1];
+            }
+            if (nq >= 64) {
+              nq -= 64;
+              count_queued(nq + (tid & 63), true);
+            }
           }
         } else if (MODE == M_PAIR) {
           // a survivor v completes the prefix of positions 0..k-3; its
@@ -1708,6 +1778,7 @@ __global__ __launch_bounds__(BLOCK) void k_expand(GView g, KPlan P, ExpandArgs a
     __syncthreads();
     }
   }
+  if constexpr (QUEUED) count_queued(tid & 63, (tid & 63) < nq);
   if constexpr (MODE == M_WRITE) {
     if (a.publish && tid == 0) {
       // every block that took part (the grid, or one block per tile when
@@ -1884,7 +1955,7 @@ __global__ __launch_bounds__(BLOCK) void k_chain_sib(GView g, KPlan P, SibArgs a
         if (v == r[L - 1]) continue;
         ++valid;
         int64_t na = 0;
-        acc += (uint64_t)chain_closed<L + 1>(g, P, r, t, a.shared[q], true, na, true, mb, bytes);
+        acc += (uint64_t)chain_closed<L + 1>(g, P, r, t, a.shared[q], true, ~0u, na, true, mb, bytes);
         pairs += (uint64_t)na;
         mb += 16;  // the survivor's node, written and read back
       }
@@ -2034,7 +2105,7 @@ __global__ __launch_bounds__(BLOCK) void k_tail_row(GView g, KPlan P, const uint
 #pragma unroll
     for (int l = 0; l < L; ++l) r[l] = rows[p * L + l];
     bytes += 4 * L;
-    acc += tail_count<L>(g, P, r, pt, stats != 0, na, mb, bytes);
+    acc += tail_count<L>(g, P, r, pt, ~0u, stats != 0, na, mb, bytes);
     if (known) continue;
     const uint32_t u = rows[p * L + P.pr_a], w = rows[p * L + P.pr_b];
     const uint32_t hc = hub ? hub_common(g, u, w) : ~0u;
@@ -2313,7 +2384,7 @@ __global__ __launch_bounds__(BLOCK) void k_chain_row(GView g, KPlan P, const uin
 #pragma unroll
     for (int l = 0; l < L; ++l) r[l] = rows[p * L + l];
     int64_t na = 0;
-    int64_t c = chain_closed<L>(g, P, r, t, shared[parent[p]], h2, na, stats != 0, mb, bytes);
+    int64_t c = chain_closed<L>(g, P, r, t, shared[parent[p]], h2, ~0u, na, stats != 0, mb, bytes);
     bytes += 4 * L + 8;  // the row and its parent's shared sum
     na_sum += (uint64_t)na;
     uint32_t u = 0;
