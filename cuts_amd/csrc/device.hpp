@@ -203,9 +203,10 @@ struct Context {
   uint64_t default_budget = 0;
   LevelBuf lv[kMaxQuery];
   // [0] embeddings, [1] level k-2 size of the fused or chain level (level
-  // k-3 with the pair level), [2] level k-2 size of the pair level, [3] demand bytes, [4..7] eight
-  // uint32 tile counters, [8] merge-model bytes, [10] rows written by one
-  // expansion
+  // k-3 with the pair level), [2] level k-2 size of the pair level, [3] demand
+  // bytes, [8] merge-model bytes, [10] rows written by one expansion; then the
+  // slots of the sums and the tile counters (kSlots in match.hip), and a copy
+  // of all for a run that may be cut short
   unsigned long long* counters = nullptr;
   hipEvent_t kev[2] = {nullptr, nullptr};
   // embedding output: rows of the last level are copied to the caller's

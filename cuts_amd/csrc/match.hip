@@ -366,6 +366,21 @@ __device__ __forceinline__ void add_wave(unsigned long long* dst, uint64_t v) {
   if ((threadIdx.x & 63) == 0 && s) atomicAdd(dst, (unsigned long long)s);
 }
 
+// The run's counter words (Context::counters): 16 words, then kSlots slots of
+// the words that every wave of a counting launch adds to (0, 1, 2 and 9), then
+// the tile counters, slots and counters on lines of their own.  Device-scope
+// atomics of all XCDs on one line are served one after another, about 13 ns
+// each: the 18,000 final adds of a full grid took 230 of the 310 us of the
+// 4,096-vertex graph's triangle + 2-edge tail.  k_publish_end adds the slots up.
+constexpr uint32_t kSlots = 64, kLine = 32, kSlot0 = kLine, kTile0 = kSlot0 + kSlots * kLine,
+                   kCounterWords = kTile0 + 8 * kLine;
+constexpr uint32_t kTileStride = 2 * kLine;  // 32-bit words between tile counters
+
+// Adds a wave's sum to word i (0, 1, 2 or 9) in the block's slot.
+__device__ __forceinline__ void add_sum(unsigned long long* counters, int i, uint64_t v) {
+  add_wave(&counters[kSlot0 + (blockIdx.x % kSlots) * kLine + i], v);
+}
+
 // ---------------------------------------------------------------- level 0
 // Level 0 in ascending vertex order: a 0/1 flag per candidate vertex, an
 // exclusive scan of the flags, and a scatter.  A deterministic level 0 makes
@@ -436,16 +451,27 @@ static __global__ __launch_bounds__(L0_THREADS) void k_level0_small(const uint32
   }
 }
 
-// The run's counters (words 0..13), the last processed root (*last, or
+// The run's counters (words 0..13, with their slots), the last processed root (*last, or
 // rows0[lvcnt[0] - 1] when level 0's size stayed on the device), and the
 // device-side level counts (16 words, to pub[48..]), written to host memory
 // (system-scope stores) for one synchronisation with no copy.
+static_assert(kSlots == 64, "a lane per slot");
 static __global__ void k_publish_end(const unsigned long long* __restrict__ ctr, const uint32_t* __restrict__ last,
                               const uint32_t* __restrict__ rows0, const unsigned long long* __restrict__ lvcnt,
                               uint64_t* pub) {
   const uint32_t t = threadIdx.x;
+  // the slots' sums, in every lane
+  uint64_t sum[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    uint64_t v = ctr[kSlot0 + t * kLine + (i < 3 ? i : 9)];
+    for (int o = 32; o > 0; o >>= 1)
+      v += ((uint64_t)__shfl_xor((uint32_t)(v >> 32), o) << 32) | __shfl_xor((uint32_t)v, o);
+    sum[i] = v;
+  }
   if (t < 14) {
-    __hip_atomic_store(&pub[t], (uint64_t)__hip_atomic_load(&ctr[t], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT),
+    const uint64_t more = t == 0 ? sum[0] : t == 1 ? sum[1] : t == 2 ? sum[2] : t == 9 ? sum[3] : 0ull;
+    __hip_atomic_store(&pub[t], (uint64_t)__hip_atomic_load(&ctr[t], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + more,
                        __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
   } else if (t == 14 && (last || rows0)) {
     const uint64_t n0 = rows0 ? lvcnt[0] : 1;
@@ -633,9 +659,9 @@ __global__ __launch_bounds__(BLOCK) void k_plan(GView g, KPlan P, const uint32_t
                             sna);
   if (merge) add_wave(merge, mb);
   if (collapse) {
-    add_wave(&counters[0], acc);
-    add_wave(&counters[1], surv);
-    add_wave(&counters[2], sna);
+    add_sum(counters, 0, acc);
+    add_sum(counters, 1, surv);
+    add_sum(counters, 2, sna);
   }
 }
 
@@ -790,7 +816,7 @@ static __global__ __launch_bounds__(BLOCK) void k_tile_index(const uint64_t* __r
                                                      unsigned int* __restrict__ tilectr,
                                                      unsigned int* __restrict__ outctr) {
   if (blockIdx.x == 0) {
-    if (threadIdx.x < 8) tilectr[threadIdx.x] = 0u;
+    if (threadIdx.x < 8) tilectr[threadIdx.x * kTileStride] = 0u;
     if (outctr && threadIdx.x < 2) outctr[threadIdx.x] = 0u;
   }
   for (uint64_t t = (uint64_t)blockIdx.x * BLOCK + threadIdx.x; t <= ntiles; t += (uint64_t)gridDim.x * BLOCK) {
@@ -832,7 +858,7 @@ static __global__ __launch_bounds__(BLOCK) void k_tile_index_dyn(const uint64_t*
   const uint64_t nt = (W + TILE - 1) / TILE;
   const bool fits = W <= max_items && nt + 1 <= tile_cap && W <= row_cap;
   if (blockIdx.x == 0) {
-    if (threadIdx.x < 8) tilectr[threadIdx.x] = 0u;
+    if (threadIdx.x < 8) tilectr[threadIdx.x * kTileStride] = 0u;
     if (outctr && threadIdx.x < 2) outctr[threadIdx.x] = 0u;
     if (threadIdx.x == 0) {
       dyn[0] = fits ? W : 0ull;
@@ -912,9 +938,9 @@ __global__ __launch_bounds__(BLOCK) void k_plan_small(GView g, KPlan P, const ui
     sum += v[i];
   }
   if (collapse) {
-    add_wave(&counters[0], acc);
-    add_wave(&counters[1], surv);
-    add_wave(&counters[2], sna);
+    add_sum(counters, 0, acc);
+    add_sum(counters, 1, surv);
+    add_sum(counters, 2, sna);
   }
   uint64_t W;
   uint64_t ex = block_excl_scan(sum, s_tmp, &W);
@@ -933,7 +959,7 @@ __global__ __launch_bounds__(BLOCK) void k_plan_small(GView g, KPlan P, const ui
   }
   const uint64_t nt = (W + TILE - 1) / TILE;
   const bool fits = !too_big && W <= max_items && nt + 1 <= tile_cap && W <= row_cap;
-  if (threadIdx.x < 8) tilectr[threadIdx.x] = 0u;
+  if (threadIdx.x < 8) tilectr[threadIdx.x * kTileStride] = 0u;
   if (outctr && threadIdx.x < 2) outctr[threadIdx.x] = 0u;
   if (threadIdx.x == 0) {
     dyn[0] = fits ? W : 0ull;
@@ -1080,7 +1106,7 @@ __global__ __launch_bounds__(BLOCK) void k_closed_form(GView g, KPlan P, const u
       mb += 8 + 4ull * (g.off_out[u + 1] - g.off_out[u]);
     }
   }
-  add_wave(&counters[0], acc);
+  add_sum(counters, 0, acc);
   if (stats) {
     add_wave(&counters[3], bytes);
     add_wave(&counters[8], mb);
@@ -1229,7 +1255,7 @@ struct ExpandArgs {
   const uint64_t* coff;      // M_GWRITE: start of every prefix's block in cand
   uint32_t* cand;            // M_GWRITE: candidates grouped by prefix
   uint32_t xcd;              // 1: XCD-contiguous tile mapping
-  unsigned int* tilectr;     // 8 tile counters, zero at launch
+  unsigned int* tilectr;     // 8 tile counters kTileStride apart, zero at launch
   uint32_t stats;            // 1: accumulate demand bytes into counters[3]
   // non-null: {w_end, ntiles} of this launch, written on the device by
   // k_tile_index_dyn (w_begin is 0), in place of w_end and ntiles
@@ -1303,7 +1329,7 @@ __device__ __forceinline__ uint64_t next_tile(unsigned int* tilectr, uint64_t nt
     const uint32_t xx = (myx + tries) % nx;
     const uint64_t lo = ntiles * xx / nx, hi = ntiles * (xx + 1) / nx;
     uint32_t got = 0;
-    if (lane == 0) got = atomicAdd(&tilectr[xx], 1u);
+    if (lane == 0) got = atomicAdd(&tilectr[xx * kTileStride], 1u);
     const uint64_t i = uni(got);
     if (lo + i < hi) return lo + i;
     // this share is drained: one counter load per lane finds the shares
@@ -1313,7 +1339,7 @@ __device__ __forceinline__ uint64_t next_tile(unsigned int* tilectr, uint64_t nt
     bool left = false;
     if (lane < nx) {
       const uint32_t yy = (myx + lane) % nx;
-      const uint64_t c = __hip_atomic_load(&tilectr[yy], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      const uint64_t c = __hip_atomic_load(&tilectr[yy * kTileStride], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       left = ntiles * yy / nx + c < ntiles * (yy + 1) / nx;
     }
     const uint64_t m = __ballot(left);
@@ -1796,11 +1822,11 @@ __global__ __launch_bounds__(BLOCK) void k_expand(GView g, KPlan P, ExpandArgs a
     }
   }
   if (MODE != M_WRITE) {
-    add_wave(&a.counters[0], acc);
+    add_sum(a.counters, 0, acc);
     if (MODE == M_FUSED || MODE == M_PAIR || MODE == M_CHAIN || MODE == M_COLLAPSE || MODE == M_TAIL)
-      add_wave(&a.counters[1], valid);
-    if (MODE == M_PAIR || MODE == M_CHAIN || MODE == M_COLLAPSE || MODE == M_TAIL) add_wave(&a.counters[2], pairs);
-    if (MODE == M_COLLAPSE) add_wave(&a.counters[9], trips);
+      add_sum(a.counters, 1, valid);
+    if (MODE == M_PAIR || MODE == M_CHAIN || MODE == M_COLLAPSE || MODE == M_TAIL) add_sum(a.counters, 2, pairs);
+    if (MODE == M_COLLAPSE) add_sum(a.counters, 9, trips);
   }
   if (a.stats) {
     add_wave(&a.counters[3], bytes);
@@ -2006,9 +2032,9 @@ __global__ __launch_bounds__(BLOCK) void k_chain_sib(GView g, KPlan P, SibArgs a
     }
     __syncthreads();
   }
-  add_wave(&a.counters[0], acc);
-  add_wave(&a.counters[1], valid);
-  add_wave(&a.counters[2], pairs);
+  add_sum(a.counters, 0, acc);
+  add_sum(a.counters, 1, valid);
+  add_sum(a.counters, 2, pairs);
   if (a.stats) {
     add_wave(&a.counters[3], bytes);
     add_wave(&a.counters[8], mb);
@@ -2061,7 +2087,7 @@ __global__ __launch_bounds__(BLOCK) void k_pair_prep(GView g, KPlan P, const uin
     minlen[p] = len;
     minsel[p] = (uint8_t)sel;
   }
-  add_wave(&counters[0], acc);
+  add_sum(counters, 0, acc);
 }
 
 // Chain level, shared part: the work of N(u) & N(r_i) for one older
@@ -2123,8 +2149,8 @@ __global__ __launch_bounds__(BLOCK) void k_tail_row(GView g, KPlan P, const uint
     minlen[p] = len;
     minsel[p] = (uint8_t)sel;
   }
-  add_wave(&counters[0], acc);
-  add_wave(&counters[1], na);
+  add_sum(counters, 0, acc);
+  add_sum(counters, 1, na);
   if (stats) {
     add_wave(&counters[8], mb);
     add_wave(&counters[3], bytes);
@@ -2287,7 +2313,7 @@ __global__ __launch_bounds__(BLOCK) void k_common(GView g, KPlan P, ExpandArgs a
     }
     __syncthreads();
   }
-  if (c.mode != 2) add_wave(&a.counters[0], acc);
+  if (c.mode != 2) add_sum(a.counters, 0, acc);
   if (a.stats) add_wave(&a.counters[3], bytes);
 }
 
@@ -2407,8 +2433,8 @@ __global__ __launch_bounds__(BLOCK) void k_chain_row(GView g, KPlan P, const uin
     minlen[p] = (!known && need) ? min(du, dv) : 0u;
     minsel[p] = (uint8_t)(du <= dv ? 0u : 1u);
   }
-  add_wave(&counters[0], acc);
-  add_wave(&counters[1], na_sum);
+  add_sum(counters, 0, acc);
+  add_sum(counters, 1, na_sum);
   if (stats) {
     add_wave(&counters[8], mb);
     add_wave(&counters[3], bytes);
@@ -2738,7 +2764,7 @@ struct Matcher {
     const uint32_t tg = (uint32_t)std::min<uint64_t>((tcap + BLOCK - 1) / BLOCK, 1024);
     hipLaunchKernelGGL(k_tile_index_dyn, dim3(tg), dim3(BLOCK), 0, c.stream, in.work_off, n,
                        outctr ? MAX_CHUNK : MAX_SPEC_ITEMS, tcap, row_cap,
-                       in.tile_p, (unsigned int*)(ctr + 4), outctr, ctr + 14, outctr ? ctr + 11 : ctr + 12, ctr + 13,
+                       in.tile_p, (unsigned int*)(ctr + kTile0), outctr, ctr + 14, outctr ? ctr + 11 : ctr + 12, ctr + 13,
                        publish);
     HIPCHECK(hipGetLastError());
     return tcap - 1;
@@ -2848,7 +2874,7 @@ struct Matcher {
       ensure_tiles(arena, in, nt);
       pbegin(false);
       hipLaunchKernelGGL(k_tile_index, dim3(grid_for(nt + 1, BLOCK, 65535)), dim3(BLOCK), 0, c.stream, in.work_off,
-                         n, w0, w1, nt, in.tile_p, (unsigned int*)(ctr + 4), mode == M_WRITE ? (unsigned int*)(ctr + 10) : nullptr);
+                         n, w0, w1, nt, in.tile_p, (unsigned int*)(ctr + kTile0), mode == M_WRITE ? (unsigned int*)(ctr + 10) : nullptr);
       pend(3, (double)(nt + 1) * (8.0 * (64 - __builtin_clzll(n + 2)) + 4.0), false);
       ExpandArgs a{};
       a.rows = rows;
@@ -2872,7 +2898,7 @@ struct Matcher {
       a.ctab = ctab;
       a.ptab = ptbl;
       a.xcd = (o.flags & 8u) ? 0 : 1;
-      a.tilectr = (unsigned int*)(ctr + 4);  // 8 x uint32 in counters[4..7], cleared by k_tile_index
+      a.tilectr = (unsigned int*)(ctr + kTile0);  // cleared by k_tile_index
       a.stats = prof ? 1 : 0;
       uint32_t grid = grid_for(nt, 1, gcap(mclass));
       // counting expansions: nthr threads per block, cgrow times the blocks
@@ -3003,7 +3029,7 @@ struct Matcher {
       ensure_tiles(arena, in, std::max<uint64_t>(in.tile_cap, 4097) - 1);
       tmax = in.tile_cap - 1;
       unsigned int* oc = mode == M_WRITE ? (unsigned int*)(ctr + 10) : nullptr;
-#define PSM(LL) hipLaunchKernelGGL((k_plan_small<LL>), dim3(1), dim3(BLOCK), 0, c.stream, g, kp, rows, n, in.minlen, in.minsel, use_cbase ? in.cbase : nullptr, tbl, mode == M_PAIR ? in.pbase : nullptr, ptbl, ctr, in.work_off, oc ? MAX_CHUNK : MAX_SPEC_ITEMS, in.tile_cap, row_cap, in.tile_p, (unsigned int*)(ctr + 4), oc, ctr + 14, st_word, ctr + 13, oc ? pub_dev : nullptr, dn, dn ? c.lvcnt + (L - 1) : nullptr)
+#define PSM(LL) hipLaunchKernelGGL((k_plan_small<LL>), dim3(1), dim3(BLOCK), 0, c.stream, g, kp, rows, n, in.minlen, in.minsel, use_cbase ? in.cbase : nullptr, tbl, mode == M_PAIR ? in.pbase : nullptr, ptbl, ctr, in.work_off, oc ? MAX_CHUNK : MAX_SPEC_ITEMS, in.tile_cap, row_cap, in.tile_p, (unsigned int*)(ctr + kTile0), oc, ctr + 14, st_word, ctr + 13, oc ? pub_dev : nullptr, dn, dn ? c.lvcnt + (L - 1) : nullptr)
       CUTS_DISPATCH_L(L, PSM)
 #undef PSM
       HIPCHECK(hipGetLastError());
@@ -3027,7 +3053,7 @@ struct Matcher {
     a.ctab = ctab;
     a.ptab = ptbl;
     a.xcd = (o.flags & 8u) ? 0 : 1;
-    a.tilectr = (unsigned int*)(ctr + 4);
+    a.tilectr = (unsigned int*)(ctr + kTile0);
     a.stats = 0;
     const int mclass = mode == M_WRITE ? 4 : mode == M_COUNT ? 5 : (mode == M_FUSED || mode == M_TAIL) ? 6 : (mode == M_PAIR || mode == M_COLLAPSE) ? 8 : 10;
     const uint32_t grid = grid_for(tmax, 1, gcap(mclass));
@@ -3158,7 +3184,7 @@ struct Matcher {
       a.counters = ctr;
       a.nsurv = weight;
       a.xcd = (o.flags & 8u) ? 0 : 1;
-      a.tilectr = (unsigned int*)(ctr + 4);
+      a.tilectr = (unsigned int*)(ctr + kTile0);
       a.stats = 0;
       r.chunks++;
 #define PCS(LL) hipLaunchKernelGGL((k_common<LL>), dim3(grid_for(tmax, 1, gcap(9))), dim3(BLOCK), 0, c.stream, g, kp, a, ca)
@@ -3177,7 +3203,7 @@ struct Matcher {
       ensure_tiles(arena, in, nt);
       pbegin(false);
       hipLaunchKernelGGL(k_tile_index, dim3(grid_for(nt + 1, BLOCK, 65535)), dim3(BLOCK), 0, c.stream, in.work_off,
-                         n, w0, w1, nt, in.tile_p, (unsigned int*)(ctr + 4), nullptr);
+                         n, w0, w1, nt, in.tile_p, (unsigned int*)(ctr + kTile0), nullptr);
       pend(3, (double)(nt + 1) * (8.0 * (64 - __builtin_clzll(n + 2)) + 4.0), false);
       ExpandArgs a{};
       a.rows = rows;
@@ -3190,7 +3216,7 @@ struct Matcher {
       a.counters = ctr;
       a.nsurv = weight;
       a.xcd = (o.flags & 8u) ? 0 : 1;
-      a.tilectr = (unsigned int*)(ctr + 4);
+      a.tilectr = (unsigned int*)(ctr + kTile0);
       a.stats = prof ? 1 : 0;
       r.chunks++;
       pbegin(true);
@@ -3259,7 +3285,7 @@ struct Matcher {
       const uint64_t nt = (w1 - w0 + TILE - 1) / TILE;
       ensure_tiles(arena, in, nt);
       hipLaunchKernelGGL(k_tile_index, dim3(grid_for(nt + 1, BLOCK, 65535)), dim3(BLOCK), 0, c.stream, in.work_off,
-                         n, w0, w1, nt, in.tile_p, (unsigned int*)(ctr + 4), nullptr);
+                         n, w0, w1, nt, in.tile_p, (unsigned int*)(ctr + kTile0), nullptr);
       ExpandArgs a{};
       a.rows = rows;
       a.work_off = in.work_off;
@@ -3273,7 +3299,7 @@ struct Matcher {
       a.coff = in.coff;
       a.cand = in.cand;
       a.xcd = (o.flags & 8u) ? 0 : 1;
-      a.tilectr = (unsigned int*)(ctr + 4);
+      a.tilectr = (unsigned int*)(ctr + kTile0);
       a.stats = prof ? 1 : 0;
       r.chunks++;
       const uint32_t grid = grid_for(nt, 1, gcap(4));
@@ -3358,7 +3384,7 @@ struct Matcher {
       const uint64_t nt = (w1 - w0 + TILE - 1) / TILE;
       ensure_tiles(arena, in, nt);
       hipLaunchKernelGGL(k_tile_index, dim3(grid_for(nt + 1, BLOCK, 65535)), dim3(BLOCK), 0, c.stream, in.work_off,
-                         n, w0, w1, nt, in.tile_p, (unsigned int*)(ctr + 4), nullptr);
+                         n, w0, w1, nt, in.tile_p, (unsigned int*)(ctr + kTile0), nullptr);
       SibArgs a{};
       a.rows = rows;
       a.pb = in.pbase;
@@ -3371,7 +3397,7 @@ struct Matcher {
       a.w_end = w1;
       a.ntiles = nt;
       a.counters = ctr;
-      a.tilectr = (unsigned int*)(ctr + 4);
+      a.tilectr = (unsigned int*)(ctr + kTile0);
       a.xcd = (o.flags & 8u) ? 0 : 1;
       a.stats = prof ? 1 : 0;
       r.chunks++;
@@ -3486,8 +3512,8 @@ struct Matcher {
     LevelBuf& l0 = lv[0];
     ensure_rows(arena, l0, std::max<uint32_t>(n0c, 1), 1);
     // counts, tile counters, merge bytes, level counts, rows written,
-    // speculation status words and device-side work: one clear
-    HIPCHECK(hipMemsetAsync(ctr, 0, 14 * 8, c.stream));
+    // speculation status words, device-side work and the sums' slots: one clear
+    HIPCHECK(hipMemsetAsync(ctr, 0, kTile0 * 8, c.stream));
     HIPCHECK(hipEventRecord(c.ev0, c.stream));
     const auto t_start = std::chrono::steady_clock::now();
     uint64_t n0 = 0;
@@ -3539,23 +3565,23 @@ struct Matcher {
       }
       for (uint64_t s = 0; s < n0; s += ts) {
         // snapshot so that a trunk interrupted by the deadline can be undone
-        uint64_t snap[3] = {0, 0, 0};
         uint64_t snap_level[kMaxQuery];
         std::memcpy(snap_level, r.level, sizeof(snap_level));
         if (has_deadline && !write) {
           if (past_deadline()) break;
-          HIPCHECK(hipMemcpyAsync(c.host_pinned, ctr, 24, hipMemcpyDeviceToHost, c.stream));
-          HIPCHECK(hipStreamSynchronize(c.stream));
-          snap[0] = c.host_pinned[0];
-          snap[1] = c.host_pinned[1];
-          snap[2] = c.host_pinned[2];
+          HIPCHECK(hipMemcpyAsync(ctr + kCounterWords, ctr, kTile0 * 8, hipMemcpyDeviceToDevice, c.stream));
         }
         level(1, l0.rows + s, std::min(ts, n0 - s), (chained_mask & 1u) ? ctr + 10 : nullptr);
         if (aborted) {
-          c.host_pinned[0] = snap[0];
-          c.host_pinned[1] = snap[1];
-          c.host_pinned[2] = snap[2];
-          HIPCHECK(hipMemcpyAsync(ctr, c.host_pinned, 24, hipMemcpyHostToDevice, c.stream));
+          // words 0..2 and the slots (a work cap has no snapshot: its count is void)
+          if (has_deadline) {
+            HIPCHECK(hipMemcpyAsync(ctr, ctr + kCounterWords, 24, hipMemcpyDeviceToDevice, c.stream));
+            HIPCHECK(hipMemcpyAsync(ctr + kSlot0, ctr + kCounterWords + kSlot0, (kTile0 - kSlot0) * 8,
+                                    hipMemcpyDeviceToDevice, c.stream));
+          } else {
+            HIPCHECK(hipMemsetAsync(ctr, 0, 24, c.stream));
+            HIPCHECK(hipMemsetAsync(ctr + kSlot0, 0, (kTile0 - kSlot0) * 8, c.stream));
+          }
           HIPCHECK(hipStreamSynchronize(c.stream));
           std::memcpy(r.level, snap_level, sizeof(snap_level));
           break;
@@ -3860,7 +3886,7 @@ void context_init(Context& c, int device) {
   HIPCHECK(hipStreamCreateWithFlags(&c.copy_stream, hipStreamNonBlocking));
   HIPCHECK(hipEventCreateWithFlags(&c.copy_ev[0], hipEventDisableTiming));
   HIPCHECK(hipEventCreateWithFlags(&c.copy_ev[1], hipEventDisableTiming));
-  HIPCHECK(hipMalloc(&c.counters, 16 * sizeof(unsigned long long)));
+  HIPCHECK(hipMalloc(&c.counters, 2 * kCounterWords * sizeof(unsigned long long)));
   HIPCHECK(hipHostMalloc(&c.host_pinned, 256, hipHostMallocDefault));
   HIPCHECK(hipHostMalloc(&c.host_res, 1024, hipHostMallocCoherent | hipHostMallocMapped));
   HIPCHECK(hipMalloc(&c.lvcnt, kMaxQuery * sizeof(unsigned long long)));
@@ -4110,8 +4136,8 @@ void run_match_noalloc(Context& c, DeviceGraph& dg, const Plan& p, const MatchOp
   ScratchArena a;
   a.base = c.scratch;
   a.size = kScratchBytes;
-  auto* ctr = (unsigned long long*)a.carve(16 * sizeof(unsigned long long));
-  HIPCHECK(hipMemsetAsync(ctr, 0, 16 * sizeof(unsigned long long), c.stream));
+  auto* ctr = (unsigned long long*)a.carve(2 * kCounterWords * sizeof(unsigned long long));
+  HIPCHECK(hipMemsetAsync(ctr, 0, kCounterWords * sizeof(unsigned long long), c.stream));
   LevelBuf lv[kMaxQuery];
   // trie rows take at most an eighth of the scratch; the scan, tile,
   // pair/chain arrays and regrowth take the rest
