@@ -128,7 +128,7 @@ __device__ int64_t chain_closed_rt(const GV& g, const KPlan& P, const uint32_t* 
                                    const uint32_t* __restrict__ tb_tbl, uint32_t shared, int64_t& na) {
   const uint32_t N = L + 1;
   const uint32_t cu = P.ch_u, ta = P.ch_ta, tb = P.ch_tb;
-  const uint32_t u = row[cu];
+  const uint32_t u = cu == L ? v : row[cu];
   const uint32_t du = g.off_out[u + 1] - g.off_out[u];
   uint32_t inu = 0;
   for (uint32_t l = 0; l < N; ++l) {
@@ -153,7 +153,13 @@ __device__ int64_t chain_closed_rt(const GV& g, const KPlan& P, const uint32_t* 
     }
   }
   c -= (int64_t)shared;
-  if (tb <= 1 || g.sig[2 * (uint64_t)v] >= tb) c -= two_hop(g, u, v);
+  if (cu == L) {
+    // the chain on the newest vertex: the intersections with all others
+    for (uint32_t i = 0; i < L; ++i)
+      if (tb <= 1 || g.sig[2 * (uint64_t)row[i]] >= tb) c -= two_hop(g, row[i], u);
+  } else if (tb <= 1 || g.sig[2 * (uint64_t)v] >= tb) {
+    c -= two_hop(g, u, v);
+  }
   return c;
 }
 
@@ -488,8 +494,11 @@ __device__ void process(const BatchArgs& a, Shared<WROW>& s, uint32_t L) {
   // the chain level needs the two-hop index (threshold of A at most 2)
   const bool chain = fuse && !pair && uni(P.ch_ok) && (a.flags & 16u) == 0 && g.h2_off != nullptr && uni(P.ch_ta) <= 2;
   // the last two positions from whole prefixes, inside the expansion of k-3
-  const bool tail = fuse && !pair && uni(P.tl_kind) && (a.flags & 8u) == 0 && k >= 4 &&
-                    (uni(P.pr_a) == uni(P.pr_b) || (g.h2_off != nullptr && uni(P.pr_tab) <= 2));
+  const uint32_t kind = uni(P.tl_kind);
+  const bool tail = fuse && !pair && kind && k >= 4 &&
+                    (kind == 3 ? (a.flags & 16u) == 0 && g.h2_off != nullptr && uni(P.ch_ta) <= 2
+                               : (a.flags & 8u) == 0 && (uni(P.pr_a) == uni(P.pr_b) ||
+                                                         (g.h2_off != nullptr && uni(P.pr_tab) <= 2)));
   uint64_t cnt = 0, surv = 0, sna = 0;
 
   if (L == 0) {
@@ -718,7 +727,8 @@ __device__ void process(const BatchArgs& a, Shared<WROW>& s, uint32_t L) {
         sna += (uint64_t)na;
       } else if (mode == 5) {
         int64_t na = 0;
-        fc = tail_count_rt(g, P, row, L, vv, dv, a.tbls[3 * q + 1], tbl, a.tbls[3 * q + 2], na);
+        fc = kind == 3 ? (uint64_t)chain_closed_rt(g, P, row, L, vv, a.chH[q], a.tbls[3 * q + 1], tbl, 0, na)
+                       : tail_count_rt(g, P, row, L, vv, dv, a.tbls[3 * q + 1], tbl, a.tbls[3 * q + 2], na);
         sna += (uint64_t)na;
       } else if (use_cbase) {
         // v is certainly in N(u) when it was drawn from u's own list
@@ -1007,12 +1017,12 @@ void batch_create(Context& c, DeviceGraph& dg, const std::vector<const Plan*>& p
     b.k.push_back(plans[q]->k);
     b.kmax = std::max(b.kmax, plans[q]->k);
     if (kp[q].sc_ok && kp[q].sc_thr > 1 && !(o.flags & 1u)) tb[3 * q] = cnt_table(c, dg, kp[q].sc_thr);
-    if ((kp[q].pr_ok || kp[q].tl_kind) && !(o.flags & (1u | 2u | 128u))) {
+    if ((kp[q].pr_ok || kp[q].tl_kind == 1 || kp[q].tl_kind == 2) && !(o.flags & (1u | 2u | 128u))) {
       if (kp[q].pr_ta > 1) tb[3 * q + 1] = cnt_table(c, dg, kp[q].pr_ta);
       if (kp[q].pr_tab > 1) tb[3 * q + 2] = cnt_table(c, dg, kp[q].pr_tab);
     }
     // chain level (never together with the pair level): A's table in slot 1
-    if (!kp[q].pr_ok && kp[q].ch_ok && dg.h2_off && kp[q].ch_ta <= 2 && !(o.flags & (1u | 2u | 256u | 512u))) {
+    if (!kp[q].pr_ok && (kp[q].ch_ok || kp[q].tl_kind == 3) && dg.h2_off && kp[q].ch_ta <= 2 && !(o.flags & (1u | 2u | 256u | 512u))) {
       if (kp[q].ch_ta > 1) tb[3 * q + 1] = cnt_table(c, dg, kp[q].ch_ta);
       chh[q] = chain_table(c, dg, kp[q].ch_ta, kp[q].ch_tb);
     }

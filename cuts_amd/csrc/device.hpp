@@ -75,7 +75,9 @@ struct KPlan {
   // that |A| * |B| - |A & B| depends on every prefix vertex; 2: position k-2
   // joined to exactly pr_a and pr_b and k-1 to one of them (pr_c), thresholds
   // <= 2, so that every vertex of A & B is in k-1's list and the prefix has
-  // |A & B| * (|C| - 1) completions
+  // |A & B| * (|C| - 1) completions; 3: a chain (the ch_* fields) on position
+  // k-3, the intersections of whose list with every prefix vertex's differ
+  // from row to row
   uint32_t tl_kind;
   uint32_t pr_c;
   // last two positions as a chain (symmetric graphs): k-1's one backward

@@ -47,10 +47,9 @@
 
 #include "batch.hpp"
 
-// The library builds this file as four objects side by side, since the
-// chain level's unrolled closed form takes the compiler as long as all else
-// together: parts 1 to 3 hold that level's kernels, part 0 the rest and the
-// host code.  Without CUTS_MATCH_PART the file is one object.
+// The library builds this file as six objects side by side, since the
+// chain's unrolled closed form takes the compiler longer than all else
+// together: parts 1 to 5 hold its kernels, part 0 the rest and the host code.  Without CUTS_MATCH_PART the file is one object.
 #if !defined(CUTS_MATCH_PART) || CUTS_MATCH_PART == 0
 #define CUTS_MATCH_HOST 1
 #else
@@ -538,6 +537,74 @@ __device__ __forceinline__ void pair_bases(const GView& g, const KPlan& P, const
   }
 }
 
+// ------------------------------------------------------------ chain level
+struct ChainTables {
+  const uint64_t* H;           // 2V, k_chain_table
+  const uint32_t *ta, *tb;     // degree-threshold tables (null: plain degree)
+};
+
+// Completions of the last two positions as a chain for the prefix r[0..N)
+// of positions 0..k-3 (N = k-2), u = r[ch_u]:
+//   H(u) - sum_{r_i in N(u), deg >= ta} cnt_tb(r_i) - [deg u >= tb] |A|
+//        - sum_{i != ch_u, deg(r_i) >= tb} (|N(u) & N(r_i)| - c_i)
+// with |A| = cnt_ta(u) - |{i : r_i in N(u), deg(r_i) >= ta}| (returned in
+// na) and c_i the prefix vertices inside N(u) & N(r_i) meeting ta.  The
+// intersections of positions < N-1 come summed in `shared`; the one with
+// r[N-1] is looked up in the two-hop index when h2, else left out (a later
+// pass subtracts it).  Adds the demand bytes of its loads to bytes and, with
+// stats, to mb the merge-model bytes of expanding the prefix by u's list and
+// each of its |A| children by its own list.
+template <int N>
+__device__ __forceinline__ int64_t chain_closed(const GView& g, const KPlan& P, const uint32_t (&r)[N],
+                                                const ChainTables& t, uint32_t shared, bool h2, uint32_t dn,
+                                                int64_t& na, bool stats, uint64_t& mb, uint64_t& bytes) {
+  uint64_t& dummy = bytes;
+  bytes += 4 * N + 8 + 8 + (t.ta ? 4 : 0);  // degrees of the row, u's offsets, H(u), cnt_ta(u)
+  uint32_t u = 0, d[N];
+#pragma unroll
+  for (int l = 0; l < N; ++l) {
+    if (l == (int)P.ch_u) u = r[l];
+    d[l] = l == N - 1 && dn != ~0u ? dn : g.sig[2 * (uint64_t)r[l]];
+  }
+  // (loop-free symmetric graphs: the signature is the degree)
+  uint32_t du = d[0];
+#pragma unroll
+  for (int l = 1; l < N; ++l)
+    if (l == (int)P.ch_u) du = d[l];
+  // prefix vertices inside N(u) that meet ta
+  uint32_t inu = 0;
+#pragma unroll
+  for (int l = 0; l < N; ++l) {
+    const bool in = l != (int)P.ch_u && (((P.qadj[P.ch_u] >> l) & 1) || adj_has(g, u, r[l], dummy));
+    if (in && d[l] >= P.ch_ta) inu |= 1u << l;
+  }
+  na = (int64_t)(t.ta ? t.ta[u] : du) - __popc(inu);
+  int64_t c = (int64_t)t.H[u];
+  uint64_t dsum = 0;
+#pragma unroll
+  for (int l = 0; l < N; ++l)
+    if ((inu >> l) & 1) {
+      c -= t.tb ? t.tb[r[l]] : d[l];
+      dsum += d[l];
+      bytes += t.tb ? 4 : 8;
+    }
+  if (P.ch_tb <= 1 || du >= P.ch_tb) c -= na;
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    if (i == (int)P.ch_u || d[i] < P.ch_tb) continue;
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+      if (j == i || !((inu >> j) & 1)) continue;
+      // (in the list of the older vertex, which the lanes of a prefix share)
+      if (((P.qadj[i] >> j) & 1) || adj_has(g, i < j ? r[i] : r[j], i < j ? r[j] : r[i], dummy)) ++c;
+    }
+  }
+  c -= (int64_t)shared;
+  if (h2 && (P.ch_tb <= 1 || d[N - 1] >= P.ch_tb)) c -= index_common(g, u, r[N - 1], dummy);
+  if (stats) mb += 8 + 4ull * du + 24ull * (uint64_t)na + 4ull * (t.H[g.V + u] - dsum);
+  return c;
+}
+
 // Completions of the prefix r[0..N) of positions 0..k-3 (N = k-2) whose last
 // two positions are counted together (tl_kind); |A & B| without its
 // intersection N(u) & N(w) where pair_bases has no index for it.  na gets the
@@ -545,8 +612,20 @@ __device__ __forceinline__ void pair_bases(const GView& g, const KPlan& P, const
 // the prefix's and its children's expansions.
 template <int N>
 __device__ __forceinline__ uint64_t tail_count(const GView& g, const KPlan& P, const uint32_t (&r)[N],
-                                               const PairTables& pt, uint32_t dn, bool stats, uint64_t& na,
-                                               uint64_t& mb, uint64_t& bytes) {
+                                               const PairTables& pt, const ChainTables& ct, uint32_t dn, bool stats,
+                                               uint64_t& na, uint64_t& mb, uint64_t& bytes) {
+  if (P.tl_kind == 3) {
+    // the chain's intersections, all from an index
+    const uint32_t u = r[N - 1];
+    uint32_t shared = 0;
+#pragma unroll
+    for (int i = 0; i < N - 1; ++i)
+      if (P.ch_tb <= 1 || g.sig[2 * (uint64_t)r[i]] >= P.ch_tb) shared += index_common(g, r[i], u, bytes);
+    int64_t n = 0;
+    const int64_t c = chain_closed<N>(g, P, r, ct, shared, false, dn, n, stats, mb, bytes);
+    na += (uint64_t)n;
+    return (uint64_t)c;
+  }
   uint32_t u, w;
   int64_t ca, cb, cab;
   pair_bases<N>(g, P, r, pt, dn, u, w, ca, cb, cab, bytes);
@@ -1126,74 +1205,6 @@ static __global__ __launch_bounds__(BLOCK) void k_cnt_table(GView g, uint32_t th
   }
 }
 
-// ------------------------------------------------------------ chain level
-struct ChainTables {
-  const uint64_t* H;           // 2V, k_chain_table
-  const uint32_t *ta, *tb;     // degree-threshold tables (null: plain degree)
-};
-
-// Completions of the last two positions as a chain for the prefix r[0..N)
-// of positions 0..k-3 (N = k-2), u = r[ch_u]:
-//   H(u) - sum_{r_i in N(u), deg >= ta} cnt_tb(r_i) - [deg u >= tb] |A|
-//        - sum_{i != ch_u, deg(r_i) >= tb} (|N(u) & N(r_i)| - c_i)
-// with |A| = cnt_ta(u) - |{i : r_i in N(u), deg(r_i) >= ta}| (returned in
-// na) and c_i the prefix vertices inside N(u) & N(r_i) meeting ta.  The
-// intersections of positions < N-1 come summed in `shared`; the one with
-// r[N-1] is looked up in the two-hop index when h2, else left out (a later
-// pass subtracts it).  Adds the demand bytes of its loads to bytes and, with
-// stats, to mb the merge-model bytes of expanding the prefix by u's list and
-// each of its |A| children by its own list.
-template <int N>
-__device__ __forceinline__ int64_t chain_closed(const GView& g, const KPlan& P, const uint32_t (&r)[N],
-                                                const ChainTables& t, uint32_t shared, bool h2, uint32_t dn,
-                                                int64_t& na, bool stats, uint64_t& mb, uint64_t& bytes) {
-  uint64_t& dummy = bytes;
-  bytes += 4 * N + 8 + 8 + (t.ta ? 4 : 0);  // degrees of the row, u's offsets, H(u), cnt_ta(u)
-  uint32_t u = 0, d[N];
-#pragma unroll
-  for (int l = 0; l < N; ++l) {
-    if (l == (int)P.ch_u) u = r[l];
-    d[l] = l == N - 1 && dn != ~0u ? dn : g.sig[2 * (uint64_t)r[l]];
-  }
-  // (loop-free symmetric graphs: the signature is the degree)
-  uint32_t du = d[0];
-#pragma unroll
-  for (int l = 1; l < N; ++l)
-    if (l == (int)P.ch_u) du = d[l];
-  // prefix vertices inside N(u) that meet ta
-  uint32_t inu = 0;
-#pragma unroll
-  for (int l = 0; l < N; ++l) {
-    const bool in = l != (int)P.ch_u && (((P.qadj[P.ch_u] >> l) & 1) || adj_has(g, u, r[l], dummy));
-    if (in && d[l] >= P.ch_ta) inu |= 1u << l;
-  }
-  na = (int64_t)(t.ta ? t.ta[u] : du) - __popc(inu);
-  int64_t c = (int64_t)t.H[u];
-  uint64_t dsum = 0;
-#pragma unroll
-  for (int l = 0; l < N; ++l)
-    if ((inu >> l) & 1) {
-      c -= t.tb ? t.tb[r[l]] : d[l];
-      dsum += d[l];
-      bytes += t.tb ? 4 : 8;
-    }
-  if (P.ch_tb <= 1 || du >= P.ch_tb) c -= na;
-#pragma unroll
-  for (int i = 0; i < N; ++i) {
-    if (i == (int)P.ch_u || d[i] < P.ch_tb) continue;
-#pragma unroll
-    for (int j = 0; j < N; ++j) {
-      if (j == i || !((inu >> j) & 1)) continue;
-      // (in the list of the older vertex, which the lanes of a prefix share)
-      if (((P.qadj[i] >> j) & 1) || adj_has(g, i < j ? r[i] : r[j], i < j ? r[j] : r[i], dummy)) ++c;
-    }
-  }
-  c -= (int64_t)shared;
-  if (h2 && (P.ch_tb <= 1 || d[N - 1] >= P.ch_tb)) c -= index_common(g, u, r[N - 1], dummy);
-  if (stats) mb += 8 + 4ull * du + 24ull * (uint64_t)na + 4ull * (t.H[g.V + u] - dsum);
-  return c;
-}
-
 // Chain level over rows of L = k-3 words whose position-(k-3) candidates are
 // their parent's block of `cand` (built once per parent, constraints and
 // threshold checked): one work item per (row, candidate); a candidate equal
@@ -1387,7 +1398,7 @@ __global__ __launch_bounds__(BLOCK) void k_expand(GView g, KPlan P, ExpandArgs a
       r[L] = s_q[wave][1][i];
       ++valid;
       if constexpr (MODE == M_TAIL) {
-        acc += tail_count<L + 1>(g, P, r, a.ptab, dv, a.stats != 0, pairs, mb, bytes);
+        acc += tail_count<L + 1>(g, P, r, a.ptab, a.ctab, dv, a.stats != 0, pairs, mb, bytes);
       } else if constexpr (MODE == M_CHAIN) {
         int64_t na = 0;
         acc += (uint64_t)chain_closed<L + 1>(g, P, r, a.ctab, a.shared[p], true, dv, na, a.stats != 0, mb, bytes);
@@ -2121,8 +2132,8 @@ __global__ __launch_bounds__(BLOCK) void k_chain_prep(GView g, KPlan P, const ui
 // hub row, or left to k_common (minlen, minsel and desc set here).
 template <int L>
 __global__ __launch_bounds__(BLOCK) void k_tail_row(GView g, KPlan P, const uint32_t* __restrict__ rows, uint64_t n,
-                                                   PairTables pt, bool known, uint32_t* __restrict__ minlen,
-                                                   uint8_t* __restrict__ minsel, uint4* __restrict__ desc,
+                                                   PairTables pt, ChainTables ct, bool known,
+                                                   uint32_t* __restrict__ minlen, uint8_t* __restrict__ minsel, uint4* __restrict__ desc,
                                                    unsigned long long* __restrict__ counters, int stats) {
   uint64_t acc = 0, na = 0, mb = 0, bytes = 0;
   const bool hub = g.hr_id && P.pr_tab <= 2;
@@ -2131,7 +2142,7 @@ __global__ __launch_bounds__(BLOCK) void k_tail_row(GView g, KPlan P, const uint
 #pragma unroll
     for (int l = 0; l < L; ++l) r[l] = rows[p * L + l];
     bytes += 4 * L;
-    acc += tail_count<L>(g, P, r, pt, ~0u, stats != 0, na, mb, bytes);
+    acc += tail_count<L>(g, P, r, pt, ct, ~0u, stats != 0, na, mb, bytes);
     if (known) continue;
     const uint32_t u = rows[p * L + P.pr_a], w = rows[p * L + P.pr_b];
     const uint32_t hc = hub ? hub_common(g, u, w) : ~0u;
@@ -2151,6 +2162,57 @@ __global__ __launch_bounds__(BLOCK) void k_tail_row(GView g, KPlan P, const uint
   }
   add_sum(counters, 0, acc);
   add_sum(counters, 1, na);
+  if (stats) {
+    add_wave(&counters[8], mb);
+    add_wave(&counters[3], bytes);
+  }
+}
+
+// The chain on position k-3 over stored rows p0 .. p0+n-1 of level k-3 (L =
+// k-2 words) without an index for all of its intersections: the closed form
+// per row, less those that the per-arc table (positions adjacent in the
+// query) or a hub row holds; the others are left to k_common as entries (row,
+// position): minlen and desc at (p - p0) * (L - 1) + i.
+template <int L>
+__global__ __launch_bounds__(BLOCK) void k_chain_tail_row(GView g, KPlan P, const uint32_t* __restrict__ rows,
+                                                         uint64_t n, ChainTables t, uint32_t* __restrict__ minlen,
+                                                         uint4* __restrict__ desc,
+                                                         unsigned long long* __restrict__ counters, int stats) {
+  uint64_t acc = 0, na_sum = 0, mb = 0, bytes = 0;
+  const bool two = P.ch_ta <= 2;  // the indexes serve the threshold
+  for (uint64_t p = (uint64_t)blockIdx.x * BLOCK + threadIdx.x; p < n; p += (uint64_t)gridDim.x * BLOCK) {
+    uint32_t r[L];
+#pragma unroll
+    for (int l = 0; l < L; ++l) r[l] = rows[p * L + l];
+    const uint32_t u = r[L - 1];
+    const uint32_t ul = g.off_out[u], uh = g.off_out[u + 1];
+    uint32_t shared = 0;
+#pragma unroll
+    for (int i = 0; i < L - 1; ++i) {
+      uint32_t len = 0;
+      if (P.ch_tb <= 1 || g.sig[2 * (uint64_t)r[i]] >= P.ch_tb) {
+        const uint32_t hc = two ? hub_common(g, r[i], u) : ~0u;
+        if (hc != ~0u) {
+          shared += hc;
+        } else if (two && g.arc_cn && ((P.qadj[L - 1] >> i) & 1)) {
+          shared += index_common(g, r[i], u, bytes);
+        } else {
+          const uint32_t wl = g.off_out[r[i]], wh = g.off_out[r[i] + 1];
+          const bool sel = uh - ul > wh - wl;  // walk r_i's list, test in u's
+          len = min(uh - ul, wh - wl);
+          const int32_t h = g.hub_id ? g.hub_id[sel ? u : r[i]] : -1;
+          desc[p * (L - 1) + i] = make_uint4(sel ? wl : ul, h >= 0 ? (uint32_t)h : ~0u, sel ? ul : wl, sel ? uh : wh);
+        }
+      }
+      minlen[p * (L - 1) + i] = len;
+    }
+    int64_t na = 0;
+    acc += (uint64_t)chain_closed<L>(g, P, r, t, shared, false, ~0u, na, stats != 0, mb, bytes);
+    na_sum += (uint64_t)na;
+    bytes += 4 * L;
+  }
+  add_sum(counters, 0, acc);
+  add_sum(counters, 1, na_sum);
   if (stats) {
     add_wave(&counters[8], mb);
     add_wave(&counters[3], bytes);
@@ -2449,17 +2511,30 @@ __global__ __launch_bounds__(BLOCK) void k_chain_row(GView g, KPlan P, const uin
   CUTS_EXTERN template __global__ void k_chain_row<L>(GView, KPlan, const uint32_t*, uint64_t, const uint32_t*,      \
                                                       const uint32_t*, ChainTables, uint32_t*, uint8_t*,            \
                                                       unsigned long long*, int);
+#define CUTS_I_TAIL(L) CUTS_EXTERN template __global__ void k_expand<L, M_TAIL>(GView, KPlan, ExpandArgs);
+#define CUTS_I_TAIL_ROW(L)                                                                                           \
+  CUTS_EXTERN template __global__ void k_tail_row<L>(GView, KPlan, const uint32_t*, uint64_t, PairTables,            \
+                                                     ChainTables, bool, uint32_t*, uint8_t*, uint4*,                 \
+                                                     unsigned long long*, int);                                      \
+  CUTS_EXTERN template __global__ void k_chain_tail_row<L>(GView, KPlan, const uint32_t*, uint64_t, ChainTables,     \
+                                                           uint32_t*, uint4*, unsigned long long*, int);
 #if CUTS_MATCH_PART == 0
 #define CUTS_EXTERN extern
 CUTS_L13(CUTS_I_CHAIN)
 CUTS_L13(CUTS_I_SIB)
 CUTS_L13(CUTS_I_ROW) CUTS_I_ROW(14) CUTS_I_ROW(15)
+CUTS_L13(CUTS_I_TAIL)
+CUTS_L13(CUTS_I_TAIL_ROW) CUTS_I_TAIL_ROW(14) CUTS_I_TAIL_ROW(15)
 #else
 #define CUTS_EXTERN
 #if CUTS_MATCH_PART == 1
 CUTS_L13(CUTS_I_CHAIN)
 #elif CUTS_MATCH_PART == 2
 CUTS_L13(CUTS_I_SIB)
+#elif CUTS_MATCH_PART == 4
+CUTS_L13(CUTS_I_TAIL)
+#elif CUTS_MATCH_PART == 5
+CUTS_L13(CUTS_I_TAIL_ROW) CUTS_I_TAIL_ROW(14) CUTS_I_TAIL_ROW(15)
 #else
 CUTS_L13(CUTS_I_ROW) CUTS_I_ROW(14) CUTS_I_ROW(15)
 #endif
@@ -2638,7 +2713,14 @@ struct Matcher {
   bool pair_cab_known() const {
     return kp.pr_tab <= 2 && (g.h2_off || (g.arc_cn && kp.pr_adj));
   }
-  bool tail_known() const { return kp.pr_a == kp.pr_b || pair_cab_known(); }
+  // every intersection that the whole-prefix tail needs comes from an index
+  bool tail_known() const {
+    if (kp.tl_kind == 3) {
+      const uint32_t others = (1u << (k - 3)) - 1;
+      return others == 0 || (kp.ch_ta <= 2 && (g.h2_off || (g.arc_cn && (others & ~kp.qadj[k - 3]) == 0)));
+    }
+    return kp.pr_a == kp.pr_b || pair_cab_known();
+  }
   bool past_deadline() {
     if (has_deadline && !aborted && std::chrono::steady_clock::now() >= deadline) aborted = true;
     return aborted;
@@ -3156,10 +3238,31 @@ struct Matcher {
   // then the intersections that no index holds.
   void tail_rows(uint32_t L, const uint32_t* rows, uint64_t n, LevelBuf& in) {
     const bool known = tail_known();
+    if (kp.tl_kind == 3 && !known) {
+      // entries (row, position) in the buffers of level k-2, whose rows are
+      // never stored, as many rows at a time as give 4 M entries
+      LevelBuf& vb = lv[L];
+      const uint64_t per = L - 1;
+      const uint64_t step = std::max<uint64_t>(1, std::min<uint64_t>(n, std::min<uint64_t>(level_cap[L], 1ull << 22) / per));
+      ensure_rows_exact(arena, vb, step * per, L + 1);
+      ensure_aux(arena, vb.pbase, vb.pbase_cap, step * per);
+      for (uint64_t p0 = 0; p0 < n && !past_deadline(); p0 += step) {
+        const uint64_t m = std::min(step, n - p0);
+        pbegin(true);
+#define CT(LL) hipLaunchKernelGGL((k_chain_tail_row<LL>), dim3(grid_for(m, BLOCK, grid_cap)), dim3(BLOCK), 0, c.stream, g, kp, rows + p0 * L, m, ctab, vb.minlen, vb.pbase, ctr, (int)prof)
+        CUTS_DISPATCH_L(L, CT)
+#undef CT
+        HIPCHECK(hipGetLastError());
+        pend(7, 0, true);
+        common_pass(L, rows, m * per, vb, CommonArgs{0, 0, kp.ch_ta, 1u, vb.pbase}, nullptr, speculate());
+        if (aborted) return;
+      }
+      return;
+    }
     if (!known) ensure_aux(arena, in.pbase, in.pbase_cap, n);
     const uint32_t grid = grid_for(n, BLOCK, grid_cap);
     pbegin(true);
-#define TR(LL) hipLaunchKernelGGL((k_tail_row<LL>), dim3(grid), dim3(BLOCK), 0, c.stream, g, kp, rows, n, ptbl, known, in.minlen, in.minsel, in.pbase, ctr, (int)prof)
+#define TR(LL) hipLaunchKernelGGL((k_tail_row<LL>), dim3(grid), dim3(BLOCK), 0, c.stream, g, kp, rows, n, ptbl, ctab, known, in.minlen, in.minsel, in.pbase, ctr, (int)prof)
     CUTS_DISPATCH_L(L, TR)
 #undef TR
     HIPCHECK(hipGetLastError());
@@ -3445,9 +3548,11 @@ struct Matcher {
     pair = fuse && kp.pr_ok && !(o.flags & 128u);
     chain = fuse && !pair && kp.ch_ok && !(o.flags & 256u);
     // the last two positions from whole prefixes: inside the expansion of
-    // position k-3 where an index holds the intersection, else over stored
-    // rows (a pair only: its intersections can be subtracted afterwards)
-    tail = fuse && !pair && !chain && !(o.flags & 128u) && (kp.tl_kind == 1 || (kp.tl_kind == 2 && tail_known()));
+    // position k-3 where an index holds the intersections, else over stored
+    // rows (a pair or a chain: their intersections are subtracted afterwards)
+    tail = fuse && !pair && !chain &&
+           (kp.tl_kind == 3 ? !(o.flags & 256u)
+                            : !(o.flags & 128u) && (kp.tl_kind == 1 || (kp.tl_kind == 2 && tail_known())));
     tail_fused = tail && tail_known() && k >= 4;
     // 6 blocks of 4 waves per CU: measured best on the power-law workloads
     // (the tiles are taken dynamically, so the grid only sets residency)
@@ -3483,12 +3588,12 @@ struct Matcher {
     collapse_fused = pair && kp.pr_collapse && pair_cab_known() && k >= 5 && !(o.time_limit_ms > 0);
     // the fused chain with position k-3's candidates shared by siblings
     sib = chain_fused && kp.ch_sib && !(o.flags & 1024u);
-    if (chain) {
+    if (chain || (tail && kp.tl_kind == 3)) {
       ctab.ta = kp.ch_ta > 1 ? cnt_table(c, dg, arena, kp.ch_ta) : nullptr;
       ctab.tb = kp.ch_tb > 1 ? cnt_table(c, dg, arena, kp.ch_tb) : nullptr;
       ctab.H = chain_table(c, dg, arena, kp.ch_ta, kp.ch_tb);
     }
-    if (pair || tail) {
+    if (pair || (tail && kp.tl_kind != 3)) {
       ptbl.a = kp.pr_ta > 1 ? cnt_table(c, dg, arena, kp.pr_ta) : nullptr;
       ptbl.b = kp.pr_tb > 1 ? cnt_table(c, dg, arena, kp.pr_tb) : nullptr;
       ptbl.ab = kp.pr_a == kp.pr_b && kp.pr_tab > 1 ? cnt_table(c, dg, arena, kp.pr_tab) : nullptr;
@@ -3809,14 +3914,15 @@ KPlan make_kplan(const Plan& p, bool symmetric, bool loop_free) {
     for (uint32_t j = 0; j < p.k; ++j)
       if (i != j && ((p.pmask[std::max(i, j)] | p.cmask[std::max(i, j)]) >> std::min(i, j) & 1)) kp.qadj[i] |= 1u << j;
   // the last two positions as a chain: k-1 hangs on k-2 only, k-2 on one
-  // position older than k-3 only
-  if (kp.sc_ok && loop_free && p.k >= 4 && kp.sc_pos == last - 1 && kp.nj[last - 1] == 1) {
+  // position u: older than k-3 only, or k-3 itself (counted per row)
+  if (kp.sc_ok && loop_free && p.k >= 3 && kp.sc_pos == last - 1 && kp.nj[last - 1] == 1) {
     const uint32_t u = kp.jc[last - 1][0] & 31;
-    if (u + 3 < p.k) {
-      kp.ch_ok = 1;
-      kp.ch_u = u;
-      kp.ch_ta = std::max(p.sig_in[last - 1], p.sig_out[last - 1]);
-      kp.ch_tb = kp.sc_thr;
+    kp.ch_ok = u + 3 < p.k;
+    if (!kp.ch_ok) kp.tl_kind = 3;
+    kp.ch_u = u;
+    kp.ch_ta = std::max(p.sig_in[last - 1], p.sig_out[last - 1]);
+    kp.ch_tb = kp.sc_thr;
+    if (kp.ch_ok) {
       // position k-3's constraints all older than k-4 (and at least one)
       const uint32_t c = last - 2;
       bool sib = p.k >= 5 && kp.nj[c] >= 1;

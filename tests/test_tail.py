@@ -3,7 +3,8 @@
 A pair of leaves of which one hangs on position k-3 itself has
 |A| * |B| - |A & B| completions per row of level k-3; a position k-2 joined
 to two older positions followed by a leaf on one of them has
-|A & B| * (|C| - 1).  Where an index holds |N(u) & N(w)| the expansion of
+|A & B| * (|C| - 1); a 2-edge tail on position k-3 takes the chain's closed
+form with an intersection per prefix vertex.  Where an index holds |N(u) & N(w)| the expansion of
 position k-3 counts them, else stored rows do and the intersections are
 walked.  Counts equal the oracle's, level sizes and merge-model bytes the CPU
 trie walk's, in every mode that changes the route.
@@ -26,10 +27,16 @@ CASES = {
                                   [0, 2, 1, 3, 4, 5, 6]),
     "diamond, leaf": ([(0, 1), (0, 2), (1, 2), (1, 3), (2, 3), (1, 4)], [0, 1, 2, 3, 4]),
     "triangle, leaf": ([(0, 1), (1, 2), (2, 0), (0, 3)], [0, 1, 2, 3]),
+    "path3 from its end": ([(0, 1), (1, 2)], [0, 1, 2]),
+    "path4 from its end": ([(0, 1), (1, 2), (2, 3)], [0, 1, 2, 3]),
+    "triangle, tail of two on the newest": ([(0, 1), (1, 2), (2, 0), (2, 3), (3, 4)], [0, 1, 2, 3, 4]),
+    "4-cycle, tail of two": ([(0, 1), (1, 2), (2, 3), (3, 0), (3, 4), (4, 5)], [0, 1, 2, 3, 4, 5]),
+    "5-cycle, chord, tail of two": ([(0, 1), (1, 2), (2, 3), (3, 4), (4, 0), (0, 2), (4, 5), (5, 6)],
+                                    [0, 1, 2, 3, 4, 5, 6]),
     "4-cycle, leaf": ([(0, 1), (1, 2), (2, 3), (3, 0), (0, 4)], [0, 1, 2, 3, 4]),
 }
 FLAGS = [0, F.FLAG_NO_BITMAP, F.FLAG_NO_TWO_HOP, F.FLAG_NO_TWO_HOP | F.FLAG_NO_BITMAP,
-         F.FLAG_NO_TWO_HOP | F.FLAG_NO_ARC_COMMON, F.FLAG_NO_PAIR]
+         F.FLAG_NO_TWO_HOP | F.FLAG_NO_ARC_COMMON, F.FLAG_NO_PAIR, F.FLAG_NO_CHAIN]
 
 
 def tail_kind(k, edges, order):
@@ -38,7 +45,9 @@ def tail_kind(k, edges, order):
     for a, b in edges:
         i, j = at[a], at[b]
         back[max(i, j)].add(min(i, j))
-    if len(back[k - 1]) != 1 or k - 2 in back[k - 1]:
+    if back[k - 1] == {k - 2}:
+        return 3 if back[k - 2] == {k - 3} else 0
+    if len(back[k - 1]) != 1:
         return 0
     (c,) = back[k - 1]
     if len(back[k - 2]) == 1:
@@ -46,9 +55,9 @@ def tail_kind(k, edges, order):
     return 2 if len(back[k - 2]) == 2 and c in back[k - 2] else 0
 
 
-def test_cases_cover_both_kinds():
+def test_cases_cover_every_kind():
     kinds = [tail_kind(len(o), e, o) for e, o in CASES.values()]
-    assert 0 not in kinds and kinds.count(1) >= 6 and kinds.count(2) >= 2
+    assert 0 not in kinds and kinds.count(1) >= 6 and kinds.count(2) >= 2 and kinds.count(3) >= 5
 
 
 @pytest.mark.gpu
@@ -124,7 +133,7 @@ def test_batch_counts_them_too(ctx, queue):
     single = [ctx.match(dg, p) for p in plans]
     assert [r.count for r in single] == want
     for kw in (dict(), dict(item_work=1), dict(item_work=50, vchunk=9), dict(item_work=1 << 20)):
-        for flags in (0, F.FLAG_NO_TWO_HOP, F.FLAG_NO_PAIR, F.FLAG_NO_BITMAP):
+        for flags in (0, F.FLAG_NO_TWO_HOP, F.FLAG_NO_PAIR, F.FLAG_NO_CHAIN, F.FLAG_NO_BITMAP):
             b = F.Batch(ctx, dg, plans, queue=queue, flags=flags, arena_bytes=1 << 28, **kw)
             for _ in range(2):
                 r = b.run()
