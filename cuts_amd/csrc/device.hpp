@@ -47,6 +47,10 @@ struct KPlan {
   uint32_t sig_in[kMaxQuery], sig_out[kMaxQuery];
   uint32_t nj[kMaxQuery];
   uint8_t jc[kMaxQuery][2 * kMaxQuery];
+  // bit i: position i's thresholds follow from its constraints (as many
+  // distinct in- and out-neighbours as they ask for), so that a candidate in
+  // every list needs no signature test
+  uint32_t sig_implied;
   // last position counted as |N(row[sc_pos])| minus prefix members
   uint32_t sc_ok;      // 1 if the closed form applies
   uint32_t sc_pos;     // position whose list is counted
@@ -127,6 +131,10 @@ struct DeviceGraph {
   int32_t* hub_id = nullptr;
   uint64_t* bits = nullptr;
   uint32_t words = 0, hubs = 0, hub_min_deg = 0;
+  // directed graphs: the same for out-lists (hub_dir[0], bits_dir[0]) and
+  // in-lists ([1]); hub_id and bits, which the closed forms read, stay null
+  int32_t* hub_dir[2] = {nullptr, nullptr};
+  uint64_t* bits_dir[2] = {nullptr, nullptr};
   // two-hop index (symmetric graphs whose wedges fit the budget): per vertex
   // u, the vertices v != u with a common neighbour, ascending (h2_v over
   // h2_off[u] .. h2_off[u+1]), and |N(u) & N(v)| for each (h2_c)

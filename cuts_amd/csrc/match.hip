@@ -128,6 +128,10 @@ struct GView {
   const uint32_t *off_out, *adj_out, *off_in, *adj_in, *sig;
   uint32_t V;
   const int32_t* hub_id;  // null when the graph has no hub bitmaps
+  // hub rows of out-lists [0] and in-lists [1] (symmetric graphs: hub_id and
+  // bits twice), or null
+  const int32_t* hub_dir[2];
+  const uint64_t* bits_dir[2];
   const uint2 *nsig_out, *nsig_in;  // signature of every list entry
   const uint64_t* bits;
   uint32_t words;
@@ -141,7 +145,11 @@ struct GView {
 };
 
 inline GView view_of(const DeviceGraph& dg) {
-  return GView{dg.off_out, dg.adj_out, dg.off_in, dg.adj_in, dg.sig, dg.V, dg.hub_id, dg.nsig_out, dg.nsig_in, dg.bits,
+  const bool sym = dg.symmetric;
+  return GView{dg.off_out, dg.adj_out, dg.off_in, dg.adj_in, dg.sig, dg.V, dg.hub_id,
+               {sym ? dg.hub_id : dg.hub_dir[0], sym ? dg.hub_id : dg.hub_dir[1]},
+               {sym ? dg.bits : dg.bits_dir[0], sym ? dg.bits : dg.bits_dir[1]},
+               dg.nsig_out, dg.nsig_in, dg.bits,
                dg.words, dg.h2_off, dg.h2_v, dg.h2_c, dg.h2_did, dg.h2_dense, dg.arc_cn, dg.hr_id, dg.hr};
 }
 
@@ -1375,6 +1383,9 @@ __global__ __launch_bounds__(BLOCK) void k_expand(GView g, KPlan P, ExpandArgs a
   if (blockIdx.x >= ntiles_) return;
   const uint32_t nj = P.nj[L];
   const uint32_t tin = P.sig_in[L], tout = P.sig_out[L];
+  // a last level that is counted entry by entry reads no signatures where its
+  // constraints imply them (always, short of query self-loops)
+  const bool need_sig = MODE != M_COUNT || !((P.sig_implied >> L) & 1);
   uint64_t acc = 0, valid = 0, pairs = 0, trips = 0, bytes = 0, mb = 0;
   // modes whose survivors wait in a queue of their wave: prefix, vertex,
   // degree (at most 63 left over and 64 new)
@@ -1477,7 +1488,7 @@ __global__ __launch_bounds__(BLOCK) void k_expand(GView g, KPlan P, ExpandArgs a
           cb[j] = (MODE == M_FUSED && a.cbase) ? a.cbase[p] : 0u;
           pb[j] = MODE == M_PAIR ? a.pbase[p] : make_uint4(0u, 0u, 0u, 0u);
           if (a.stats) {
-            bytes += 12;
+            bytes += need_sig ? 12 : 4;
             if (in[j] && idx[j] == 0) bytes += 4 * L + 9 + 8 * nj;
           }
         }
@@ -1495,7 +1506,7 @@ __global__ __launch_bounds__(BLOCK) void k_expand(GView g, KPlan P, ExpandArgs a
 #pragma unroll
             for (int l = 0; l < L; ++l)
               if (l == (int)(jcc & 31)) uu = row[j][l];
-            hpre[cc][j] = (g.hub_id && cc < (int)nj) ? g.hub_id[uu] : -1;
+            hpre[cc][j] = (g.hub_dir[0] && cc < (int)nj) ? g.hub_dir[jcc >> 7][uu] : -1;
           }
         }
 #pragma unroll
@@ -1511,7 +1522,8 @@ __global__ __launch_bounds__(BLOCK) void k_expand(GView g, KPlan P, ExpandArgs a
         for (int j = 0; j < G; ++j) v[j] = in[j] ? ((jc[j] >> 7) ? g.adj_in : g.adj_out)[lb[j] + idx[j]] : 0u;
         uint2 sg[G];
 #pragma unroll
-        for (int j = 0; j < G; ++j) sg[j] = in[j] ? ((jc[j] >> 7) ? g.nsig_in : g.nsig_out)[lb[j] + idx[j]] : make_uint2(0u, 0u);
+        for (int j = 0; j < G; ++j)
+          sg[j] = (in[j] && need_sig) ? ((jc[j] >> 7) ? g.nsig_in : g.nsig_out)[lb[j] + idx[j]] : make_uint2(~0u, ~0u);
 #pragma unroll
         for (int j = 0; j < G; ++j) {
           ok[j] = in[j] && sg[j].x >= tin && sg[j].y >= tout;
@@ -1529,11 +1541,13 @@ __global__ __launch_bounds__(BLOCK) void k_expand(GView g, KPlan P, ExpandArgs a
               if (l == (int)(jc2 & 31)) u2[j] = row[j][l];
           }
           // bit tests for hub lists; the other items' lower-bound searches
-          // in lock-step (symmetric graphs with hubs: every constraint is an
-          // out-list)
-          const bool hubs = g.hub_id != nullptr;
-          const uint32_t* off2 = (!hubs && (jc2 >> 7)) ? g.off_in : g.off_out;
-          const uint32_t* adj2 = (!hubs && (jc2 >> 7)) ? g.adj_in : g.adj_out;
+          // in lock-step
+          const uint32_t dir = jc2 >> 7;
+          const int32_t* hid = g.hub_dir[dir];
+          const uint64_t* hbits = g.bits_dir[dir];
+          const bool hubs = hid != nullptr;
+          const uint32_t* off2 = dir ? g.off_in : g.off_out;
+          const uint32_t* adj2 = dir ? g.adj_in : g.adj_out;
           bool srch[G];
           if (hubs) {
             int32_t h[G];
@@ -1544,11 +1558,11 @@ __global__ __launch_bounds__(BLOCK) void k_expand(GView g, KPlan P, ExpandArgs a
 #pragma unroll
               for (int cc = 0; cc < NJP; ++cc)
                 if ((int)c == cc) hh = hpre[cc][j];
-              h[j] = c < (uint32_t)NJP ? hh : g.hub_id[u2[j]];
+              h[j] = c < (uint32_t)NJP ? hh : hid[u2[j]];
             }
 #pragma unroll
             for (int j = 0; j < G; ++j)
-              bw[j] = g.bits[h[j] >= 0 ? (uint64_t)h[j] * g.words + (v[j] >> 6) : 0];
+              bw[j] = hbits[h[j] >= 0 ? (uint64_t)h[j] * g.words + (v[j] >> 6) : 0];
 #pragma unroll
             for (int j = 0; j < G; ++j) {
               srch[j] = false;
@@ -2592,12 +2606,24 @@ uint32_t grid_for(uint64_t work, uint64_t per_block, uint32_t cap) {
   return (uint32_t)std::min<uint64_t>(b, cap);
 }
 
+// Back to the pool, once the device has finished with it (as hipFree waits).
+void dev_free(void* p) {
+  if (!p) return;
+  int device = 0;
+  (void)hipGetDevice(&device);
+  (void)hipDeviceSynchronize();
+  pool_give(device, p);
+}
+
+// An array on the current device, from the pool; the old one goes back.
 template <typename T>
 void dev_alloc(T*& p, uint64_t n) {
-  if (p) HIPCHECK(hipFree(p));
+  dev_free(p);
   p = nullptr;
-  if (device_malloc((void**)&p, std::max<uint64_t>(n, 1) * sizeof(T)) != hipSuccess)
-    throw Error(-5, "device allocation of " + std::to_string(n * sizeof(T)) + " bytes failed");
+  int device = 0;
+  HIPCHECK(hipGetDevice(&device));
+  p = (T*)pool_take(device, std::max<uint64_t>(n, 1) * sizeof(T));
+  if (!p) throw Error(-5, "device allocation of " + std::to_string(n * sizeof(T)) + " bytes failed");
 }
 
 // An array of the device graph's own, from the pool.
@@ -3534,7 +3560,7 @@ struct Matcher {
     if (k == 0 || k > kMaxQuery) throw Error(-3, "query must have between 1 and 16 vertices");
     kp = make_kplan(plan, dg.symmetric, dg.loops == 0);
     g = view_of(dg);
-    if (o.flags & 32u) g.hub_id = nullptr;  // CUTS_FLAG_NO_BITMAP
+    if (o.flags & 32u) g.hub_id = g.hub_dir[0] = g.hub_dir[1] = nullptr;  // CUTS_FLAG_NO_BITMAP
     if (o.flags & 512u) g.h2_off = nullptr;  // CUTS_FLAG_NO_TWO_HOP
     if (o.flags & 512u) g.h2_did = nullptr;
     if (o.flags & 512u) g.hr_id = nullptr;
@@ -3835,8 +3861,8 @@ double copy_probe(Context& c, uint64_t bytes, uint32_t iters) {
   HIPCHECK(hipEventSynchronize(c.kev[1]));
   float ms = 0;
   HIPCHECK(hipEventElapsedTime(&ms, c.kev[0], c.kev[1]));
-  (void)hipFree(a);
-  (void)hipFree(b);
+  dev_free(a);
+  dev_free(b);
   return (double)iters * 2.0 * (double)n * 16.0 / (ms / 1e3) / 1e9;
 }
 
@@ -3859,6 +3885,9 @@ KPlan make_kplan(const Plan& p, bool symmetric, bool loop_free) {
         if (p.cmask[i] >> j & 1) kp.jc[i][n++] = (uint8_t)(j | 0x80);
     }
     kp.nj[i] = n;
+    const uint32_t par = (uint32_t)__builtin_popcount(p.pmask[i]), chi = (uint32_t)__builtin_popcount(p.cmask[i]);
+    if (symmetric ? std::max(p.sig_in[i], p.sig_out[i]) <= n : p.sig_in[i] <= par && p.sig_out[i] <= chi)
+      kp.sig_implied |= 1u << i;
   }
   const uint32_t last = p.k - 1;
   if (symmetric && p.k >= 2 && kp.nj[last] == 1) {
@@ -3944,21 +3973,23 @@ DeviceGraph::~DeviceGraph() {
     nsig_in = nullptr;
   }
   for (void* p : {(void*)off_out, (void*)adj_out, (void*)sig, (void*)nsig_out, (void*)off_in, (void*)adj_in,
-                  (void*)nsig_in, (void*)hub_id, (void*)bits, (void*)arc_cn, (void*)h2_off, (void*)h2_v, (void*)h2_c,
+                  (void*)nsig_in, (void*)hub_id, (void*)bits, (void*)hub_dir[0], (void*)hub_dir[1],
+                  (void*)bits_dir[0], (void*)bits_dir[1], (void*)arc_cn, (void*)h2_off, (void*)h2_v, (void*)h2_c,
                   (void*)h2_did, (void*)h2_dense, (void*)hr_id, (void*)hr})
     pool_give(device, p);
-  for (auto& kv : cnt_tables) (void)hipFree(kv.second);
-  for (auto& kv : chain_tables) (void)hipFree(kv.second);
+  for (auto& kv : cnt_tables) pool_give(device, kv.second);
+  for (auto& kv : chain_tables) pool_give(device, kv.second);
   (void)hipSetDevice(prev);
 }
 
 Context::~Context() {
   (void)hipSetDevice(device);
+  (void)hipDeviceSynchronize();  // the level buffers' next owner may use them on any stream
   for (auto& b : lv) {
     for (void* p : {(void*)b.rows, (void*)b.rows2, (void*)b.minlen, (void*)b.minsel, (void*)b.work_off, (void*)b.bsum,
                     (void*)b.tile_p, (void*)b.cbase, (void*)b.pbase,
                     (void*)b.nsurv, (void*)b.parent, (void*)b.coff, (void*)b.cand})
-      if (p) (void)hipFree(p);
+      pool_give(device, p);
   }
   if (counters) (void)hipFree(counters);
   if (host_pinned) (void)hipHostFree(host_pinned);
@@ -4043,53 +4074,78 @@ void upload_graph(Context& c, const Graph& g, DeviceGraph& dg) {
   HIPCHECK(hipGetLastError());
   HIPCHECK(hipMemcpyAsync(stats, d_stats, sizeof(stats), hipMemcpyDeviceToHost, c.stream));
   HIPCHECK(hipStreamSynchronize(c.stream));
-  (void)hipFree(d_stats);
+  dev_free(d_stats);
   dg.max_deg = (uint32_t)stats[0];
   dg.loops = stats[1];
   const uint64_t wedges = stats[2];
   // Hub bitmaps: the lowest power-of-two degree threshold (>= 32) whose
-  // bitmaps fit the budget (1/32 of free HBM, at most 4 GiB).
-  if (g.symmetric && g.V >= 64) {
+  // bitmaps fit the budget (1/32 of free HBM, at most 4 GiB); a directed
+  // graph's out-lists and in-lists have half of it each.
+  if (g.V >= 64) {
     const uint64_t fr = device_free_bytes(c.device);
     uint64_t cap = std::min<uint64_t>(fr / 32, 4ull << 30);
     // CUTS_HUB_BITMAP_MB replaces the cap (at most half of free HBM)
     if (const char* e = std::getenv("CUTS_HUB_BITMAP_MB"))
       cap = std::min<uint64_t>((uint64_t)std::strtoull(e, nullptr, 10) << 20, fr / 2);
     const uint32_t words = (g.V + 63) / 64;
-    std::vector<uint32_t> deg(g.V);
-    for (uint32_t v = 0; v < g.V; ++v) deg[v] = g.out_off[v + 1] - g.out_off[v];
-    uint32_t t = 32;
+    uint32_t tmin = 32;
     // CUTS_HUB_MIN_DEG raises the starting threshold (fewer, larger hubs:
     // a bitmap set small enough to stay in L2)
-    if (const char* e = std::getenv("CUTS_HUB_MIN_DEG")) t = std::max<uint32_t>(t, (uint32_t)std::strtoul(e, nullptr, 10));
-    for (; t <= (1u << 30); t *= 2) {
-      uint64_t nh = 0;
-      for (uint32_t d : deg) nh += d >= t;
-      if (nh * words * 8 <= cap) break;
-    }
-    std::vector<uint32_t> hubs;
-    std::vector<int32_t> hid(g.V, -1);
-    for (uint32_t v = 0; v < g.V; ++v)
-      if (deg[v] >= t) {
-        hid[v] = (int32_t)hubs.size();
-        hubs.push_back(v);
+    if (const char* e = std::getenv("CUTS_HUB_MIN_DEG"))
+      tmin = std::max<uint32_t>(tmin, (uint32_t)std::strtoul(e, nullptr, 10));
+    // the rows of one side's lists; returns their number, t the threshold
+    auto build = [&](const std::vector<uint32_t>& off, const uint32_t* d_off, const uint32_t* d_adj, uint64_t most,
+                     int32_t*& hub_id, uint64_t*& bits, uint32_t& t) {
+      std::vector<uint32_t> deg(g.V);
+      for (uint32_t v = 0; v < g.V; ++v) deg[v] = off[v + 1] - off[v];
+      for (t = tmin; t <= (1u << 30); t *= 2) {
+        uint64_t nh = 0;
+        for (uint32_t d : deg) nh += d >= t;
+        if (nh * words * 8 <= most) break;
       }
-    if (!hubs.empty()) {
-      dg.words = words;
-      dg.hubs = (uint32_t)hubs.size();
-      dg.hub_min_deg = t;
-      graph_alloc(dg, dg.hub_id, g.V);
-      HIPCHECK(hipMemcpy(dg.hub_id, hid.data(), g.V * 4, hipMemcpyHostToDevice));
-      graph_alloc(dg, dg.bits, (uint64_t)hubs.size() * words);
-      HIPCHECK(hipMemset(dg.bits, 0, (uint64_t)hubs.size() * words * 8));
+      std::vector<uint32_t> hubs;
+      std::vector<int32_t> hid(g.V, -1);
+      for (uint32_t v = 0; v < g.V; ++v)
+        if (deg[v] >= t) {
+          hid[v] = (int32_t)hubs.size();
+          hubs.push_back(v);
+        }
+      if (hubs.empty()) return (uint32_t)0;
+      graph_alloc(dg, hub_id, g.V);
+      HIPCHECK(hipMemcpy(hub_id, hid.data(), g.V * 4, hipMemcpyHostToDevice));
+      graph_alloc(dg, bits, (uint64_t)hubs.size() * words);
+      HIPCHECK(hipMemset(bits, 0, (uint64_t)hubs.size() * words * 8));
       uint32_t* dh = nullptr;
       dev_alloc(dh, hubs.size());
       HIPCHECK(hipMemcpy(dh, hubs.data(), hubs.size() * 4, hipMemcpyHostToDevice));
       hipLaunchKernelGGL(k_hub_bits, dim3((uint32_t)std::min<size_t>(hubs.size(), 65535)), dim3(256), 0, c.stream,
-                         dg.off_out, dg.adj_out, dh, (uint32_t)hubs.size(), words, dg.bits);
+                         d_off, d_adj, dh, (uint32_t)hubs.size(), words, bits);
       HIPCHECK(hipGetLastError());
       HIPCHECK(hipStreamSynchronize(c.stream));
-      (void)hipFree(dh);
+      dev_free(dh);
+      return (uint32_t)hubs.size();
+    };
+    uint32_t t = 0;
+    if (g.symmetric) {
+      dg.hubs = build(g.out_off, dg.off_out, dg.adj_out, cap, dg.hub_id, dg.bits, t);
+      if (dg.hubs) {
+        dg.words = words;
+        dg.hub_min_deg = t;
+      }
+    } else {
+      const uint32_t o = build(g.out_off, dg.off_out, dg.adj_out, cap / 2, dg.hub_dir[0], dg.bits_dir[0], t);
+      const uint32_t i = build(g.in_off, dg.off_in, dg.adj_in, cap / 2, dg.hub_dir[1], dg.bits_dir[1], t);
+      dg.words = words;
+      // the kernels ask for both sides or neither: a side without hubs has a
+      // table of none (and no row that could be read)
+      for (int d = 0; d < 2; ++d)
+        if ((o || i) && !(d ? i : o)) {
+          const std::vector<int32_t> none(g.V, -1);
+          graph_alloc(dg, dg.hub_dir[d], g.V);
+          HIPCHECK(hipMemcpy(dg.hub_dir[d], none.data(), (uint64_t)g.V * 4, hipMemcpyHostToDevice));
+          graph_alloc(dg, dg.bits_dir[d], 1);
+          HIPCHECK(hipMemset(dg.bits_dir[d], 0, 8));
+        }
     }
   }
   // Per-arc common-neighbour counts (symmetric loop-free graphs): 4 bytes

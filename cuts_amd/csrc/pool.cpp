@@ -1,4 +1,4 @@
-// Device memory of graphs and index builds, kept between uploads.  A graph's
+// Device memory of graphs, index builds and trie levels, kept between uses.  A graph's
 // index takes gigabytes, and the driver clears what one upload frees before
 // the next may have it, at about 35 GB/s once the card's free memory has been
 // handed out once: uploads of a few milliseconds of kernels then waited 40 to
@@ -71,7 +71,7 @@ void* pool_take(int device, uint64_t bytes) {
     if (it != p.kept.end() && it->first <= bytes + bytes / 4) {
       void* b = it->second;
       p.held -= it->first;
-      p.handed.emplace(b, it->first);
+      p.handed[b] = it->first;
       p.kept.erase(it);
       return b;
     }
@@ -80,7 +80,7 @@ void* pool_take(int device, uint64_t bytes) {
   if (device_malloc(&b, bytes) != hipSuccess) return nullptr;
   if (bytes >= kKeepMin) {
     std::lock_guard<std::mutex> lk(p.mu);
-    p.handed.emplace(b, bytes);
+    p.handed[b] = bytes;
   }
   return b;
 }
