@@ -1367,9 +1367,29 @@ __device__ __forceinline__ uint64_t next_tile(unsigned int* tilectr, uint64_t nt
   return ~0ull;
 }
 
+// Four waves per SIMD for rows of up to 5 words (128 registers): at three the
+// R-MAT 20 tail expansion took 6.0 ms for 5.0.
 template <int L, int MODE>
-__global__ __launch_bounds__(BLOCK) void k_expand(GView g, KPlan P, ExpandArgs a) {
-  __shared__ uint64_t s_off[LDS_OFF + 1];
+__global__ __launch_bounds__(BLOCK, L <= 5 ? 4 : 1) void k_expand(GView g, KPlan P, ExpandArgs a) {
+  // A tile of at most SP prefixes stages them in LDS, one thread per prefix:
+  // where its items start in the tile, its row, the list position of its
+  // items (less their index in the tile), its list's constraint and the hub
+  // rows of the first NJP constraints.  An item then takes its prefix from
+  // LDS by 32-bit searches and reads instead of repeating the prefix's loads
+  // and address arithmetic, which bound the kernel by instruction issue
+  // (a directed last level of 1.3e10 items: 111 -> 79.6 ms).  Tiles
+  // of more prefixes (short lists) keep the offsets alone, or nothing.
+  constexpr uint32_t SP = 256, NJP = 3;
+  constexpr uint32_t STAGE_WORDS = (SP + 1) + (L + 3 + NJP) * SP;
+  constexpr uint32_t RAW_WORDS = STAGE_WORDS > 2 * (LDS_OFF + 1) ? STAGE_WORDS : 2 * (LDS_OFF + 1);
+  __shared__ __align__(8) uint32_t s_raw[RAW_WORDS];
+  uint64_t* const s_off = (uint64_t*)s_raw;
+  uint32_t* const s_rel = s_raw;                 // SP + 1
+  uint32_t* const s_row = s_rel + SP + 1;        // L x SP
+  uint32_t* const s_li = s_row + L * SP;         // SP
+  uint32_t* const s_meta = s_li + SP;            // SP: constraint index | jc << 8
+  uint32_t* const s_cb = s_meta + SP;            // SP
+  int32_t* const s_hub = (int32_t*)(s_cb + SP);  // NJP x SP
   __shared__ uint32_t s_w[BLOCK / 64], s_pre[BLOCK / 64], s_base;
   const uint32_t tid = threadIdx.x, wave = tid >> 6;
   // threads per block: BLOCK for the writing expansion; 64, 128 or 256 for
@@ -1438,8 +1458,38 @@ __global__ __launch_bounds__(BLOCK) void k_expand(GView g, KPlan P, ExpandArgs a
     const uint32_t plo = a.tile_p[tile], phi = a.tile_p[tile + 1];
     const uint32_t span = phi - plo + 1;  // offsets plo .. phi+1
     const bool lds = span <= LDS_OFF;
-    if (lds)
+    const bool staged = span <= SP && !a.stats;
+    if (staged) {
+      for (uint32_t i = tid; i < span; i += NT) {
+        const uint64_t p = (uint64_t)plo + i;
+        const uint64_t o = a.work_off[p];
+        const uint32_t sl = a.minsel[p], jcv = P.jc[L][sl];
+        uint32_t r[L], u = 0;
+#pragma unroll
+        for (int l = 0; l < L; ++l) r[l] = a.rows[p * L + l];
+#pragma unroll
+        for (int l = 0; l < L; ++l) {
+          s_row[l * SP + i] = r[l];
+          if (l == (int)(jcv & 31)) u = r[l];
+        }
+        s_rel[i] = o <= w0 ? 0u : (uint32_t)(o - w0);  // below TILE but for empty prefixes at the end
+        s_li[i] = ((jcv >> 7) ? g.off_in : g.off_out)[u] - (uint32_t)(o - w0);
+        s_meta[i] = sl | jcv << 8;
+        if (MODE == M_FUSED) s_cb[i] = a.cbase ? a.cbase[p] : 0u;
+#pragma unroll
+        for (int cc = 0; cc < (int)NJP; ++cc) {
+          const uint32_t jcc = cc < (int)nj ? P.jc[L][cc] : 0u;
+          uint32_t uu = 0;
+#pragma unroll
+          for (int l = 0; l < L; ++l)
+            if (l == (int)(jcc & 31)) uu = r[l];
+          if (cc < (int)nj && nj > 1) s_hub[cc * SP + i] = g.hub_dir[0] ? g.hub_dir[jcc >> 7][uu] : -1;
+        }
+      }
+      if (tid == 0) s_rel[span] = ~0u;
+    } else if (lds) {
       for (uint32_t i = tid; i <= span; i += NT) s_off[i] = a.work_off[plo + i];
+    }
     __syncthreads();
     {
       // Each thread's items are processed in lock-step stages (search,
@@ -1452,117 +1502,145 @@ __global__ __launch_bounds__(BLOCK) void k_expand(GView g, KPlan P, ExpandArgs a
                         : (MODE != M_COUNT && MODE != M_GWRITE && MODE != M_WRITE)
                             ? ((L <= 6) ? 4 : 2)
                             : ((L <= 6) ? 4 : (L <= 10 ? COUNT_G_LARGE : 1));
+      const uint32_t n_items = (uint32_t)(w1 - w0);
       for (uint32_t g0 = 0; g0 < ipt; g0 += G) {
-        uint64_t w[G];
-        uint32_t pi[G];
-        bool in[G];
-#pragma unroll
-        for (int j = 0; j < G; ++j) {
-          w[j] = w0 + (uint64_t)(g0 + j) * NT + tid;
-          in[j] = w[j] < w1;
-          pi[j] = 0;
-        }
-        // largest pi with off(pi) <= w: a fixed number of halvings for the
-        // whole block (off(0) <= w0 <= w and off(span) >= w1)
-        for (uint32_t n = span + 1; n > 1;) {
-          const uint32_t half = n >> 1;
-#pragma unroll
-          for (int j = 0; j < G; ++j) {
-            const uint64_t o = lds ? s_off[pi[j] + half] : a.work_off[plo + pi[j] + half];
-            pi[j] = (o <= w[j]) ? pi[j] + half : pi[j];
-          }
-          n -= half;
-        }
-        uint32_t row[G][L], sel[G], jc[G], idx[G], lb[G], v[G], cb[G];
+        uint32_t pi[G], row[G][L], sel[G], jc[G], li[G], v[G], cb[G];
         uint4 pb[G];
-        bool ok[G];
-#pragma unroll
-        for (int j = 0; j < G; ++j) {
-          const uint32_t pj = min(pi[j], span - 1);
-          const uint64_t p = (uint64_t)plo + pj;
-          const uint64_t pbase = lds ? s_off[pj] : a.work_off[p];
-          idx[j] = (uint32_t)(w[j] - pbase);
-#pragma unroll
-          for (int l = 0; l < L; ++l) row[j][l] = a.rows[p * L + l];
-          sel[j] = a.minsel[p];
-          cb[j] = (MODE == M_FUSED && a.cbase) ? a.cbase[p] : 0u;
-          pb[j] = MODE == M_PAIR ? a.pbase[p] : make_uint4(0u, 0u, 0u, 0u);
-          if (a.stats) {
-            bytes += need_sig ? 12 : 4;
-            if (in[j] && idx[j] == 0) bytes += 4 * L + 9 + 8 * nj;
-          }
-        }
-        // hub rows of the first constraints' vertices: they depend on the
-        // row only, so their loads go out with the list base's instead of
-        // after the candidate's
-        constexpr int NJP = 3;
-        int32_t hpre[NJP][G];
-#pragma unroll
-        for (int cc = 0; cc < NJP; ++cc) {
-          const uint32_t jcc = cc < (int)nj ? P.jc[L][cc] : 0u;
+        bool in[G], ok[G];
+        int32_t hpre[NJP][G];  // (not staged)
+        if (staged) {
+          uint32_t w[G];
 #pragma unroll
           for (int j = 0; j < G; ++j) {
-            uint32_t uu = 0;
+            w[j] = (uint32_t)(g0 + j) * NT + tid;
+            in[j] = w[j] < n_items;
+            pi[j] = 0;
+          }
+          for (uint32_t n = span + 1; n > 1;) {
+            const uint32_t half = n >> 1;
+#pragma unroll
+            for (int j = 0; j < G; ++j) pi[j] = s_rel[pi[j] + half] <= w[j] ? pi[j] + half : pi[j];
+            n -= half;
+          }
+#pragma unroll
+          for (int j = 0; j < G; ++j) {
+            li[j] = s_li[pi[j]] + w[j];
+            const uint32_t m = s_meta[pi[j]];
+            sel[j] = m & 255u;
+            jc[j] = m >> 8;
+            if (MODE == M_FUSED) cb[j] = s_cb[pi[j]];
+            if (MODE == M_PAIR) pb[j] = a.pbase[plo + pi[j]];
+#pragma unroll
+            for (int l = 0; l < L; ++l) row[j][l] = s_row[l * SP + pi[j]];
+          }
+        } else {
+          uint64_t w[G];
+#pragma unroll
+          for (int j = 0; j < G; ++j) {
+            w[j] = w0 + (uint64_t)(g0 + j) * NT + tid;
+            in[j] = w[j] < w1;
+            pi[j] = 0;
+          }
+          // largest pi with off(pi) <= w: a fixed number of halvings for the
+          // whole block (off(0) <= w0 <= w and off(span) >= w1)
+          for (uint32_t n = span + 1; n > 1;) {
+            const uint32_t half = n >> 1;
+#pragma unroll
+            for (int j = 0; j < G; ++j) {
+              const uint64_t o = lds ? s_off[pi[j] + half] : a.work_off[plo + pi[j] + half];
+              pi[j] = (o <= w[j]) ? pi[j] + half : pi[j];
+            }
+            n -= half;
+          }
+#pragma unroll
+          for (int j = 0; j < G; ++j) {
+            const uint32_t pj = min(pi[j], span - 1);
+            const uint64_t p = (uint64_t)plo + pj;
+            li[j] = (uint32_t)(w[j] - (lds ? s_off[pj] : a.work_off[p]));
+#pragma unroll
+            for (int l = 0; l < L; ++l) row[j][l] = a.rows[p * L + l];
+            sel[j] = a.minsel[p];
+            cb[j] = (MODE == M_FUSED && a.cbase) ? a.cbase[p] : 0u;
+            pb[j] = MODE == M_PAIR ? a.pbase[p] : make_uint4(0u, 0u, 0u, 0u);
+            if (a.stats) {
+              bytes += need_sig ? 12 : 4;
+              if (in[j] && li[j] == 0) bytes += 4 * L + 9 + 8 * nj;
+            }
+          }
+          // hub rows of the first constraints' vertices: they depend on the
+          // row only, so their loads go out with the list base's instead of
+          // after the candidate's
+#pragma unroll
+          for (int cc = 0; cc < (int)NJP; ++cc) {
+            const uint32_t jcc = cc < (int)nj ? P.jc[L][cc] : 0u;
+#pragma unroll
+            for (int j = 0; j < G; ++j) {
+              uint32_t uu = 0;
+#pragma unroll
+              for (int l = 0; l < L; ++l)
+                if (l == (int)(jcc & 31)) uu = row[j][l];
+              hpre[cc][j] = (g.hub_dir[0] && cc < (int)nj) ? g.hub_dir[jcc >> 7][uu] : -1;
+            }
+          }
+#pragma unroll
+          for (int j = 0; j < G; ++j) {
+            jc[j] = P.jc[L][sel[j]];
+            uint32_t u = 0;
 #pragma unroll
             for (int l = 0; l < L; ++l)
-              if (l == (int)(jcc & 31)) uu = row[j][l];
-            hpre[cc][j] = (g.hub_dir[0] && cc < (int)nj) ? g.hub_dir[jcc >> 7][uu] : -1;
+              if (l == (int)(jc[j] & 31)) u = row[j][l];
+            li[j] += ((jc[j] >> 7) ? g.off_in : g.off_out)[u];
           }
         }
 #pragma unroll
-        for (int j = 0; j < G; ++j) {
-          jc[j] = P.jc[L][sel[j]];
-          uint32_t u = 0;
-#pragma unroll
-          for (int l = 0; l < L; ++l)
-            if (l == (int)(jc[j] & 31)) u = row[j][l];
-          lb[j] = ((jc[j] >> 7) ? g.off_in : g.off_out)[u];
-        }
-#pragma unroll
-        for (int j = 0; j < G; ++j) v[j] = in[j] ? ((jc[j] >> 7) ? g.adj_in : g.adj_out)[lb[j] + idx[j]] : 0u;
+        for (int j = 0; j < G; ++j) v[j] = in[j] ? ((jc[j] >> 7) ? g.adj_in : g.adj_out)[li[j]] : 0u;
         uint2 sg[G];
 #pragma unroll
         for (int j = 0; j < G; ++j)
-          sg[j] = (in[j] && need_sig) ? ((jc[j] >> 7) ? g.nsig_in : g.nsig_out)[lb[j] + idx[j]] : make_uint2(~0u, ~0u);
+          sg[j] = (in[j] && need_sig) ? ((jc[j] >> 7) ? g.nsig_in : g.nsig_out)[li[j]] : make_uint2(~0u, ~0u);
 #pragma unroll
         for (int j = 0; j < G; ++j) {
           ok[j] = in[j] && sg[j].x >= tin && sg[j].y >= tout;
 #pragma unroll
           for (int l = 0; l < L; ++l) ok[j] = ok[j] && v[j] != row[j][l];
         }
-        for (uint32_t c = 0; c < nj; ++c) {
+        // the other constraints (a single one is the list itself)
+        for (uint32_t c = 0; nj > 1 && c < nj; ++c) {
           const uint32_t jc2 = P.jc[L][c];
-          uint32_t u2[G];
-#pragma unroll
-          for (int j = 0; j < G; ++j) {
-            u2[j] = 0;
-#pragma unroll
-            for (int l = 0; l < L; ++l)
-              if (l == (int)(jc2 & 31)) u2[j] = row[j][l];
-          }
           // bit tests for hub lists; the other items' lower-bound searches
           // in lock-step
           const uint32_t dir = jc2 >> 7;
           const int32_t* hid = g.hub_dir[dir];
           const uint64_t* hbits = g.bits_dir[dir];
-          const bool hubs = hid != nullptr;
           const uint32_t* off2 = dir ? g.off_in : g.off_out;
           const uint32_t* adj2 = dir ? g.adj_in : g.adj_out;
-          bool srch[G];
-          if (hubs) {
+          auto owner = [&](int j) {
+            uint32_t u = 0;
+#pragma unroll
+            for (int l = 0; l < L; ++l)
+              if (l == (int)(jc2 & 31)) u = row[j][l];
+            return u;
+          };
+          bool srch[G], any = false;
+          if (hid) {
             int32_t h[G];
             uint64_t bw[G];
 #pragma unroll
             for (int j = 0; j < G; ++j) {
-              int32_t hh = 0;
+              if (c >= NJP) {
+                h[j] = hid[owner(j)];
+              } else if (staged) {
+                h[j] = s_hub[c * SP + pi[j]];
+              } else {
+                h[j] = 0;
 #pragma unroll
-              for (int cc = 0; cc < NJP; ++cc)
-                if ((int)c == cc) hh = hpre[cc][j];
-              h[j] = c < (uint32_t)NJP ? hh : hid[u2[j]];
+                for (int cc = 0; cc < (int)NJP; ++cc)
+                  if ((int)c == cc) h[j] = hpre[cc][j];
+              }
             }
 #pragma unroll
             for (int j = 0; j < G; ++j)
-              bw[j] = hbits[h[j] >= 0 ? (uint64_t)h[j] * g.words + (v[j] >> 6) : 0];
+              bw[j] = (ok[j] && c != sel[j] && h[j] >= 0) ? hbits[(uint64_t)h[j] * g.words + (v[j] >> 6)] : 0ull;
 #pragma unroll
             for (int j = 0; j < G; ++j) {
               srch[j] = false;
@@ -1571,25 +1649,31 @@ __global__ __launch_bounds__(BLOCK) void k_expand(GView g, KPlan P, ExpandArgs a
                 ok[j] = (bw[j] >> (v[j] & 63)) & 1ull;
                 if (a.stats) bytes += 12;
               } else {
-                srch[j] = true;
+                srch[j] = any = true;
               }
             }
           } else {
 #pragma unroll
-            for (int j = 0; j < G; ++j) srch[j] = ok[j] && c != sel[j];
+            for (int j = 0; j < G; ++j) {
+              srch[j] = ok[j] && c != sel[j];
+              any = any || srch[j];
+            }
           }
-          uint32_t sb[G], sn[G];
-          bool fnd[G];
+          if (any) {
+            uint32_t sb[G], sn[G];
+            bool fnd[G];
 #pragma unroll
-          for (int j = 0; j < G; ++j) {
-            sb[j] = srch[j] ? off2[u2[j]] : 0u;
-            sn[j] = srch[j] ? off2[u2[j] + 1] - sb[j] : 0u;
-            if (a.stats && srch[j]) bytes += (hubs ? 12 : 8) + bs_bytes(sn[j]);
+            for (int j = 0; j < G; ++j) {
+              const uint32_t u2 = owner(j);
+              sb[j] = srch[j] ? off2[u2] : 0u;
+              sn[j] = srch[j] ? off2[u2 + 1] - sb[j] : 0u;
+              if (a.stats && srch[j]) bytes += (hid ? 12 : 8) + bs_bytes(sn[j]);
+            }
+            members_lockstep<G>(adj2, sb, sn, v, fnd);
+#pragma unroll
+            for (int j = 0; j < G; ++j)
+              if (srch[j]) ok[j] = fnd[j];
           }
-          members_lockstep<G>(adj2, sb, sn, v, fnd);
-#pragma unroll
-          for (int j = 0; j < G; ++j)
-            if (srch[j]) ok[j] = fnd[j];
         }
         if (MODE == M_WRITE) {
           // survivors of the G items: one block-wide reservation on
