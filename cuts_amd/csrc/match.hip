@@ -1367,10 +1367,11 @@ __device__ __forceinline__ uint64_t next_tile(unsigned int* tilectr, uint64_t nt
   return ~0ull;
 }
 
-// Four waves per SIMD for rows of up to 5 words (128 registers): at three the
-// R-MAT 20 tail expansion took 6.0 ms for 5.0.
+// Five waves per SIMD for rows of up to 4 words (96 registers), four for 5:
+// the R-MAT 20 tail query took 6.0 / 5.0 / 4.5 / 4.5 ms at three to six, the
+// directed last level 79.8 / 79.6 / 68.1 / 70.8.
 template <int L, int MODE>
-__global__ __launch_bounds__(BLOCK, L <= 5 ? 4 : 1) void k_expand(GView g, KPlan P, ExpandArgs a) {
+__global__ __launch_bounds__(BLOCK, L <= 4 ? 5 : L <= 5 ? 4 : 1) void k_expand(GView g, KPlan P, ExpandArgs a) {
   // A tile of at most SP prefixes stages them in LDS, one thread per prefix:
   // where its items start in the tile, its row, the list position of its
   // items (less their index in the tile), its list's constraint and the hub
