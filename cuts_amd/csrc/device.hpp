@@ -188,7 +188,7 @@ struct LevelBuf {
   // of its block in `cand` (n+1; a block holds as many entries as the
   // prefix's shortest constraint list) and the candidates of position k-3
   uint64_t* coff = nullptr;
-  uint32_t* cand = nullptr;
+  uint2* cand = nullptr;        // (vertex, degree)
   uint64_t coff_cap = 0, cand_cap = 0;
   uint64_t* bsum = nullptr;     // scan partials
   uint64_t bsum_cap = 0;

@@ -1220,7 +1220,7 @@ static __global__ __launch_bounds__(BLOCK) void k_cnt_table(GView g, uint32_t th
 // the chain count of the row + candidate.  Tiles as in k_expand.
 struct SibArgs {
   const uint32_t* rows;
-  const uint32_t* cand;
+  const uint2* cand;           // (vertex, degree)
   const uint32_t* shared;      // per row: its own positions' intersections with u
   const uint4* pb;             // per row: the chain closed form's row part (k_sib_base)
   const uint64_t* rstart;      // per row: start of its parent's block in cand
@@ -1272,7 +1272,7 @@ struct ExpandArgs {
   ChainTables ctab;          // M_CHAIN
   PairTables ptab;           // M_COLLAPSE, M_TAIL
   const uint64_t* coff;      // M_GWRITE: start of every prefix's block in cand
-  uint32_t* cand;            // M_GWRITE: candidates grouped by prefix
+  uint2* cand;               // M_GWRITE: candidates (vertex, degree) grouped by prefix
   uint32_t xcd;              // 1: XCD-contiguous tile mapping
   unsigned int* tilectr;     // 8 tile counters kTileStride apart, zero at launch
   uint32_t stats;            // 1: accumulate demand bytes into counters[3]
@@ -1378,7 +1378,7 @@ __global__ __launch_bounds__(BLOCK, L <= 4 ? 5 : L <= 5 ? 4 : 1) void k_expand(G
   // rows of the first NJP constraints.  An item then takes its prefix from
   // LDS by 32-bit searches and reads instead of repeating the prefix's loads
   // and address arithmetic, which bound the kernel by instruction issue
-  // (a directed last level of 1.3e10 items: 111 -> 79.6 ms).  Tiles
+  // (a directed last level of 1.3e10 items: 111 -> 56.8 ms).  Tiles
   // of more prefixes (short lists) keep the offsets alone, or nothing.
   constexpr uint32_t SP = 256, NJP = 3;
   constexpr uint32_t STAGE_WORDS = (SP + 1) + (L + 3 + NJP) * SP;
@@ -1391,6 +1391,8 @@ __global__ __launch_bounds__(BLOCK, L <= 4 ? 5 : L <= 5 ? 4 : 1) void k_expand(G
   uint32_t* const s_meta = s_li + SP;            // SP: constraint index | jc << 8
   uint32_t* const s_cb = s_meta + SP;            // SP
   int32_t* const s_hub = (int32_t*)(s_cb + SP);  // NJP x SP
+  __shared__ uint32_t s_pos[NJP];                // owner positions of the first constraints
+  if (threadIdx.x < NJP) s_pos[threadIdx.x] = P.jc[L][threadIdx.x] & 31u;  // before the tile loop's first barrier
   __shared__ uint32_t s_w[BLOCK / 64], s_pre[BLOCK / 64], s_base;
   const uint32_t tid = threadIdx.x, wave = tid >> 6;
   // threads per block: BLOCK for the writing expansion; 64, 128 or 256 for
@@ -1407,6 +1409,13 @@ __global__ __launch_bounds__(BLOCK, L <= 4 ? 5 : L <= 5 ? 4 : 1) void k_expand(G
   // a last level that is counted entry by entry reads no signatures where its
   // constraints imply them (always, short of query self-loops)
   const bool need_sig = MODE != M_COUNT || !((P.sig_implied >> L) & 1);
+  // all constraints on lists of one direction (every symmetric graph's): their
+  // tables are the same for all lanes
+  bool onedir = true;
+  const uint32_t dir0 = P.jc[L][0] >> 7;
+  for (uint32_t c = 1; c < nj; ++c) onedir = onedir && (uint32_t)(P.jc[L][c] >> 7) == dir0;
+  const uint32_t* const adj1 = dir0 ? g.adj_in : g.adj_out;
+  const uint2* const nsig1 = dir0 ? g.nsig_in : g.nsig_out;
   uint64_t acc = 0, valid = 0, pairs = 0, trips = 0, bytes = 0, mb = 0;
   // modes whose survivors wait in a queue of their wave: prefix, vertex,
   // degree (at most 63 left over and 64 new)
@@ -1594,19 +1603,61 @@ __global__ __launch_bounds__(BLOCK, L <= 4 ? 5 : L <= 5 ? 4 : 1) void k_expand(G
           }
         }
 #pragma unroll
-        for (int j = 0; j < G; ++j) v[j] = in[j] ? ((jc[j] >> 7) ? g.adj_in : g.adj_out)[li[j]] : 0u;
+        for (int j = 0; j < G; ++j) v[j] = in[j] ? (onedir ? adj1 : (jc[j] >> 7) ? g.adj_in : g.adj_out)[li[j]] : 0u;
         uint2 sg[G];
 #pragma unroll
         for (int j = 0; j < G; ++j)
-          sg[j] = (in[j] && need_sig) ? ((jc[j] >> 7) ? g.nsig_in : g.nsig_out)[li[j]] : make_uint2(~0u, ~0u);
+          sg[j] = (in[j] && need_sig) ? (onedir ? nsig1 : (jc[j] >> 7) ? g.nsig_in : g.nsig_out)[li[j]]
+                                      : make_uint2(~0u, ~0u);
 #pragma unroll
         for (int j = 0; j < G; ++j) {
           ok[j] = in[j] && sg[j].x >= tin && sg[j].y >= tout;
 #pragma unroll
           for (int l = 0; l < L; ++l) ok[j] = ok[j] && v[j] != row[j][l];
         }
-        // the other constraints (a single one is the list itself)
-        for (uint32_t c = 0; nj > 1 && c < nj; ++c) {
+        // the other constraints (a single one is the list itself).  Staged and
+        // of one direction, each item goes through its own others alone, with
+        // the list's owner and hub row from LDS
+        const bool others = staged && onedir && nj <= NJP;
+        for (uint32_t t = 0; others && t + 1 < nj; ++t) {
+          const int32_t* hid = g.hub_dir[dir0];
+          const uint64_t* hbits = g.bits_dir[dir0];
+          uint32_t c[G];
+          int32_t h[G];
+          uint64_t bw[G];
+          bool any = false;
+#pragma unroll
+          for (int j = 0; j < G; ++j) {
+            c[j] = t + (t >= sel[j] ? 1u : 0u);
+            h[j] = hid ? s_hub[c[j] * SP + pi[j]] : -1;
+            bw[j] = ~0ull;
+          }
+#pragma unroll
+          for (int j = 0; j < G; ++j)
+            if (ok[j] && h[j] >= 0) bw[j] = hbits[(uint64_t)h[j] * g.words + (v[j] >> 6)];
+#pragma unroll
+          for (int j = 0; j < G; ++j) {
+            ok[j] = ok[j] && ((bw[j] >> (v[j] & 63)) & 1ull);
+            any = any || (ok[j] && h[j] < 0);
+          }
+          if (any) {
+            const uint32_t* off2 = dir0 ? g.off_in : g.off_out;
+            uint32_t sb[G], sn[G];
+            bool fnd[G];
+#pragma unroll
+            for (int j = 0; j < G; ++j) {
+              const bool s = ok[j] && h[j] < 0;
+              const uint32_t u2 = s_row[s_pos[c[j]] * SP + pi[j]];
+              sb[j] = s ? off2[u2] : 0u;
+              sn[j] = s ? off2[u2 + 1] - sb[j] : 0u;
+            }
+            members_lockstep<G>(adj1, sb, sn, v, fnd);
+#pragma unroll
+            for (int j = 0; j < G; ++j)
+              if (ok[j] && h[j] < 0) ok[j] = fnd[j];
+          }
+        }
+        for (uint32_t c = 0; !others && nj > 1 && c < nj; ++c) {
           const uint32_t jc2 = P.jc[L][c];
           // bit tests for hub lists; the other items' lower-bound searches
           // in lock-step
@@ -1720,8 +1771,8 @@ __global__ __launch_bounds__(BLOCK, L <= 4 ? 5 : L <= 5 ? 4 : 1) void k_expand(G
           for (int j = 0; j < G; ++j) {
             if (!ok[j]) continue;
             const uint64_t p = (uint64_t)plo + min(pi[j], span - 1);
-            a.cand[a.coff[p] + atomicAdd(&a.nsurv[p], 1u)] = v[j];
-            if (a.stats) bytes += 16;  // block start, slot counter, candidate
+            a.cand[a.coff[p] + atomicAdd(&a.nsurv[p], 1u)] = make_uint2(v[j], sg[j].x);
+            if (a.stats) bytes += 20;  // block start, slot counter, candidate
           }
         } else if (MODE == M_COLLAPSE) {
           // a survivor v completes the prefix of positions 0..k-4 of a
@@ -2011,42 +2062,20 @@ __global__ __launch_bounds__(BLOCK) void k_sib_base(GView g, KPlan P, const uint
   }
 }
 
-// The candidate's part of the chain closed form on top of the row's base
-// (k_sib_base); na receives na_old - inv.
-template <int L>
-__device__ __forceinline__ int64_t chain_sib_item(const GView& g, const KPlan& P, const uint32_t (&r)[L], uint32_t v,
-                                                  uint4 pbq, const ChainTables& t, int64_t& na, uint64_t& bytes) {
-  const uint32_t inu = pbq.w & 0x7FFFu, dold = (pbq.w >> 15) & 0x7FFFu;
-  const bool dtb = (pbq.w >> 30) & 1u;
-  int64_t c = (int64_t)(((uint64_t)pbq.y << 32) | pbq.x);
-  uint32_t u = 0;
-#pragma unroll
-  for (int l = 0; l < L; ++l)
-    if (l == (int)P.ch_u) u = r[l];
-  const uint32_t dv = g.sig[2 * (uint64_t)v];
-  bytes += 4;
-  const bool inv = dv >= P.ch_ta && (((P.qadj[P.ch_u] >> L) & 1) || adj_has(g, u, v, bytes));
-  na = (int64_t)pbq.z - (inv ? 1 : 0);
-  if (inv) {
-    c -= t.tb ? t.tb[v] : g.off_out[v + 1] - g.off_out[v];
-    bytes += t.tb ? 4 : 8;
-    if (dtb) ++c;
-#pragma unroll
-    for (int i = 0; i < L; ++i)
-      if (((dold >> i) & 1) && (((P.qadj[i] >> L) & 1) || adj_has(g, r[i], v, bytes))) ++c;
-  }
-  if (P.ch_tb <= 1 || dv >= P.ch_tb) {
-#pragma unroll
-    for (int j = 0; j < L; ++j)
-      if (((inu >> j) & 1) && (((P.qadj[L] >> j) & 1) || adj_has(g, v, r[j], bytes))) ++c;
-    c -= two_hop(g, u, v, bytes);
-  }
-  return c;
-}
-
+// The rows of a tile are staged in LDS (a thread per row, at most SP rows;
+// else read from memory), with the hub rows of their vertices and the dense
+// two-hop row of u: an item then gathers its candidate's dense count, one bit
+// word per uncertain adjacency and nothing else (17 loads per item before,
+// which bound the kernel; the two 6-vertex queries at 36,692 vertices, with
+// 2.0e8 items here: 4.99 -> 4.21 ms).
 template <int L>
 __global__ __launch_bounds__(BLOCK) void k_chain_sib(GView g, KPlan P, SibArgs a, ChainTables t) {
+  constexpr uint32_t SP = 256;
   __shared__ uint64_t s_off[LDS_OFF + 1];
+  __shared__ uint4 s_pb[SP];
+  __shared__ uint64_t s_start[SP];
+  __shared__ uint32_t s_row[L][SP];
+  __shared__ int32_t s_hub[L][SP], s_did[SP];
   __shared__ uint64_t s_tile;
   const uint32_t tid = threadIdx.x;
   uint64_t acc = 0, valid = 0, pairs = 0, bytes = 0, mb = 0;
@@ -2065,6 +2094,38 @@ __global__ __launch_bounds__(BLOCK) void k_chain_sib(GView g, KPlan P, SibArgs a
     const bool lds = span <= LDS_OFF;
     if (lds)
       for (uint32_t i = tid; i <= span; i += BLOCK) s_off[i] = a.work_off[plo + i];
+    // what an item needs of row q: its vertices, their hub rows, u's dense
+    // two-hop row, the row's base, the start of its candidates less its items'
+    // start
+    auto load_row = [&](uint64_t q, uint32_t (&r)[L], int32_t (&h)[L], int32_t& did, uint4& pbq, uint64_t& start) {
+      pbq = a.pb[q];
+      start = a.rstart[q] - a.work_off[q];
+      uint32_t u = 0;
+#pragma unroll
+      for (int l = 0; l < L; ++l) {
+        r[l] = a.rows[q * L + l];
+        if (l == (int)P.ch_u) u = r[l];
+      }
+#pragma unroll
+      for (int l = 0; l < L; ++l) h[l] = g.hub_id ? g.hub_id[r[l]] : -1;
+      did = g.h2_did ? g.h2_did[u] : -1;
+    };
+    const bool staged = span <= SP && !a.stats;
+    if (staged && tid < span) {
+      uint32_t r[L];
+      int32_t h[L], did;
+      uint4 pbq;
+      uint64_t start;
+      load_row((uint64_t)plo + tid, r, h, did, pbq, start);
+#pragma unroll
+      for (int l = 0; l < L; ++l) {
+        s_row[l][tid] = r[l];
+        s_hub[l][tid] = h[l];
+      }
+      s_did[tid] = did;
+      s_pb[tid] = pbq;
+      s_start[tid] = start;
+    }
     __syncthreads();
     if (a.stats) {
       // profiling: the full closed form per item (it also counts the merge
@@ -2082,7 +2143,7 @@ __global__ __launch_bounds__(BLOCK) void k_chain_sib(GView g, KPlan P, SibArgs a
         const uint32_t pi = lo - 1;
         const uint64_t q = (uint64_t)plo + pi;
         const uint64_t qbase = lds ? s_off[pi] : a.work_off[q];
-        const uint32_t v = a.cand[a.rstart[q] + (w - qbase)];
+        const uint32_t v = a.cand[a.rstart[q] + (w - qbase)].x;
         uint32_t r[L + 1];
 #pragma unroll
         for (int l = 0; l < L; ++l) r[l] = a.rows[q * L + l];
@@ -2116,28 +2177,82 @@ __global__ __launch_bounds__(BLOCK) void k_chain_sib(GView g, KPlan P, SibArgs a
         }
         nn -= half;
       }
-      uint64_t q[IPT], cidx[IPT];
+      uint32_t r[IPT][L];
+      int32_t h[IPT][L], did[IPT];
       uint4 pbq[IPT];
-      uint32_t r[IPT][L], v[IPT];
+      uint64_t at[IPT];
+      uint2 cd[IPT];
 #pragma unroll
       for (int j = 0; j < IPT; ++j) {
         const uint32_t pj = min(pi[j], span - 1);
-        q[j] = (uint64_t)plo + pj;
-        const uint64_t qbase = lds ? s_off[pj] : a.work_off[q[j]];
-        cidx[j] = a.rstart[q[j]] + (w[j] - qbase);
-        pbq[j] = a.pb[q[j]];
+        if (staged) {
 #pragma unroll
-        for (int l = 0; l < L; ++l) r[j][l] = a.rows[q[j] * L + l];
+          for (int l = 0; l < L; ++l) {
+            r[j][l] = s_row[l][pj];
+            h[j][l] = s_hub[l][pj];
+          }
+          did[j] = s_did[pj];
+          pbq[j] = s_pb[pj];
+          at[j] = s_start[pj];
+        } else {
+          load_row((uint64_t)plo + pj, r[j], h[j], did[j], pbq[j], at[j]);
+        }
       }
 #pragma unroll
-      for (int j = 0; j < IPT; ++j) v[j] = in[j] ? a.cand[cidx[j]] : 0u;
+      for (int j = 0; j < IPT; ++j) cd[j] = in[j] ? a.cand[at[j] + w[j]] : make_uint2(0u, 0u);
+      // |N(u) & N(v)| and the vertices' adjacency to the candidate: bit words
+      // and dense counts of all items first
+      const uint32_t sure = P.qadj[L];
+      uint32_t adj[IPT], ask[IPT], cn[IPT];
 #pragma unroll
       for (int j = 0; j < IPT; ++j) {
-        if (!in[j] || v[j] == r[j][L - 1]) continue;
+        in[j] = in[j] && cd[j].x != r[j][L - 1];
+        const uint32_t inu = pbq[j].w & 0x7FFFu, dold = (pbq[j].w >> 15) & 0x7FFFu;
+        const bool va = cd[j].y >= P.ch_ta, vb = P.ch_tb <= 1 || cd[j].y >= P.ch_tb;
+        // vertices whose adjacency to v the count takes: u for [v in N(u)],
+        // dold when v is in N(u), inu when v meets tb
+        ask[j] = !in[j] ? 0u : (va ? dold | (1u << P.ch_u) : 0u) | (vb ? inu : 0u);
+        adj[j] = sure & ask[j];
+        ask[j] &= ~sure;
+        cn[j] = 0;
+        if (in[j] && vb && did[j] >= 0) cn[j] = g.h2_dense[(uint64_t)did[j] * g.V + cd[j].x];
+      }
+#pragma unroll
+      for (int l = 0; l < L; ++l) {
+        uint64_t bw[IPT];
+#pragma unroll
+        for (int j = 0; j < IPT; ++j)
+          bw[j] = ((ask[j] >> l) & 1) && h[j][l] >= 0 ? g.bits[(uint64_t)h[j][l] * g.words + (cd[j].x >> 6)] : 0ull;
+#pragma unroll
+        for (int j = 0; j < IPT; ++j) {
+          bool yes = (bw[j] >> (cd[j].x & 63)) & 1ull;
+          if (((ask[j] >> l) & 1) && h[j][l] < 0)
+            yes = member_safe(g.adj_out, g.off_out[r[j][l]], g.off_out[r[j][l] + 1], cd[j].x);
+          adj[j] |= (uint32_t)yes << l;
+        }
+      }
+#pragma unroll
+      for (int j = 0; j < IPT; ++j) {
+        if (!in[j]) continue;
         ++valid;
-        int64_t na = 0;
-        acc += (uint64_t)chain_sib_item<L>(g, P, r[j], v[j], pbq[j], t, na, bytes);
-        pairs += (uint64_t)na;
+        const uint32_t v = cd[j].x, dv = cd[j].y;
+        const uint32_t inu = pbq[j].w & 0x7FFFu, dold = (pbq[j].w >> 15) & 0x7FFFu;
+        int64_t cc = (int64_t)(((uint64_t)pbq[j].y << 32) | pbq[j].x);
+        const bool inv = dv >= P.ch_ta && ((adj[j] >> P.ch_u) & 1);
+        if (inv) cc += (int64_t)((pbq[j].w >> 30) & 1u) + __popc(adj[j] & dold) - (int64_t)(t.tb ? t.tb[v] : dv);
+        if (P.ch_tb <= 1 || dv >= P.ch_tb) {
+          cc += __popc(adj[j] & inu);
+          if (did[j] < 0) {
+            uint32_t u = 0;
+#pragma unroll
+            for (int l = 0; l < L; ++l)
+              if (l == (int)P.ch_u) u = r[j][l];
+            cn[j] = index_common(g, u, v, bytes);
+          }
+          cc -= cn[j];
+        }
+        acc += (uint64_t)cc;
+        pairs += (uint64_t)((int64_t)pbq[j].z - (inv ? 1 : 0));
       }
     }
     __syncthreads();
@@ -3688,7 +3803,7 @@ struct Matcher {
       level_cap[l] = std::max<uint64_t>(per / ((l + 1) * 4 + 17 + 24), 1024);
     }
     // shared chain candidates: up to one level's share of the budget
-    cand_limit = std::max<uint64_t>((nlev ? budget / nlev : budget) / 4, 1u << 10);
+    cand_limit = std::max<uint64_t>((nlev ? budget / nlev : budget) / 8, 1u << 10);
     if (closed_last && kp.sc_thr > 1) tbl = cnt_table(c, dg, arena, kp.sc_thr);
     // with the two-hop index the chain is counted inside the expansion of
     // position k-3 (no rows of level k-3 are stored)
