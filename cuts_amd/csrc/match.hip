@@ -379,7 +379,7 @@ __device__ __forceinline__ void add_wave(unsigned long long* dst, uint64_t v) {
 // atomics of all XCDs on one line are served one after another, about 13 ns
 // each: the 18,000 final adds of a full grid took 230 of the 310 us of the
 // 4,096-vertex graph's triangle + 2-edge tail.  k_publish_end adds the slots up.
-constexpr uint32_t kSlots = 64, kLine = 32, kSlot0 = kLine, kTile0 = kSlot0 + kSlots * kLine,
+[[maybe_unused]] constexpr uint32_t kSlots = 64, kLine = 32, kSlot0 = kLine, kTile0 = kSlot0 + kSlots * kLine,
                    kCounterWords = kTile0 + 8 * kLine;
 constexpr uint32_t kTileStride = 2 * kLine;  // 32-bit words between tile counters
 
@@ -3128,7 +3128,10 @@ struct Matcher {
     else if (L == k - 2 && fuse) mode = M_FUSED;
     const int mclass = mode == M_WRITE ? 4 : mode == M_COUNT ? 5 : (mode == M_FUSED || mode == M_TAIL) ? 6 : (mode == M_PAIR || mode == M_COLLAPSE) ? 8 : 10;
     if (mode == M_PAIR) ensure_aux(arena, in.pbase, in.pbase_cap, n);
-    const bool spec = speculate() && !(mode == M_WRITE && L == k - 1);
+    // a last level that writes embeddings runs without the readback of its
+    // work only where one block plans it (an interactive look at a few rows:
+    // three launches and two readbacks fewer); larger ones go out in chunks
+    const bool spec = speculate() && !(mode == M_WRITE && L == k - 1 && n > (uint64_t)SCAN_TILE);
     // a speculative level of at most SCAN_TILE rows plans, scans and indexes
     // its tiles in one launch (k_plan_small, inside level_spec)
     const bool small = spec && n <= (uint64_t)SCAN_TILE;
@@ -3315,6 +3318,11 @@ struct Matcher {
       // the level's share of the budget)
       ensure_rows_exact(arena, out, std::min<uint64_t>(std::max<uint64_t>(out.cap, 1ull << 16), level_cap[L]), L + 1);
       row_cap = std::min<uint64_t>(out.cap, level_cap[L]);
+      if (L == k - 1) {
+        row_cap = std::min<uint64_t>(row_cap, 1ull << 16);
+        // copies of earlier chunks out of this buffer
+        for (int b = 0; b < 2 && emb_chunks; ++b) HIPCHECK(hipStreamWaitEvent(c.stream, c.copy_ev[b], 0));
+      }
       if (want_parent) ensure_aux(arena, out.parent, out.parent_cap, out.cap);
     }
     const bool pair_common = mode == M_PAIR && kp.pr_a != kp.pr_b && !pair_cab_known();
@@ -3408,7 +3416,18 @@ struct Matcher {
         return false;
       }
       r.level[L] += m;
-      if (m) level(L + 1, out.rows, m);
+      if (L == k - 1) {
+        // embeddings, copied in stream order: the buffer's next rows and the
+        // end of the run come after
+        r.count += m;
+        const uint64_t take = std::min(o.emb_cap > r.emb_written ? o.emb_cap - r.emb_written : 0, m);
+        if (take && o.emb_rows) {
+          HIPCHECK(hipMemcpyAsync(o.emb_rows + r.emb_written * k, out.rows, take * k * 4, hipMemcpyDeviceToHost, c.stream));
+          r.emb_written += take;
+        }
+      } else if (m) {
+        level(L + 1, out.rows, m);
+      }
       return true;
     }
 #define EXS(LL, MD) hipLaunchKernelGGL((k_expand<LL, MD>), dim3(grid * cgrow), dim3(nthr), 0, c.stream, g, kp, a)
