@@ -926,6 +926,25 @@ __device__ __forceinline__ void publish_rows(uint64_t* publish, uint32_t rows, u
   __hip_atomic_store(&publish[0], (uint64_t)rows, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
+// One thread: the tiles of a speculative level handed to its expansion, or
+// withheld (dyn = {0, 0}) with a bit of *status set: 0, it does not fit; 1,
+// with it the run would examine more than work_cap candidates (the work cap
+// less what the host has counted).  Only this thread looks at *work, which it
+// alone changes: the other threads may index tiles that nothing then takes.
+// The work of a counting level beyond the cap is added all the same, as the
+// readback does; a writing level is run again with the readback.
+static __device__ __forceinline__ bool claim_work(bool fits, uint64_t W, uint64_t nt, unsigned long long* dyn,
+                                           unsigned long long* status, unsigned long long* work, uint64_t work_cap,
+                                           bool writes) {
+  const bool over = W > work_cap || *work > work_cap - W;
+  const bool go = fits && !over;
+  dyn[0] = go ? W : 0ull;
+  dyn[1] = go ? nt : 0ull;
+  if (go || (over && !writes)) *work += W;
+  if (!go) *status |= over ? 2ull : 1ull;
+  return go;
+}
+
 // The same index without a host readback of the level's work: W = off[n] is
 // read on the device.  When it fits (W <= max_items, ceil(W / TILE) + 1 <=
 // tile_cap entries, W <= row_cap) the tiles of [0, W) are indexed, dyn =
@@ -940,7 +959,8 @@ static __global__ __launch_bounds__(BLOCK) void k_tile_index_dyn(const uint64_t*
                                                          unsigned int* __restrict__ outctr,
                                                          unsigned long long* __restrict__ dyn,
                                                          unsigned long long* __restrict__ status,
-                                                         unsigned long long* __restrict__ work, uint64_t* publish) {
+                                                         unsigned long long* __restrict__ work, uint64_t work_cap,
+                                                         uint64_t* publish) {
   const uint64_t W = off[n];
   const uint64_t nt = (W + TILE - 1) / TILE;
   const bool fits = W <= max_items && nt + 1 <= tile_cap && W <= row_cap;
@@ -948,12 +968,9 @@ static __global__ __launch_bounds__(BLOCK) void k_tile_index_dyn(const uint64_t*
     if (threadIdx.x < 8) tilectr[threadIdx.x * kTileStride] = 0u;
     if (outctr && threadIdx.x < 2) outctr[threadIdx.x] = 0u;
     if (threadIdx.x == 0) {
-      dyn[0] = fits ? W : 0ull;
-      dyn[1] = fits ? nt : 0ull;
-      if (fits) *work += W;
-      else *status |= 1ull;
+      const bool go = claim_work(fits, W, nt, dyn, status, work, work_cap, publish != nullptr);
       // a writing level with no tiles: no expansion block will publish
-      if (publish && (!fits || W == 0)) publish_rows(publish, 0u, fits ? 0ull : 1ull);
+      if (publish && (!go || W == 0)) publish_rows(publish, 0u, go ? 0ull : 1ull);
     }
   }
   if (!fits || W == 0) return;
@@ -988,7 +1005,8 @@ __global__ __launch_bounds__(BLOCK) void k_plan_small(GView g, KPlan P, const ui
                                                       unsigned int* __restrict__ outctr,
                                                       unsigned long long* __restrict__ dyn,
                                                       unsigned long long* __restrict__ status,
-                                                      unsigned long long* __restrict__ work, uint64_t* publish,
+                                                      unsigned long long* __restrict__ work, uint64_t work_cap,
+                                                      uint64_t* publish,
                                                       const unsigned long long* __restrict__ dn,
                                                       unsigned long long* __restrict__ lvc) {
   __shared__ uint64_t s_off[SCAN_TILE + 1];
@@ -1049,11 +1067,8 @@ __global__ __launch_bounds__(BLOCK) void k_plan_small(GView g, KPlan P, const ui
   if (threadIdx.x < 8) tilectr[threadIdx.x * kTileStride] = 0u;
   if (outctr && threadIdx.x < 2) outctr[threadIdx.x] = 0u;
   if (threadIdx.x == 0) {
-    dyn[0] = fits ? W : 0ull;
-    dyn[1] = fits ? nt : 0ull;
-    if (fits) *work += W;
-    else *status |= 1ull;
-    if (publish && (!fits || W == 0)) publish_rows(publish, 0u, fits ? 0ull : 1ull);
+    const bool go = claim_work(fits, W, nt, dyn, status, work, work_cap, publish != nullptr);
+    if (publish && (!go || W == 0)) publish_rows(publish, 0u, go ? 0ull : 1ull);
   }
   __syncthreads();
   if (!fits || W == 0) return;
@@ -2957,6 +2972,7 @@ struct Matcher {
     if (o.max_work && r.work > o.max_work) {
       aborted = true;
       r.work_capped = 1;
+      cap_exact = !dev_work;
     }
     return aborted;
   }
@@ -3027,10 +3043,22 @@ struct Matcher {
   // counting level none.  A writing level that did not fit is redone with
   // the readback at once; a counting level that did not fit leaves the
   // status bit for the end of the run, which then repeats the whole query
-  // with readbacks.  Off for profiling, work caps, deadlines, the
-  // no-allocation entry point and CUTS_FLAG_SYNC_LEVELS.
+  // with readbacks.  Off for profiling, deadlines, the no-allocation entry
+  // point and CUTS_FLAG_SYNC_LEVELS.
+  // A work cap is tested on the device too (claim_work), against the cap less
+  // the work counted on the host, so a level beyond it is never expanded: a
+  // writing level is then run with the readback, which decides as it does
+  // without speculation; a counting level ends the run where it is the run's
+  // only branch (capped_at_end), and otherwise the run is repeated with
+  // readbacks.  A capped run that stays below its cap thus has the launches
+  // and readbacks of one without: a 6-vertex query of 4.1 M candidates on
+  // R-MAT 20, more than 0.185 ms with its levels read back, takes 0.129.
   bool no_spec = false;
   bool spec_overflow = false;
+  bool dev_work = false;     // candidates counted on the device and not yet in r.work
+  bool cap_exact = false;    // the cap was passed with all work counted
+  bool common_spec = false;  // a speculative pass over stored rows' intersections was planned
+  uint64_t work_left() const { return o.max_work ? o.max_work - std::min(o.max_work, r.work) : ~0ull; }
   // level sizes of the last complete run of this query, or null; bit l:
   // level l's size was handed on on the device (read from lvcnt at the end)
   const uint64_t* hint = nullptr;
@@ -3051,7 +3079,7 @@ struct Matcher {
     return true;
   }
   bool speculate() const {
-    return !no_spec && !prof && !o.max_work && !has_deadline && !arena && !(o.flags & 8192u);
+    return !no_spec && !prof && !has_deadline && !arena && !(o.flags & 8192u);
   }
   // Word w of the coherent host words once the stream has drained: true
   // when a kernel published it (it holds ~0 until then).  Polling the word
@@ -3063,17 +3091,17 @@ struct Matcher {
   }
   // tile index over [0, W) with W read on the device; returns the launch
   // shape bound (the most tiles the index may hold)
-  // status: ctr[11] for a writing level (read back with its row count),
-  // ctr[12] for the counting levels (read at the end of the run)
+  // status: ctr[11] for a writing level whose row count is read back (with
+  // it), ctr[12] for the others (read at the end of the run)
   // (a writing level: at most MAX_CHUNK items; a counting one MAX_SPEC_ITEMS)
-  uint64_t tile_index_dyn(LevelBuf& in, uint64_t n, uint64_t row_cap, unsigned int* outctr, uint64_t* publish = nullptr) {
+  uint64_t tile_index_dyn(LevelBuf& in, uint64_t n, uint64_t row_cap, unsigned int* outctr, unsigned long long* status,
+                          uint64_t* publish = nullptr) {
     ensure_tiles(arena, in, std::max<uint64_t>(in.tile_cap, 4097) - 1);
     const uint64_t tcap = in.tile_cap;
     const uint32_t tg = (uint32_t)std::min<uint64_t>((tcap + BLOCK - 1) / BLOCK, 1024);
     hipLaunchKernelGGL(k_tile_index_dyn, dim3(tg), dim3(BLOCK), 0, c.stream, in.work_off, n,
                        outctr ? MAX_CHUNK : MAX_SPEC_ITEMS, tcap, row_cap,
-                       in.tile_p, (unsigned int*)(ctr + kTile0), outctr, ctr + 14, outctr ? ctr + 11 : ctr + 12, ctr + 13,
-                       publish);
+                       in.tile_p, (unsigned int*)(ctr + kTile0), outctr, ctr + 14, status, ctr + 13, work_left(), publish);
     HIPCHECK(hipGetLastError());
     return tcap - 1;
   }
@@ -3309,6 +3337,7 @@ struct Matcher {
   bool level_spec(uint32_t L, const uint32_t* rows, uint64_t n, LevelBuf& in, int mode, bool use_cbase, bool small,
                   const unsigned long long* dn = nullptr) {
     if (!small) scan_launch(in, n);
+    dev_work = true;
     LevelBuf& out = lv[L];
     uint64_t row_cap = ~0ull;
     const bool want_parent = (chain && !chain_fused && mode == M_WRITE && L == k - 3) ||
@@ -3336,21 +3365,24 @@ struct Matcher {
     uint64_t* pub_dev = c.host_res_dev + 32 + 2 * L;
     volatile uint64_t* pub = c.host_res + 32 + 2 * L;
     if (mode == M_WRITE) pub[0] = ~0ull;
-    // a level whose input size is on the device cannot be redone here: a
-    // misfit goes to the end-of-run status word and repeats the run
-    unsigned long long* st_word = (mode == M_WRITE && !dn) ? ctr + 11 : ctr + 12;
+    // the last complete run's size of this level fits one planning block:
+    // the next level takes it from the device, with no synchronisation
+    const bool chain_next = mode == M_WRITE && hint && hint[L] > 0 && hint[L] <= (uint64_t)SCAN_TILE && chainable(L + 1);
+    // a level whose input or output size stays on the device cannot be redone
+    // here: a misfit goes to the end-of-run status word and repeats the run
+    unsigned long long* st_word = (mode == M_WRITE && !dn && !chain_next) ? ctr + 11 : ctr + 12;
     uint64_t tmax;
     if (small) {
       // plan + scan + tile index in one launch
       ensure_tiles(arena, in, std::max<uint64_t>(in.tile_cap, 4097) - 1);
       tmax = in.tile_cap - 1;
       unsigned int* oc = mode == M_WRITE ? (unsigned int*)(ctr + 10) : nullptr;
-#define PSM(LL) hipLaunchKernelGGL((k_plan_small<LL>), dim3(1), dim3(BLOCK), 0, c.stream, g, kp, rows, n, in.minlen, in.minsel, use_cbase ? in.cbase : nullptr, tbl, mode == M_PAIR ? in.pbase : nullptr, ptbl, ctr, in.work_off, oc ? MAX_CHUNK : MAX_SPEC_ITEMS, in.tile_cap, row_cap, in.tile_p, (unsigned int*)(ctr + kTile0), oc, ctr + 14, st_word, ctr + 13, oc ? pub_dev : nullptr, dn, dn ? c.lvcnt + (L - 1) : nullptr)
+#define PSM(LL) hipLaunchKernelGGL((k_plan_small<LL>), dim3(1), dim3(BLOCK), 0, c.stream, g, kp, rows, n, in.minlen, in.minsel, use_cbase ? in.cbase : nullptr, tbl, mode == M_PAIR ? in.pbase : nullptr, ptbl, ctr, in.work_off, oc ? MAX_CHUNK : MAX_SPEC_ITEMS, in.tile_cap, row_cap, in.tile_p, (unsigned int*)(ctr + kTile0), oc, ctr + 14, st_word, ctr + 13, work_left(), oc ? pub_dev : nullptr, dn, dn ? c.lvcnt + (L - 1) : nullptr)
       CUTS_DISPATCH_L(L, PSM)
 #undef PSM
       HIPCHECK(hipGetLastError());
     } else {
-      tmax = tile_index_dyn(in, n, row_cap, mode == M_WRITE ? (unsigned int*)(ctr + 10) : nullptr,
+      tmax = tile_index_dyn(in, n, row_cap, mode == M_WRITE ? (unsigned int*)(ctr + 10) : nullptr, st_word,
                             mode == M_WRITE ? pub_dev : nullptr);
     }
     ExpandArgs a{};
@@ -3390,9 +3422,7 @@ struct Matcher {
       CUTS_DISPATCH_L(L, EW)
 #undef EW
       HIPCHECK(hipGetLastError());
-      // the last complete run's size of this level fits one planning block:
-      // the next level takes it from the device, with no synchronisation
-      if (hint && hint[L] > 0 && hint[L] <= (uint64_t)SCAN_TILE && chainable(L + 1)) {
+      if (chain_next) {
         chained_mask |= 1u << L;
         level(L + 1, out.rows, SCAN_TILE, ctr + 10);
         return true;
@@ -3409,9 +3439,15 @@ struct Matcher {
       const uint64_t m = got[0] & 0xFFFFFFFFu;
       // a level whose input size was on the device and that did not fit:
       // the end-of-run word repeats the run
-      if (dn && (got[1] & 1ull)) return true;
-      if (got[1] & 1ull) {
+      if (dn && (got[1] & 3ull)) return true;
+      if (got[1] & 3ull) {
         HIPCHECK(hipMemsetAsync(ctr + 11, 0, 8, c.stream));
+        if (o.max_work) {
+          // the readback's test of the cap counts the levels before this one
+          r.work += read_u64(ctr + 13);
+          dev_work = false;
+          HIPCHECK(hipMemsetAsync(ctr + 13, 0, 8, c.stream));
+        }
         r.chunks--;
         return false;
       }
@@ -3521,8 +3557,9 @@ struct Matcher {
                    bool spec = false) {
     if (spec) {
       // the pair level's second pass without the readback of its work
+      common_spec = dev_work = true;
       scan_launch(in, n);
-      const uint64_t tmax = tile_index_dyn(in, n, ~0ull, nullptr);
+      const uint64_t tmax = tile_index_dyn(in, n, ~0ull, nullptr, ctr + 12);
       ExpandArgs a{};
       a.rows = rows;
       a.work_off = in.work_off;
@@ -3954,8 +3991,14 @@ struct Matcher {
         r.last_root = (uint32_t)(hp[14] & 0xFFFFFFFFu);
         last_root_read = true;
       }
-      spec_overflow = (hp[12] & 1ull) != 0;
+      const bool host_work = r.work != 0;
       r.work += hp[13];
+      // a run stopped by its work cap at its last, counting level: one path
+      // down the levels, all of it counted on the device
+      const bool capped_at_end = hp[12] == 2ull && !host_work && !common_spec && !chained_mask && o.trunks <= 1;
+      spec_overflow = hp[12] != 0 && !capped_at_end;
+      if (o.max_work && r.work > o.max_work && speculate() && !capped_at_end && !(cap_exact && !chained_mask))
+        spec_overflow = true;
       // sizes of the levels whose successor read them on the device (level
       // 0's: every root processed in one trunk)
       for (uint32_t l = 0; l < k; ++l)
@@ -3978,6 +4021,15 @@ struct Matcher {
         } else if (fuse) {
           r.level[k - 2] = hp[1];
         }
+      }
+      if (capped_at_end) {
+        aborted = true;
+        r.work_capped = 1;
+        r.complete = 0;
+        r.roots_done = 0;
+        r.last_root = 0;
+        r.chunks--;
+        for (uint32_t l = 1; l < k; ++l) r.level[l] = 0;
       }
       if (r.work_capped) r.count = 0;
     }
