@@ -1396,7 +1396,7 @@ __global__ __launch_bounds__(BLOCK, L <= 4 ? 5 : L <= 5 ? 4 : 1) void k_expand(G
   // (a directed last level of 1.3e10 items: 111 -> 56.8 ms).  Tiles
   // of more prefixes (short lists) keep the offsets alone, or nothing.
   constexpr uint32_t SP = 256, NJP = 3;
-  constexpr uint32_t STAGE_WORDS = (SP + 1) + (L + 3 + NJP) * SP;
+  constexpr uint32_t STAGE_WORDS = (SP + 1) + (L + 3 + NJP + (MODE == M_FUSED ? 1 : 0)) * SP;
   constexpr uint32_t RAW_WORDS = STAGE_WORDS > 2 * (LDS_OFF + 1) ? STAGE_WORDS : 2 * (LDS_OFF + 1);
   __shared__ __align__(8) uint32_t s_raw[RAW_WORDS];
   uint64_t* const s_off = (uint64_t*)s_raw;
@@ -1406,6 +1406,7 @@ __global__ __launch_bounds__(BLOCK, L <= 4 ? 5 : L <= 5 ? 4 : 1) void k_expand(G
   uint32_t* const s_meta = s_li + SP;            // SP: constraint index | jc << 8
   uint32_t* const s_cb = s_meta + SP;            // SP
   int32_t* const s_hub = (int32_t*)(s_cb + SP);  // NJP x SP
+  int32_t* const s_sch = s_hub + NJP * SP;       // SP (fused): hub row of the closed form's vertex
   __shared__ uint32_t s_pos[NJP];                // owner positions of the first constraints
   if (threadIdx.x < NJP) s_pos[threadIdx.x] = P.jc[L][threadIdx.x] & 31u;  // before the tile loop's first barrier
   __shared__ uint32_t s_w[BLOCK / 64], s_pre[BLOCK / 64], s_base;
@@ -1423,7 +1424,11 @@ __global__ __launch_bounds__(BLOCK, L <= 4 ? 5 : L <= 5 ? 4 : 1) void k_expand(G
   const uint32_t tin = P.sig_in[L], tout = P.sig_out[L];
   // a last level that is counted entry by entry reads no signatures where its
   // constraints imply them (always, short of query self-loops)
-  const bool need_sig = MODE != M_COUNT || !((P.sig_implied >> L) & 1);
+  // (nor does a fused level whose closed form asks for no degree: with the
+  // closed form's hub row staged per prefix, 5-cycle + chord + 2 tails on
+  // R-MAT 20 219 -> 189 ms)
+  const bool need_sig = !((P.sig_implied >> L) & 1) ||
+                        (MODE != M_COUNT && !(MODE == M_FUSED && a.cbase && P.sc_thr <= 1 && !a.stats));
   // all constraints on lists of one direction (every symmetric graph's): their
   // tables are the same for all lanes
   bool onedir = true;
@@ -1500,7 +1505,14 @@ __global__ __launch_bounds__(BLOCK, L <= 4 ? 5 : L <= 5 ? 4 : 1) void k_expand(G
         s_rel[i] = o <= w0 ? 0u : (uint32_t)(o - w0);  // below TILE but for empty prefixes at the end
         s_li[i] = ((jcv >> 7) ? g.off_in : g.off_out)[u] - (uint32_t)(o - w0);
         s_meta[i] = sl | jcv << 8;
-        if (MODE == M_FUSED) s_cb[i] = a.cbase ? a.cbase[p] : 0u;
+        if (MODE == M_FUSED) {
+          s_cb[i] = a.cbase ? a.cbase[p] : 0u;
+          uint32_t us = 0;
+#pragma unroll
+          for (int l = 0; l < L; ++l)
+            if (l == (int)P.sc_pos) us = r[l];
+          s_sch[i] = g.hub_id ? g.hub_id[us] : -1;
+        }
 #pragma unroll
         for (int cc = 0; cc < (int)NJP; ++cc) {
           const uint32_t jcc = cc < (int)nj ? P.jc[L][cc] : 0u;
@@ -1926,10 +1938,10 @@ __global__ __launch_bounds__(BLOCK, L <= 4 ? 5 : L <= 5 ? 4 : 1) void k_expand(G
 #pragma unroll
             for (int l = 0; l < L; ++l)
               if (l == (int)P.sc_pos) us[j] = row[j][l];
-            h[j] = g.hub_id ? g.hub_id[us[j]] : -1;
+            h[j] = staged ? s_sch[pi[j]] : g.hub_id ? g.hub_id[us[j]] : -1;
           }
 #pragma unroll
-          for (int j = 0; j < G; ++j) bw[j] = h[j] >= 0 ? g.bits[(uint64_t)h[j] * g.words + (v[j] >> 6)] : 0;
+          for (int j = 0; j < G; ++j) bw[j] = (ok[j] && h[j] >= 0) ? g.bits[(uint64_t)h[j] * g.words + (v[j] >> 6)] : 0;
           // the other survivors' searches of v in N(u), in lock-step
           uint32_t sb[G], sn[G];
           bool fnd[G];
