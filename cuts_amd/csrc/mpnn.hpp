@@ -1,6 +1,8 @@
 // Table-size predictor (message-passing network): device state shared by
 // mpnn.hip and the C ABI.  Not part of the public ABI.
 #pragma once
+#include <algorithm>
+
 #include "device.hpp"
 
 namespace cuts {
@@ -21,12 +23,18 @@ struct Mpnn {
   uint32_t step = 0;
   // staging for one batch of samples
   uint32_t cap = 0;
-  float* x = nullptr;
+  float* stage = nullptr;   // pinned, what the live rows are packed into
+  uint64_t staged = 0;      // its bytes
+  float* x = nullptr;       // live rows of the samples, one after the other
+  uint32_t* row = nullptr;  // first row of every sample
   uint16_t* adj = nullptr;
   uint32_t* meta = nullptr;
   float *t = nullptr, *y = nullptr;
   ~Mpnn();
 };
+
+// The live rows of samples first .. last-1 (row: their first rows) to out.
+void pack_rows(const float* x, const uint32_t* meta, const uint32_t* row, uint32_t first, uint32_t last, float* out);
 
 void mpnn_init(Context& c, Mpnn& n, const float* params);
 void mpnn_set(Mpnn& n, const float* params);
