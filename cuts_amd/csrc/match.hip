@@ -1383,8 +1383,9 @@ __device__ __forceinline__ uint64_t next_tile(unsigned int* tilectr, uint64_t nt
 }
 
 // Five waves per SIMD for rows of up to 4 words (96 registers), four for 5:
-// the R-MAT 20 tail query took 6.0 / 5.0 / 4.5 / 4.5 ms at three to six, the
-// directed last level 79.8 / 79.6 / 68.1 / 70.8.
+// the R-MAT 20 5-cycle + chord + 2 tails query, counted from whole prefixes,
+// took 6.0 / 5.0 / 4.5 / 4.5 ms at three to six, the directed last level
+// 79.8 / 79.6 / 68.1 / 70.8.
 template <int L, int MODE>
 __global__ __launch_bounds__(BLOCK, L <= 4 ? 5 : L <= 5 ? 4 : 1) void k_expand(GView g, KPlan P, ExpandArgs a) {
   // A tile of at most SP prefixes stages them in LDS, one thread per prefix:
@@ -2988,11 +2989,16 @@ struct Matcher {
   }
   // deterministic work cap: the candidates examined so far
   bool add_work(uint64_t w) {
+    if (o.max_work && dev_work) {
+      // the cap counts the levels before this one
+      r.work += read_u64(ctr + 13);
+      HIPCHECK(hipMemsetAsync(ctr + 13, 0, 8, c.stream));
+      dev_work = false;
+    }
     r.work += w;
     if (o.max_work && r.work > o.max_work) {
       aborted = true;
       r.work_capped = 1;
-      cap_exact = !dev_work;
     }
     return aborted;
   }
@@ -3065,18 +3071,18 @@ struct Matcher {
   // status bit for the end of the run, which then repeats the whole query
   // with readbacks.  Off for profiling, deadlines, the no-allocation entry
   // point and CUTS_FLAG_SYNC_LEVELS.
-  // A work cap is tested on the device too (claim_work), against the cap less
-  // the work counted on the host, so a level beyond it is never expanded: a
-  // writing level is then run with the readback, which decides as it does
-  // without speculation; a counting level ends the run where it is the run's
-  // only branch (capped_at_end), and otherwise the run is repeated with
-  // readbacks.  A capped run that stays below its cap thus has the launches
-  // and readbacks of one without: a 6-vertex query of 4.1 M candidates on
-  // R-MAT 20, more than 0.185 ms with its levels read back, takes 0.129.
+  // A work cap is tested on the device too (claim_work), so a level beyond it
+  // is never expanded: a writing level is then run with the readback, which
+  // decides as it does without speculation, and so are all levels after one
+  // that the host counted; a counting level ends the run (capped_at_end), or
+  // repeats it with readbacks where other work may have followed.  A capped
+  // run that stays below its cap thus has the launches and readbacks of one
+  // without: a 6-vertex query of 4.1 M candidates on R-MAT 20, more than
+  // 0.185 ms with its levels read back, takes 0.142; 598 runs of an admission
+  // that end at their cap take 663 ms for 653.
   bool no_spec = false;
   bool spec_overflow = false;
   bool dev_work = false;     // candidates counted on the device and not yet in r.work
-  bool cap_exact = false;    // the cap was passed with all work counted
   bool common_spec = false;  // a speculative pass over stored rows' intersections was planned
   uint64_t work_left() const { return o.max_work ? o.max_work - std::min(o.max_work, r.work) : ~0ull; }
   // level sizes of the last complete run of this query, or null; bit l:
@@ -3099,7 +3105,7 @@ struct Matcher {
     return true;
   }
   bool speculate() const {
-    return !no_spec && !prof && !has_deadline && !arena && !(o.flags & 8192u);
+    return !no_spec && !prof && !has_deadline && !arena && !(o.flags & 8192u) && !(o.max_work && r.work);
   }
   // Word w of the coherent host words once the stream has drained: true
   // when a kernel published it (it holds ~0 until then).  Polling the word
@@ -3197,8 +3203,8 @@ struct Matcher {
       if (merge) r.merge_bytes[mclass] += (double)read_u64(merge);
     }
     if (spec && level_spec(L, rows, n, in, mode, use_cbase, small, dn)) return;
-    // (a small level that did not fit has been planned: the scan below reads it)
-    const uint64_t W = scan(in, n);
+    // (a level that did not fit has been planned and scanned)
+    const uint64_t W = spec ? read_u64(in.work_off + n) : scan(in, n);
     if (W == 0) return;
     if (add_work(W)) return;
     // a counting level sizes the tile index for all of W, so that its next
@@ -3462,12 +3468,6 @@ struct Matcher {
       if (dn && (got[1] & 3ull)) return true;
       if (got[1] & 3ull) {
         HIPCHECK(hipMemsetAsync(ctr + 11, 0, 8, c.stream));
-        if (o.max_work) {
-          // the readback's test of the cap counts the levels before this one
-          r.work += read_u64(ctr + 13);
-          dev_work = false;
-          HIPCHECK(hipMemsetAsync(ctr + 13, 0, 8, c.stream));
-        }
         r.chunks--;
         return false;
       }
@@ -4018,8 +4018,7 @@ struct Matcher {
       // down the levels, all of it counted on the device
       const bool capped_at_end = hp[12] == 2ull && !host_work && !common_spec && !chained_mask && o.trunks <= 1;
       spec_overflow = hp[12] != 0 && !capped_at_end;
-      if (o.max_work && r.work > o.max_work && speculate() && !capped_at_end && !(cap_exact && !chained_mask))
-        spec_overflow = true;
+      if (r.work_capped && chained_mask) spec_overflow = true;
       // sizes of the levels whose successor read them on the device (level
       // 0's: every root processed in one trunk)
       for (uint32_t l = 0; l < k; ++l)
