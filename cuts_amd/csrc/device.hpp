@@ -237,7 +237,7 @@ struct Context {
   // a writing level of at most one planning block's rows in that run hands
   // its size to the next level on the device
   unsigned long long* lvcnt = nullptr;
-  std::unordered_map<std::string, std::array<uint64_t, kMaxQuery>> level_hints;
+  std::unordered_map<std::string, std::array<uint64_t, kMaxQuery + 1>> level_hints;  // sizes; work
   char* scratch = nullptr;                // this device's no-allocation scratch array
   bool counted = false;                   // known to the device's pool (pool_context)
   ~Context();

@@ -918,12 +918,13 @@ static __global__ __launch_bounds__(BLOCK) void k_tile_index(const uint64_t* __r
   }
 }
 
-// A writing level's rows written and status, to coherent host memory
-// (system-scope stores; the row count last, with release order), for a host
-// that polls the count word instead of synchronising with the stream.
-__device__ __forceinline__ void publish_rows(uint64_t* publish, uint32_t rows, unsigned long long status) {
+// A writing level's rows written (or, of a level withheld, the work of the
+// levels before it) and status, to coherent host memory (system-scope stores;
+// the count last, with release order), for a host that polls the count word
+// instead of synchronising with the stream.
+__device__ __forceinline__ void publish_rows(uint64_t* publish, uint64_t rows, unsigned long long status) {
   __hip_atomic_store(&publish[1], (uint64_t)status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-  __hip_atomic_store(&publish[0], (uint64_t)rows, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+  __hip_atomic_store(&publish[0], rows, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // One thread: the tiles of a speculative level handed to its expansion, or
@@ -932,16 +933,23 @@ __device__ __forceinline__ void publish_rows(uint64_t* publish, uint32_t rows, u
 // less what the host has counted).  Only this thread looks at *work, which it
 // alone changes: the other threads may index tiles that nothing then takes.
 // The work of a counting level beyond the cap is added all the same, as the
-// readback does; a writing level is run again with the readback.
+// readback does, and that of the counting levels after it is not: the run has
+// ended there.  publish (a writing level): a level without tiles has no
+// expansion block to publish its size; one withheld tells the host its work
+// (from bit 2 of the status word) and that of the levels before it (in place
+// of the rows), so that no readback follows.
 static __device__ __forceinline__ bool claim_work(bool fits, uint64_t W, uint64_t nt, unsigned long long* dyn,
                                            unsigned long long* status, unsigned long long* work, uint64_t work_cap,
-                                           bool writes) {
-  const bool over = W > work_cap || *work > work_cap - W;
+                                           uint64_t* publish) {
+  const unsigned long long before = *work;
+  const bool over = W > work_cap || before > work_cap - W;
   const bool go = fits && !over;
   dyn[0] = go ? W : 0ull;
   dyn[1] = go ? nt : 0ull;
-  if (go || (over && !writes)) *work += W;
+  if (go || (over && !publish && !(*status & 2ull))) *work = before + W;
   if (!go) *status |= over ? 2ull : 1ull;
+  if (publish && !go) publish_rows(publish, before, (over ? 2ull : 1ull) | W << 2);
+  else if (publish && W == 0) publish_rows(publish, 0u, 0ull);
   return go;
 }
 
@@ -968,9 +976,7 @@ static __global__ __launch_bounds__(BLOCK) void k_tile_index_dyn(const uint64_t*
     if (threadIdx.x < 8) tilectr[threadIdx.x * kTileStride] = 0u;
     if (outctr && threadIdx.x < 2) outctr[threadIdx.x] = 0u;
     if (threadIdx.x == 0) {
-      const bool go = claim_work(fits, W, nt, dyn, status, work, work_cap, publish != nullptr);
-      // a writing level with no tiles: no expansion block will publish
-      if (publish && (!go || W == 0)) publish_rows(publish, 0u, go ? 0ull : 1ull);
+      claim_work(fits, W, nt, dyn, status, work, work_cap, publish);
     }
   }
   if (!fits || W == 0) return;
@@ -1067,8 +1073,7 @@ __global__ __launch_bounds__(BLOCK) void k_plan_small(GView g, KPlan P, const ui
   if (threadIdx.x < 8) tilectr[threadIdx.x * kTileStride] = 0u;
   if (outctr && threadIdx.x < 2) outctr[threadIdx.x] = 0u;
   if (threadIdx.x == 0) {
-    const bool go = claim_work(fits, W, nt, dyn, status, work, work_cap, publish != nullptr);
-    if (publish && (!go || W == 0)) publish_rows(publish, 0u, go ? 0ull : 1ull);
+    claim_work(fits, W, nt, dyn, status, work, work_cap, publish);
   }
   __syncthreads();
   if (!fits || W == 0) return;
@@ -2991,8 +2996,10 @@ struct Matcher {
   bool add_work(uint64_t w) {
     if (o.max_work && dev_work) {
       // the cap counts the levels before this one
-      r.work += read_u64(ctr + 13);
-      HIPCHECK(hipMemsetAsync(ctr + 13, 0, 8, c.stream));
+      const uint64_t d = dev_before != ~0ull ? dev_before : read_u64(ctr + 13);
+      r.work += d - dev_taken;
+      dev_taken = d;
+      dev_before = ~0ull;
       dev_work = false;
     }
     r.work += w;
@@ -3072,18 +3079,17 @@ struct Matcher {
   // with readbacks.  Off for profiling, deadlines, the no-allocation entry
   // point and CUTS_FLAG_SYNC_LEVELS.
   // A work cap is tested on the device too (claim_work), so a level beyond it
-  // is never expanded: a writing level is then run with the readback, which
-  // decides as it does without speculation, and so are all levels after one
-  // that the host counted; a counting level ends the run (capped_at_end), or
-  // repeats it with readbacks where other work may have followed.  A capped
-  // run that stays below its cap thus has the launches and readbacks of one
-  // without: a 6-vertex query of 4.1 M candidates on R-MAT 20, more than
-  // 0.185 ms with its levels read back, takes 0.142; 598 runs of an admission
-  // that end at their cap take 663 ms for 653.
+  // is never expanded: a writing level tells the host, which ends the run
+  // there; a counting level ends it too (capped_at_end).  All levels after one
+  // that the host counted are read back, and so are all of a run of several
+  // trunks.  A capped run that stays below its cap thus has the launches and
+  // readbacks of one without: a 6-vertex query of 4.1 M candidates on R-MAT
+  // 20, more than 0.185 ms with its levels read back, takes 0.142.
   bool no_spec = false;
   bool spec_overflow = false;
-  bool dev_work = false;     // candidates counted on the device and not yet in r.work
-  bool common_spec = false;  // a speculative pass over stored rows' intersections was planned
+  bool dev_work = false;        // candidates counted on the device and not yet in r.work
+  uint64_t dev_taken = 0;       // of the device's count, what r.work holds
+  uint64_t dev_before = ~0ull;  // the device's count before the level being read back, where it told
   uint64_t work_left() const { return o.max_work ? o.max_work - std::min(o.max_work, r.work) : ~0ull; }
   // level sizes of the last complete run of this query, or null; bit l:
   // level l's size was handed on on the device (read from lvcnt at the end)
@@ -3105,7 +3111,8 @@ struct Matcher {
     return true;
   }
   bool speculate() const {
-    return !no_spec && !prof && !has_deadline && !arena && !(o.flags & 8192u) && !(o.max_work && r.work);
+    return !no_spec && !prof && !has_deadline && !arena && !(o.flags & 8192u) &&
+           !(o.max_work && (r.work || o.trunks > 1));
   }
   // Word w of the coherent host words once the stream has drained: true
   // when a kernel published it (it holds ~0 until then).  Polling the word
@@ -3202,9 +3209,10 @@ struct Matcher {
       // the prefixes' list reads belong to the expansion that performs them
       if (merge) r.merge_bytes[mclass] += (double)read_u64(merge);
     }
-    if (spec && level_spec(L, rows, n, in, mode, use_cbase, small, dn)) return;
+    uint64_t spec_W = ~0ull;  // work of a level that did not fit, where the device told
+    if (spec && level_spec(L, rows, n, in, mode, use_cbase, small, spec_W, dn)) return;
     // (a level that did not fit has been planned and scanned)
-    const uint64_t W = spec ? read_u64(in.work_off + n) : scan(in, n);
+    const uint64_t W = !spec ? scan(in, n) : spec_W != ~0ull ? spec_W : read_u64(in.work_off + n);
     if (W == 0) return;
     if (add_work(W)) return;
     // a counting level sizes the tile index for all of W, so that its next
@@ -3358,10 +3366,11 @@ struct Matcher {
   }
 
   // One level without the readback of its work (see speculate()).  Returns
-  // false when a writing level did not fit: the caller then runs it with the
-  // readback (its scan is repeated; nothing was written or counted).
+  // false when a writing level did not fit: the caller then runs it in chunks
+  // (it has been planned and scanned, its work goes to W; nothing was written
+  // or counted).
   bool level_spec(uint32_t L, const uint32_t* rows, uint64_t n, LevelBuf& in, int mode, bool use_cbase, bool small,
-                  const unsigned long long* dn = nullptr) {
+                  uint64_t& W, const unsigned long long* dn = nullptr) {
     if (!small) scan_launch(in, n);
     dev_work = true;
     LevelBuf& out = lv[L];
@@ -3467,8 +3476,17 @@ struct Matcher {
       // the end-of-run word repeats the run
       if (dn && (got[1] & 3ull)) return true;
       if (got[1] & 3ull) {
-        HIPCHECK(hipMemsetAsync(ctr + 11, 0, 8, c.stream));
         r.chunks--;
+        W = got[1] >> 2;
+        if (got[1] & 2ull) {
+          // the work cap: the run ends as add_work ends it
+          r.work += W;
+          r.work_capped = 1;
+          aborted = true;
+          return true;
+        }
+        dev_before = got[0];
+        HIPCHECK(hipMemsetAsync(ctr + 11, 0, 8, c.stream));
         return false;
       }
       r.level[L] += m;
@@ -3577,7 +3595,7 @@ struct Matcher {
                    bool spec = false) {
     if (spec) {
       // the pair level's second pass without the readback of its work
-      common_spec = dev_work = true;
+      dev_work = true;
       scan_launch(in, n);
       const uint64_t tmax = tile_index_dyn(in, n, ~0ull, nullptr, ctr + 12);
       ExpandArgs a{};
@@ -3911,6 +3929,9 @@ struct Matcher {
     if (!arena) {
       const auto it = c.level_hints.find(hint_key);
       hint = it == c.level_hints.end() ? nullptr : it->second.data();
+      // levels that a work cap is known to end are not handed on on the
+      // device, where the host would not see which of them ended the run
+      if (hint && o.max_work && hint[kMaxQuery] > o.max_work) hint = nullptr;
     }
     // level 0
     const uint32_t rb = o.root_stride ? o.root_begin : 0;
@@ -3981,16 +4002,12 @@ struct Matcher {
         }
         level(1, l0.rows + s, std::min(ts, n0 - s), (chained_mask & 1u) ? ctr + 10 : nullptr);
         if (aborted) {
-          // words 0..2 and the slots (a work cap has no snapshot: its count is void)
+          // words 0..2 and the slots (a work cap has no snapshot: its counts are void)
           if (has_deadline) {
             HIPCHECK(hipMemcpyAsync(ctr, ctr + kCounterWords, 24, hipMemcpyDeviceToDevice, c.stream));
             HIPCHECK(hipMemcpyAsync(ctr + kSlot0, ctr + kCounterWords + kSlot0, (kTile0 - kSlot0) * 8,
                                     hipMemcpyDeviceToDevice, c.stream));
-          } else {
-            HIPCHECK(hipMemsetAsync(ctr, 0, 24, c.stream));
-            HIPCHECK(hipMemsetAsync(ctr + kSlot0, 0, (kTile0 - kSlot0) * 8, c.stream));
           }
-          HIPCHECK(hipStreamSynchronize(c.stream));
           std::memcpy(r.level, snap_level, sizeof(snap_level));
           break;
         }
@@ -4013,10 +4030,11 @@ struct Matcher {
         last_root_read = true;
       }
       const bool host_work = r.work != 0;
-      r.work += hp[13];
-      // a run stopped by its work cap at its last, counting level: one path
-      // down the levels, all of it counted on the device
-      const bool capped_at_end = hp[12] == 2ull && !host_work && !common_spec && !chained_mask && o.trunks <= 1;
+      r.work += hp[13] - dev_taken;
+      const bool void_counts = aborted && !has_deadline;  // ended by the work cap on the host
+      // a run stopped by its work cap at a counting level: one path down the
+      // levels, all of it counted on the device
+      const bool capped_at_end = hp[12] == 2ull && !host_work && !chained_mask && o.trunks <= 1;
       spec_overflow = hp[12] != 0 && !capped_at_end;
       if (r.work_capped && chained_mask) spec_overflow = true;
       // sizes of the levels whose successor read them on the device (level
@@ -4029,17 +4047,18 @@ struct Matcher {
         if (last_root_read) r.last_root = (uint32_t)(hp[14] & 0xFFFFFFFFu);
       }
       if (!write) {
-        r.count = hp[0];
+        auto sum = [&](int i) { return void_counts ? 0ull : hp[i]; };
+        r.count = sum(0);
         r.level[k - 1] = r.count;
         if (collapse_fused) {
-          r.level[k - 4] = hp[1];
-          r.level[k - 3] = hp[2];
-          r.level[k - 2] = hp[9];
+          r.level[k - 4] = sum(1);
+          r.level[k - 3] = sum(2);
+          r.level[k - 2] = sum(9);
         } else if (pair || chain_fused || tail_fused) {
-          r.level[k - 3] = hp[1];
-          r.level[k - 2] = hp[2];
+          r.level[k - 3] = sum(1);
+          r.level[k - 2] = sum(2);
         } else if (fuse) {
-          r.level[k - 2] = hp[1];
+          r.level[k - 2] = sum(1);
         }
       }
       if (capped_at_end) {
@@ -4074,8 +4093,9 @@ struct Matcher {
       // at most 2^16 queries remembered (about 10 MB); past that the
       // table starts over
       if (c.level_hints.size() >= (1u << 16) && !c.level_hints.count(hint_key)) c.level_hints.clear();
-      std::array<uint64_t, kMaxQuery> sizes{};
+      std::array<uint64_t, kMaxQuery + 1> sizes{};
       for (uint32_t l = 0; l < k; ++l) sizes[l] = r.level[l];
+      sizes[kMaxQuery] = r.work;
       c.level_hints[hint_key] = sizes;
     }
   }
