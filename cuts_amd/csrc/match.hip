@@ -3216,8 +3216,9 @@ struct Matcher {
     if (W == 0) return;
     if (add_work(W)) return;
     // a counting level sizes the tile index for all of W, so that its next
-    // speculative run fits in one launch
-    if (mode != M_WRITE && W <= MAX_SPEC_ITEMS) ensure_tiles(arena, in, (W + TILE - 1) / TILE);
+    // speculative run fits in one launch (a scratch run never speculates: its
+    // index holds one chunk, at most 16 MB where 2^35 items' takes 256)
+    if (mode != M_WRITE && !arena && W <= MAX_SPEC_ITEMS) ensure_tiles(arena, in, (W + TILE - 1) / TILE);
     uint64_t chunk = MAX_CHUNK;
     LevelBuf& out = lv[L];
     if (mode == M_WRITE) {
@@ -3618,7 +3619,7 @@ struct Matcher {
     }
     const uint64_t W = scan(in, n);
     if (W == 0 || add_work(W)) return;
-    if (W <= MAX_SPEC_ITEMS) ensure_tiles(arena, in, (W + TILE - 1) / TILE);
+    if (!arena && W <= MAX_SPEC_ITEMS) ensure_tiles(arena, in, (W + TILE - 1) / TILE);
     for (uint64_t w0 = 0; w0 < W; w0 += MAX_CHUNK) {
       if (past_deadline()) return;
       const uint64_t w1 = std::min(W, w0 + MAX_CHUNK);
