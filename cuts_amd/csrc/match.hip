@@ -2988,6 +2988,14 @@ struct Matcher {
   // held to a tenth of the score order's time there
   // (tests/test_learned.py, training on R-MAT 18 and judging on R-MAT 20)
   bool tail_left() const { return kp.tl_kind == 1 && kp.pr_a != kp.pr_b && !g.h2_off && g.arc_cn && kp.pr_adj; }
+  // the tables of the whole-prefix tail are none or with the graph already
+  bool tail_tables_held() const {
+    std::lock_guard<std::recursive_mutex> lk(dg.tables_mu);
+    auto held = [&](uint32_t t) { return t <= 1 || dg.cnt_tables.count(t) != 0; };
+    if (kp.tl_kind == 3)
+      return held(kp.ch_ta) && held(kp.ch_tb) && dg.chain_tables.count(std::make_pair(kp.ch_ta, kp.ch_tb)) != 0;
+    return held(kp.pr_ta) && held(kp.pr_tb) && (kp.pr_a != kp.pr_b || held(kp.pr_tab));
+  }
   bool past_deadline() {
     if (has_deadline && !aborted && std::chrono::steady_clock::now() >= deadline) aborted = true;
     return aborted;
@@ -3875,6 +3883,14 @@ struct Matcher {
            (kp.tl_kind == 3 ? !(o.flags & 256u)
                             : !(o.flags & 128u) && !tail_left() &&
                                   (kp.tl_kind == 1 || (kp.tl_kind == 2 && tail_known())));
+    const uint32_t rb = o.root_stride ? o.root_begin : 0;
+    const uint32_t re = o.root_stride ? std::min(o.root_end, dg.V) : dg.V;
+    const uint32_t rs = o.root_stride ? o.root_stride : 1;
+    const uint32_t n0c = re > rb ? (re - rb + rs - 1) / rs : 0;
+    // a scratch run builds the tables that the graph does not hold on every
+    // call, each a pass over all lists: not for a few roots (path of 4 from
+    // one root, R-MAT 20: 0.12 ms, 1.5 with the tables)
+    if (tail && arena && (uint64_t)n0c * 16 < dg.V && !tail_tables_held()) tail = false;
     tail_fused = tail && tail_known() && k >= 4;
     // 6 blocks of 4 waves per CU: measured best on the power-law workloads
     // (the tiles are taken dynamically, so the grid only sets residency)
@@ -3935,10 +3951,6 @@ struct Matcher {
       if (hint && o.max_work && hint[kMaxQuery] > o.max_work) hint = nullptr;
     }
     // level 0
-    const uint32_t rb = o.root_stride ? o.root_begin : 0;
-    const uint32_t re = o.root_stride ? std::min(o.root_end, dg.V) : dg.V;
-    const uint32_t rs = o.root_stride ? o.root_stride : 1;
-    const uint32_t n0c = re > rb ? (re - rb + rs - 1) / rs : 0;
     LevelBuf& l0 = lv[0];
     ensure_rows(arena, l0, std::max<uint32_t>(n0c, 1), 1);
     // counts, tile counters, merge bytes, level counts, rows written,
