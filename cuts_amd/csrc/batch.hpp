@@ -111,7 +111,8 @@ const uint32_t* cnt_table(Context& c, DeviceGraph& dg, uint32_t thr);
 const uint64_t* chain_table(Context& c, DeviceGraph& dg, uint32_t ta, uint32_t tb);
 // The same, built in `arena` for one call (not cached) when the graph has
 // not cached them and arena is non-null.
-const uint32_t* cnt_table(Context& c, DeviceGraph& dg, ScratchArena* arena, uint32_t thr);
-const uint64_t* chain_table(Context& c, DeviceGraph& dg, ScratchArena* arena, uint32_t ta, uint32_t tb);
+const uint32_t* cnt_table(Context& c, DeviceGraph& dg, ScratchArena* arena, uint32_t thr, bool* built = nullptr);
+const uint64_t* chain_table(Context& c, DeviceGraph& dg, ScratchArena* arena, uint32_t ta, uint32_t tb,
+                            bool* built = nullptr);
 
 }  // namespace cuts

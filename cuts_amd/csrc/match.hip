@@ -1220,14 +1220,16 @@ __global__ __launch_bounds__(BLOCK) void k_closed_form(GView g, KPlan P, const u
   }
 }
 
-// Degree-threshold table: tbl[u] = |{x in N(u) : deg(x) >= thr}|, one wave per vertex.
+// Degree-threshold table: tbl[u] = |{x in N(u) : deg(x) >= thr}|, one wave per
+// vertex.  Degrees from the list entries' signatures (of a symmetric graph),
+// read in order.
 static __global__ __launch_bounds__(BLOCK) void k_cnt_table(GView g, uint32_t thr, uint32_t* __restrict__ tbl) {
   const uint32_t lane = threadIdx.x & 63;
   const uint64_t nw = (uint64_t)gridDim.x * (BLOCK / 64);
   for (uint64_t u = (uint64_t)blockIdx.x * (BLOCK / 64) + (threadIdx.x >> 6); u < g.V; u += nw) {
     const uint32_t lo = g.off_out[u], hi = g.off_out[u + 1];
     uint32_t c = 0;
-    for (uint32_t i = lo + lane; i < hi; i += 64) c += g.sig[2 * (uint64_t)g.adj_out[i]] >= thr;
+    for (uint32_t i = lo + lane; i < hi; i += 64) c += g.nsig_out[i].x >= thr;
     for (int o = 32; o > 0; o >>= 1) c += __shfl_xor(c, o);
     if (lane == 0) tbl[u] = c;
   }
@@ -2672,7 +2674,7 @@ __global__ __launch_bounds__(BLOCK) void k_chain_shared_h2(GView g, KPlan P, con
 // position-(k-3) candidates (cnt = the parents' filled lengths).
 // Chain tables for thresholds (ta, tb): H[u] = sum over x in N(u) with
 // deg(x) >= ta of |{y in N(x) : deg(y) >= tb}|, H[V + u] = sum of those
-// deg(x).  One wave per vertex.
+// deg(x).  One wave per vertex; degrees as in k_cnt_table.
 static __global__ __launch_bounds__(BLOCK) void k_chain_table(GView g, uint32_t ta, const uint32_t* __restrict__ tb_tbl,
                                                       uint64_t* __restrict__ H) {
   const uint32_t lane = threadIdx.x & 63;
@@ -2681,10 +2683,9 @@ static __global__ __launch_bounds__(BLOCK) void k_chain_table(GView g, uint32_t 
     const uint32_t lo = g.off_out[u], hi = g.off_out[u + 1];
     uint64_t h = 0, hd = 0;
     for (uint32_t i = lo + lane; i < hi; i += 64) {
-      const uint32_t x = g.adj_out[i];
-      const uint32_t dx = g.off_out[x + 1] - g.off_out[x];
+      const uint32_t dx = g.nsig_out[i].x;
       if (dx >= ta) {
-        h += tb_tbl ? tb_tbl[x] : dx;
+        h += tb_tbl ? tb_tbl[g.adj_out[i]] : dx;
         hd += dx;
       }
     }
@@ -2995,6 +2996,32 @@ struct Matcher {
     if (kp.tl_kind == 3)
       return held(kp.ch_ta) && held(kp.ch_tb) && dg.chain_tables.count(std::make_pair(kp.ch_ta, kp.ch_tb)) != 0;
     return held(kp.pr_ta) && held(kp.pr_tb) && (kp.pr_a != kp.pr_b || held(kp.pr_tab));
+  }
+  // the degree and chain tables of this run's closed forms.  Other matchers
+  // may use a cached one on their streams once tables_mu is free: it is built
+  // by then
+  void get_tables() {
+    struct Hold {
+      Context& c;
+      std::lock_guard<std::recursive_mutex> lk;
+      bool built = false;
+      Hold(Context& ctx, std::recursive_mutex& mu) : c(ctx), lk(mu) {}
+      ~Hold() {
+        if (built) (void)hipStreamSynchronize(c.stream);
+      }
+    } hold(c, dg.tables_mu);
+    auto cnt = [&](uint32_t t) { return t > 1 ? cnt_table(c, dg, arena, t, &hold.built) : nullptr; };
+    if (closed_last) tbl = cnt(kp.sc_thr);
+    if (chain || (tail && kp.tl_kind == 3)) {
+      ctab.ta = cnt(kp.ch_ta);
+      ctab.tb = cnt(kp.ch_tb);
+      ctab.H = chain_table(c, dg, arena, kp.ch_ta, kp.ch_tb, &hold.built);
+    }
+    if (pair || (tail && kp.tl_kind != 3)) {
+      ptbl.a = cnt(kp.pr_ta);
+      ptbl.b = cnt(kp.pr_tb);
+      ptbl.ab = kp.pr_a == kp.pr_b ? cnt(kp.pr_tab) : nullptr;
+    }
   }
   bool past_deadline() {
     if (has_deadline && !aborted && std::chrono::steady_clock::now() >= deadline) aborted = true;
@@ -3916,7 +3943,6 @@ struct Matcher {
     }
     // shared chain candidates: up to one level's share of the budget
     cand_limit = std::max<uint64_t>((nlev ? budget / nlev : budget) / 8, 1u << 10);
-    if (closed_last && kp.sc_thr > 1) tbl = cnt_table(c, dg, arena, kp.sc_thr);
     // with the two-hop index the chain is counted inside the expansion of
     // position k-3 (no rows of level k-3 are stored)
     chain_fused = chain && g.h2_off && kp.ch_ta <= 2;
@@ -3926,16 +3952,7 @@ struct Matcher {
     collapse_fused = pair && kp.pr_collapse && pair_cab_known() && k >= 5 && !(o.time_limit_ms > 0);
     // the fused chain with position k-3's candidates shared by siblings
     sib = chain_fused && kp.ch_sib && !(o.flags & 1024u);
-    if (chain || (tail && kp.tl_kind == 3)) {
-      ctab.ta = kp.ch_ta > 1 ? cnt_table(c, dg, arena, kp.ch_ta) : nullptr;
-      ctab.tb = kp.ch_tb > 1 ? cnt_table(c, dg, arena, kp.ch_tb) : nullptr;
-      ctab.H = chain_table(c, dg, arena, kp.ch_ta, kp.ch_tb);
-    }
-    if (pair || (tail && kp.tl_kind != 3)) {
-      ptbl.a = kp.pr_ta > 1 ? cnt_table(c, dg, arena, kp.pr_ta) : nullptr;
-      ptbl.b = kp.pr_tb > 1 ? cnt_table(c, dg, arena, kp.pr_tb) : nullptr;
-      ptbl.ab = kp.pr_a == kp.pr_b && kp.pr_tab > 1 ? cnt_table(c, dg, arena, kp.pr_tab) : nullptr;
-    }
+    get_tables();
     // level sizes of this query's last complete run (a hint only: a level
     // that outgrows it repeats the run)
     std::string hint_key = std::to_string((uintptr_t)&dg) + "/" + std::to_string((uintptr_t)&plan);
@@ -4134,8 +4151,10 @@ void* ScratchArena::carve(uint64_t bytes) {
 }
 
 // Degree-threshold table: cached on the device graph, or, with an arena,
-// built in the scratch for this call only (and not cached).
-const uint32_t* cnt_table(Context& c, DeviceGraph& dg, ScratchArena* arena, uint32_t thr) {
+// built in the scratch for this call only (and not cached).  With `built` the
+// caller holds tables_mu and waits for c.stream before it lets go (one wait
+// for all tables of a run); *built is set when a table is on its way.
+const uint32_t* cnt_table(Context& c, DeviceGraph& dg, ScratchArena* arena, uint32_t thr, bool* built) {
   // concurrent matchers (cuts_match_many) share the device graph
   std::lock_guard<std::recursive_mutex> lk(dg.tables_mu);
   auto it = dg.cnt_tables.find(thr);
@@ -4145,13 +4164,14 @@ const uint32_t* cnt_table(Context& c, DeviceGraph& dg, ScratchArena* arena, uint
   const GView g = view_of(dg);
   hipLaunchKernelGGL(k_cnt_table, dim3(grid_for(dg.V, BLOCK / 64, 65535)), dim3(BLOCK), 0, c.stream, g, thr, t);
   HIPCHECK(hipGetLastError());
-  HIPCHECK(hipStreamSynchronize(c.stream));
+  if (built) *built = true;
+  else HIPCHECK(hipStreamSynchronize(c.stream));
   if (!arena) dg.cnt_tables.emplace(thr, t);
   return t;
 }
 const uint32_t* cnt_table(Context& c, DeviceGraph& dg, uint32_t thr) { return cnt_table(c, dg, nullptr, thr); }
 
-const uint64_t* chain_table(Context& c, DeviceGraph& dg, ScratchArena* arena, uint32_t ta, uint32_t tb) {
+const uint64_t* chain_table(Context& c, DeviceGraph& dg, ScratchArena* arena, uint32_t ta, uint32_t tb, bool* built) {
   std::lock_guard<std::recursive_mutex> lk(dg.tables_mu);
   const auto key = std::make_pair(ta, tb);
   auto it = dg.chain_tables.find(key);
@@ -4159,10 +4179,11 @@ const uint64_t* chain_table(Context& c, DeviceGraph& dg, ScratchArena* arena, ui
   uint64_t* t = nullptr;
   dev_alloc(arena, t, 2 * (uint64_t)dg.V + 1);
   const GView g = view_of(dg);
-  const uint32_t* tbt = tb > 1 ? cnt_table(c, dg, arena, tb) : nullptr;
+  const uint32_t* tbt = tb > 1 ? cnt_table(c, dg, arena, tb, built) : nullptr;
   hipLaunchKernelGGL(k_chain_table, dim3(grid_for(dg.V, BLOCK / 64, 65535)), dim3(BLOCK), 0, c.stream, g, ta, tbt, t);
   HIPCHECK(hipGetLastError());
-  HIPCHECK(hipStreamSynchronize(c.stream));
+  if (built) *built = true;
+  else HIPCHECK(hipStreamSynchronize(c.stream));
   if (!arena) dg.chain_tables.emplace(key, t);
   return t;
 }
