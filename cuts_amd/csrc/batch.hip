@@ -946,6 +946,43 @@ T* balloc(Batch& b, int slot, uint64_t n) {
 }
 }  // namespace
 
+// The level-0 items of at most `chunk` of every query's roots, and their number
+// per query.
+static void level0_items(const std::vector<uint32_t>& cnt, uint32_t chunk, std::vector<Item>& init,
+                         std::vector<unsigned long long>& qinit) {
+  init.clear();
+  qinit.assign(cnt.size(), 0);
+  for (uint32_t q = 0; q < cnt.size(); ++q)
+    for (uint64_t off = 0; off < cnt[q]; off += chunk) {
+      Item it;
+      it.qL = q << 8;
+      it.n = (uint32_t)std::min<uint64_t>(chunk, cnt[q] - off);
+      it.off = off;
+      init.push_back(it);
+      ++qinit[q];
+    }
+}
+
+// Level-0 items of vchunk roots and one item per flush from here on: the
+// fewest flushes.  Finer items end in flushes of their own, up to a fifth
+// more of them, which the queue's capacity has not been asked to hold (4-clique
+// on the 4,000-vertex graph: 204 at the largest level for 171).
+static void coarse_items(Batch& b) {
+  std::vector<Item> init;
+  std::vector<unsigned long long> qinit;
+  level0_items(b.root_counts, b.vchunk, init, qinit);
+  if (!init.empty())
+    HIPCHECK(hipMemcpy((void*)b.args.init_items, init.data(), init.size() * sizeof(Item), hipMemcpyHostToDevice));
+  HIPCHECK(hipMemcpy((void*)b.args.qinit, qinit.data(), qinit.size() * 8, hipMemcpyHostToDevice));
+  b.args.n_init = init.size();
+  b.args.item_split = ~0ull;
+  b.coarse = true;
+  if (b.exec) (void)hipGraphExecDestroy(b.exec);
+  if (b.graph) (void)hipGraphDestroy(b.graph);
+  b.exec = nullptr;
+  b.graph = nullptr;
+}
+
 Batch::~Batch() {
   if (ctx) (void)hipSetDevice(ctx->device);
   if (exec) (void)hipGraphExecDestroy(exec);
@@ -972,8 +1009,9 @@ void batch_create(Context& c, DeviceGraph& dg, const std::vector<const Plan*>& p
   const uint64_t qcap = o.queue_cap ? o.queue_cap : (1ull << 22);
   // position-0 roots per query (first, stride, count) and the level-0 items
   std::vector<uint32_t> roots(3 * (size_t)b.nq);
-  std::vector<unsigned long long> qinit(b.nq);
+  std::vector<unsigned long long> qinit;
   std::vector<Item> init;
+  b.root_counts.resize(b.nq);
   uint64_t coarse = 0, fine = 0;  // items of vchunk roots, and of at most L0_ROOTS
   const uint32_t small = std::min<uint32_t>(b.vchunk, L0_ROOTS);
   for (uint32_t q = 0; q < b.nq; ++q) {
@@ -988,23 +1026,13 @@ void batch_create(Context& c, DeviceGraph& dg, const std::vector<const Plan*>& p
     roots[3 * q] = first;
     roots[3 * q + 1] = stride;
     roots[3 * q + 2] = cnt;
+    b.root_counts[q] = cnt;
     coarse += ((uint64_t)cnt + b.vchunk - 1) / b.vchunk;
     fine += ((uint64_t)cnt + small - 1) / small;
   }
   if (coarse > qcap) throw Error(-1, "batch: queue too small for the level-0 items");
   // the queue's extra slots take the finer items
-  const uint32_t chunk = fine <= kExtraItems ? small : b.vchunk;
-  for (uint32_t q = 0; q < b.nq; ++q) {
-    const uint32_t cnt = roots[3 * q + 2];
-    for (uint64_t off = 0; off < cnt; off += chunk) {
-      Item it;
-      it.qL = q << 8;
-      it.n = (uint32_t)std::min<uint64_t>(chunk, cnt - off);
-      it.off = off;
-      init.push_back(it);
-      ++qinit[q];
-    }
-  }
+  level0_items(b.root_counts, fine <= kExtraItems ? small : b.vchunk, init, qinit);
   const uint64_t half_words = (o.arena_bytes ? o.arena_bytes : (8ull << 30)) / 8;
   if (half_words < 16) throw Error(-1, "batch: arena too small");
   std::vector<KPlan> kp(b.nq);
@@ -1169,6 +1197,11 @@ void batch_run(Batch& b, std::vector<BatchQueryResult>& out, double& device_ms, 
   device_ms = ms;
   BState st;
   HIPCHECK(hipMemcpy(&st, b.args.st, sizeof(BState), hipMemcpyDeviceToHost));
+  if ((st.abort.v & 1) && !(st.abort.v & 12) && !b.coarse) {
+    coarse_items(b);
+    batch_run(b, out, device_ms, arena_words);
+    return;
+  }
   if (st.abort.v) {
     const char* why = (st.abort.v & 4)   ? "corrupt work item"
                       : (st.abort.v & 8) ? "a block waited at the level barrier longer than the limit"

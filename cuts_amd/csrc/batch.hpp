@@ -91,6 +91,8 @@ struct Batch {
   uint32_t nq = 0, vchunk = 0, grid = 0, kmax = 0;
   BatchArgs args{};
   std::vector<uint32_t> k;   // query sizes
+  std::vector<uint32_t> root_counts;  // position-0 roots per query
+  bool coarse = false;       // whole level-0 items, one item per flush: a run with finer ones filled the queue
   void* allocs[13] = {nullptr};
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
