@@ -28,7 +28,9 @@ struct Pool {
 };
 
 Pool& pool_of(int device) {
-  static Pool pools[64];
+  // for as long as the process: a graph or a context of static lifetime may
+  // end after everything that was constructed later than it
+  static Pool* const pools = new Pool[64];
   if (device < 0 || device >= 64) throw Error(-1, "device index out of range");
   return pools[device];
 }

@@ -1,0 +1,50 @@
+// CPU driver of the library's device-memory code over a fake device
+// (fake_hip.hpp), built with the sanitizers by tests/test_memory_host.py.  The
+// first argument names the check.
+#include "fake_hip.hpp"
+
+#include <cstring>
+#include <thread>
+#include <vector>
+
+#include "../../cuts_amd/csrc/device.hpp"
+
+namespace cuts {
+void hip_check(hipError_t e, const char* what) {
+  if (e != hipSuccess) throw Error(-4, what);
+}
+}  // namespace cuts
+
+using namespace cuts;
+constexpr uint64_t MB = 1ull << 20;
+
+// A graph of static lifetime: it ends after what was constructed later, the
+// pool among it.
+struct Late {
+  void* block = nullptr;
+  ~Late() {
+    if (!block) return;
+    pool_give(0, block);
+    void* again = pool_take(0, 2 * MB);
+    CHECK(again == block);
+    pool_give(0, again);
+    pool_context(0, -1);
+    CHECK(fake::device().used == 0);
+    std::printf("late ok\n");
+    std::fflush(stdout);
+  }
+} late;
+
+static void end_of_process() {
+  pool_context(0, 1);
+  late.block = pool_take(0, 2 * MB);
+  CHECK(late.block);
+}
+
+int main(int, char** argv) {
+  const std::string what = argv[1];
+  if (what == "end_of_process") end_of_process();
+  else return 3;
+  std::printf("%s ok\n", argv[1]);
+  return 0;
+}

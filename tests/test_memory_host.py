@@ -1,0 +1,31 @@
+"""The library's host-side device-memory code (csrc/pool.cpp) on the CPU, over
+a fake device, under AddressSanitizer and UndefinedBehaviorSanitizer."""
+import os
+import shutil
+import subprocess
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
+
+
+@pytest.fixture(scope="module")
+def driver(tmp_path_factory):
+    if shutil.which("g++") is None or not os.path.isdir(os.path.join(ROCM, "include", "hip")):
+        pytest.skip("needs g++ and the HIP headers")
+    out = tmp_path_factory.mktemp("memory")
+    subprocess.run(["make", "-s", "-C", os.path.join(HERE, "sanitize"), f"OUT={out}", f"ROCM={ROCM}",
+                    f"{out}/memory_driver"], check=True, capture_output=True, timeout=600)
+    return str(out / "memory_driver")
+
+
+def run(driver, check, want):
+    env = dict(os.environ, ASAN_OPTIONS="detect_leaks=0:exitcode=3", OMP_NUM_THREADS="2")
+    r = subprocess.run([driver, check], capture_output=True, text=True, env=env, timeout=120)
+    assert r.returncode == 0 and r.stdout.split("\n")[:len(want)] == want, r.stdout[-2000:] + r.stderr[-4000:]
+    assert "runtime error" not in r.stderr and "AddressSanitizer" not in r.stderr, r.stderr[-4000:]
+
+
+def test_memory_given_back_while_the_process_ends(driver):
+    run(driver, "end_of_process", ["end_of_process ok", "late ok"])
