@@ -4368,10 +4368,10 @@ void context_init(Context& c, int device) {
   HIPCHECK(hipStreamCreateWithFlags(&c.copy_stream, hipStreamNonBlocking));
   HIPCHECK(hipEventCreateWithFlags(&c.copy_ev[0], hipEventDisableTiming));
   HIPCHECK(hipEventCreateWithFlags(&c.copy_ev[1], hipEventDisableTiming));
-  HIPCHECK(hipMalloc(&c.counters, 2 * kCounterWords * sizeof(unsigned long long)));
+  HIPCHECK(device_malloc((void**)&c.counters, 2 * kCounterWords * sizeof(unsigned long long)));
   HIPCHECK(hipHostMalloc(&c.host_pinned, 256, hipHostMallocDefault));
   HIPCHECK(hipHostMalloc(&c.host_res, 1024, hipHostMallocCoherent | hipHostMallocMapped));
-  HIPCHECK(hipMalloc(&c.lvcnt, kMaxQuery * sizeof(unsigned long long)));
+  HIPCHECK(device_malloc((void**)&c.lvcnt, kMaxQuery * sizeof(unsigned long long)));
   HIPCHECK(hipHostGetDevicePointer((void**)&c.host_res_dev, c.host_res, 0));
   pool_context(device, 1);
   c.counted = true;

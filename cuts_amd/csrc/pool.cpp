@@ -53,8 +53,9 @@ hipError_t device_malloc(void** out, uint64_t bytes) {
   if (hipGetDevice(&device) != hipSuccess || device < 0 || device >= 64) return e;
   Pool& p = pool_of(device);
   {
+    // nothing may be kept by now: another thread's failure has given it back,
+    // and there is memory all the same
     std::lock_guard<std::mutex> lk(p.mu);
-    if (p.kept.empty()) return e;
     release(p);
   }
   e = hipMalloc(out, bytes);

@@ -41,9 +41,33 @@ static void end_of_process() {
   CHECK(late.block);
 }
 
+// Another thread gives the kept blocks back between this one's failed
+// allocation and its own look at them.
+static void flushed_by_another() {
+  auto& d = fake::device();
+  d.total = 100 * MB;
+  pool_context(0, 1);
+  pool_give(0, pool_take(0, 3 * MB));  // kept (the limit is 1/32)
+  CHECK(d.used == 3 * MB);
+  void* big = nullptr;
+  CHECK(device_malloc(&big, 96 * MB) == hipSuccess);
+  d.on_failure = [] {
+    void* p = nullptr;
+    CHECK(device_malloc(&p, 4 * MB) == hipSuccess);  // gives the kept block back
+    CHECK(hipFree(p) == hipSuccess);
+  };
+  void* p = nullptr;
+  CHECK(device_malloc(&p, 4 * MB) == hipSuccess);
+  CHECK(hipFree(p) == hipSuccess && hipFree(big) == hipSuccess);
+  CHECK(device_malloc(&p, 200 * MB) == hipErrorOutOfMemory && p == nullptr);
+  pool_context(0, -1);
+  CHECK(d.used == 0);
+}
+
 int main(int, char** argv) {
   const std::string what = argv[1];
   if (what == "end_of_process") end_of_process();
+  else if (what == "flushed_by_another") flushed_by_another();
   else return 3;
   std::printf("%s ok\n", argv[1]);
   return 0;

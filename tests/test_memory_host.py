@@ -29,3 +29,7 @@ def run(driver, check, want):
 
 def test_memory_given_back_while_the_process_ends(driver):
     run(driver, "end_of_process", ["end_of_process ok", "late ok"])
+
+
+def test_allocation_that_fails_while_another_thread_flushes(driver):
+    run(driver, "flushed_by_another", ["flushed_by_another ok"])
