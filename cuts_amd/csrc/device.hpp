@@ -30,12 +30,14 @@ void hip_check(hipError_t e, const char* what);
 // Device memory (pool.cpp).  device_malloc: hipMalloc on the current device
 // that gives the pool's blocks back before it fails.  pool_take / pool_give:
 // blocks kept between graphs; null when there is no memory; a block is given
-// back once the device has finished with it.  pool_context: a context of the
-// device begins (+1) or ends (-1).  device_free_bytes: free memory, kept
-// blocks included.
+// back once the device has finished with it, or, where that is not known
+// (idle false), freed.  device_idle: waits for the current device; false when
+// it could not.  pool_context: a context of the device begins (+1) or ends
+// (-1).  device_free_bytes: free memory, kept blocks included.
 hipError_t device_malloc(void** out, uint64_t bytes);
 void* pool_take(int device, uint64_t bytes);
-void pool_give(int device, void* b);
+void pool_give(int device, void* b, bool idle = true);
+bool device_idle();
 void pool_context(int device, int change);
 uint64_t device_free_bytes(int device);
 

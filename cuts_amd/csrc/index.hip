@@ -250,8 +250,7 @@ struct Temp {
     if (!p) throw Error(-5, "device allocation of " + std::to_string(n * sizeof(T)) + " bytes failed (index build)");
   }
   ~Temp() {
-    (void)hipStreamSynchronize(c.stream);
-    pool_give(c.device, p);
+    pool_give(c.device, p, hipStreamSynchronize(c.stream) == hipSuccess);
   }
   Temp(const Temp&) = delete;
   Temp& operator=(const Temp&) = delete;

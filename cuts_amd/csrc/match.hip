@@ -46,6 +46,7 @@
 #include <mutex>
 
 #include "batch.hpp"
+#include "levels.hpp"
 
 // The library builds this file as six objects side by side, since the
 // chain's unrolled closed form takes the compiler longer than all else
@@ -2840,90 +2841,6 @@ uint32_t grid_for(uint64_t work, uint64_t per_block, uint32_t cap) {
   return (uint32_t)std::min<uint64_t>(b, cap);
 }
 
-// Back to the pool, once the device has finished with it (as hipFree waits).
-void dev_free(void* p) {
-  if (!p) return;
-  int device = 0;
-  (void)hipGetDevice(&device);
-  (void)hipDeviceSynchronize();
-  pool_give(device, p);
-}
-
-// An array on the current device, from the pool; the old one goes back.
-template <typename T>
-void dev_alloc(T*& p, uint64_t n) {
-  dev_free(p);
-  p = nullptr;
-  int device = 0;
-  HIPCHECK(hipGetDevice(&device));
-  p = (T*)pool_take(device, std::max<uint64_t>(n, 1) * sizeof(T));
-  if (!p) throw Error(-5, "device allocation of " + std::to_string(n * sizeof(T)) + " bytes failed");
-}
-
-// An array of the device graph's own, from the pool.
-template <typename T>
-void graph_alloc(const DeviceGraph& dg, T*& p, uint64_t n) {
-  p = (T*)pool_take(dg.device, std::max<uint64_t>(n, 1) * sizeof(T));
-  if (!p) throw Error(-5, "device allocation of " + std::to_string(n * sizeof(T)) + " bytes failed");
-}
-
-// Device buffer of n elements: hipMalloc'd (the old one freed), or carved
-// from the arena when there is one (nothing freed; sizes are rounded up to a
-// power of two so that regrowth wastes at most half of what was carved).
-template <typename T>
-void dev_alloc(ScratchArena* a, T*& p, uint64_t n) {
-  if (!a) {
-    dev_alloc(p, n);
-    return;
-  }
-  uint64_t m = 1;
-  while (m < std::max<uint64_t>(n, 1)) m <<= 1;
-  p = (T*)a->carve(m * sizeof(T));
-}
-
-// Makes sure level buffer `lv` can hold `rows` rows of `words` words plus
-// the planning arrays for them.
-void ensure_rows(ScratchArena* ar, LevelBuf& b, uint64_t rows, uint32_t words) {
-  if (b.cap >= rows && b.rows) return;
-  uint64_t cap = std::max<uint64_t>(rows, 1024);
-  if (b.cap) cap = std::max<uint64_t>(cap, b.cap + b.cap / 2);
-  dev_alloc(ar, b.rows, cap * words);
-  dev_alloc(ar, b.minlen, cap);
-  dev_alloc(ar, b.minsel, cap);
-  dev_alloc(ar, b.work_off, cap + 1);
-  dev_alloc(ar, b.cbase, cap);
-  b.cap = cap;
-}
-void ensure_rows_exact(ScratchArena* ar, LevelBuf& b, uint64_t rows, uint32_t words) {
-  // like ensure_rows but never grows beyond `rows` (budget-bound levels)
-  if (b.cap >= rows && b.rows) return;
-  dev_alloc(ar, b.rows, std::max<uint64_t>(rows, 1) * words);
-  dev_alloc(ar, b.minlen, std::max<uint64_t>(rows, 1));
-  dev_alloc(ar, b.minsel, std::max<uint64_t>(rows, 1));
-  dev_alloc(ar, b.work_off, std::max<uint64_t>(rows, 1) + 1);
-  dev_alloc(ar, b.cbase, std::max<uint64_t>(rows, 1));
-  b.cap = rows;
-}
-// The per-row arrays of the pair and chain levels, allocated only for the
-// levels that use them (each grows to the level's row capacity).
-template <typename T>
-void ensure_aux(ScratchArena* ar, T*& p, uint64_t& cap, uint64_t rows) {
-  if (cap >= rows && p) return;
-  dev_alloc(ar, p, std::max<uint64_t>(rows, 1));
-  cap = std::max<uint64_t>(rows, 1);
-}
-
-void ensure_bsum(ScratchArena* ar, LevelBuf& b, uint64_t nb) {
-  if (b.bsum_cap >= nb + 1 && b.bsum) return;
-  dev_alloc(ar, b.bsum, nb + 1);
-  b.bsum_cap = nb + 1;
-}
-void ensure_tiles(ScratchArena* ar, LevelBuf& b, uint64_t nt) {
-  if (b.tile_cap >= nt + 1 && b.tile_p) return;
-  dev_alloc(ar, b.tile_p, nt + 1);
-  b.tile_cap = nt + 1;
-}
-
 struct Matcher {
   Context& c;
   DeviceGraph& dg;
@@ -4312,7 +4229,7 @@ DeviceGraph::~DeviceGraph() {
   (void)hipGetDevice(&prev);
   (void)hipSetDevice(device);
   // the next owner of these blocks may use them on any stream
-  (void)hipDeviceSynchronize();
+  const bool idle = device_idle();
   if (symmetric) {
     off_in = adj_in = nullptr;  // the out-side's
     nsig_in = nullptr;
@@ -4321,20 +4238,20 @@ DeviceGraph::~DeviceGraph() {
                   (void*)nsig_in, (void*)hub_id, (void*)bits, (void*)hub_dir[0], (void*)hub_dir[1],
                   (void*)bits_dir[0], (void*)bits_dir[1], (void*)arc_cn, (void*)h2_off, (void*)h2_v, (void*)h2_c,
                   (void*)h2_did, (void*)h2_dense, (void*)hr_id, (void*)hr})
-    pool_give(device, p);
-  for (auto& kv : cnt_tables) pool_give(device, kv.second);
-  for (auto& kv : chain_tables) pool_give(device, kv.second);
+    pool_give(device, p, idle);
+  for (auto& kv : cnt_tables) pool_give(device, kv.second, idle);
+  for (auto& kv : chain_tables) pool_give(device, kv.second, idle);
   (void)hipSetDevice(prev);
 }
 
 Context::~Context() {
   (void)hipSetDevice(device);
-  (void)hipDeviceSynchronize();  // the level buffers' next owner may use them on any stream
+  const bool idle = device_idle();  // the level buffers' next owner may use them on any stream
   for (auto& b : lv) {
     for (void* p : {(void*)b.rows, (void*)b.rows2, (void*)b.minlen, (void*)b.minsel, (void*)b.work_off, (void*)b.bsum,
                     (void*)b.tile_p, (void*)b.cbase, (void*)b.pbase,
                     (void*)b.nsurv, (void*)b.parent, (void*)b.coff, (void*)b.cand})
-      pool_give(device, p);
+      pool_give(device, p, idle);
   }
   if (counters) (void)hipFree(counters);
   if (host_pinned) (void)hipHostFree(host_pinned);

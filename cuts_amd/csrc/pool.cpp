@@ -88,7 +88,13 @@ void* pool_take(int device, uint64_t bytes) {
   return b;
 }
 
-void pool_give(int device, void* b) {
+bool device_idle() {
+  if (hipDeviceSynchronize() == hipSuccess) return true;
+  (void)hipGetLastError();
+  return false;
+}
+
+void pool_give(int device, void* b, bool idle) {
   if (!b) return;
   Pool& p = pool_of(device);
   {
@@ -97,7 +103,7 @@ void pool_give(int device, void* b) {
     if (it != p.handed.end()) {
       const uint64_t bytes = it->second;
       p.handed.erase(it);
-      if (p.contexts > 0 && p.held + bytes <= p.limit) {
+      if (idle && p.contexts > 0 && p.held + bytes <= p.limit) {
         p.kept.emplace(bytes, b);
         p.held += bytes;
         return;

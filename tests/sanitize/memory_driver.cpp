@@ -7,12 +7,13 @@
 #include <thread>
 #include <vector>
 
-#include "../../cuts_amd/csrc/device.hpp"
+#include "../../cuts_amd/csrc/levels.hpp"
 
 namespace cuts {
 void hip_check(hipError_t e, const char* what) {
   if (e != hipSuccess) throw Error(-4, what);
 }
+void* ScratchArena::carve(uint64_t) { return nullptr; }
 }  // namespace cuts
 
 using namespace cuts;
@@ -64,10 +65,40 @@ static void flushed_by_another() {
   CHECK(d.used == 0);
 }
 
+// A block whose users cannot be waited for is not handed to another stream.
+static void given_while_capturing() {
+  auto& d = fake::device();
+  pool_context(0, 1);
+  uint32_t* p = nullptr;
+  dev_alloc(p, MB);
+  CHECK(d.used == 4 * MB);
+  const size_t syncs = d.syncs;
+  dev_free(p);
+  CHECK(d.syncs == syncs + 1 && d.used == 4 * MB);  // waited for, and kept
+  p = nullptr;
+  dev_alloc(p, MB);
+  d.capturing = true;
+  dev_free(p);
+  CHECK(d.used == 0);  // freed, as hipFree waits by itself
+  d.capturing = false;
+  p = nullptr;
+  dev_alloc(p, MB / 2);
+  uint32_t* const first = p;
+  d.capturing = true;
+  dev_alloc(p, MB);  // grown: the old block is freed too
+  d.capturing = false;
+  CHECK(p != first || d.used == 4 * MB);
+  CHECK(d.used == 4 * MB);
+  dev_free(p);
+  pool_context(0, -1);
+  CHECK(d.used == 0);
+}
+
 int main(int, char** argv) {
   const std::string what = argv[1];
   if (what == "end_of_process") end_of_process();
   else if (what == "flushed_by_another") flushed_by_another();
+  else if (what == "given_while_capturing") given_while_capturing();
   else return 3;
   std::printf("%s ok\n", argv[1]);
   return 0;

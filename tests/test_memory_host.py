@@ -1,4 +1,5 @@
-"""The library's host-side device-memory code (csrc/pool.cpp) on the CPU, over
+"""The library's host-side device-memory code (csrc/pool.cpp,
+csrc/levels.hpp) on the CPU, over
 a fake device, under AddressSanitizer and UndefinedBehaviorSanitizer."""
 import os
 import shutil
@@ -33,3 +34,7 @@ def test_memory_given_back_while_the_process_ends(driver):
 
 def test_allocation_that_fails_while_another_thread_flushes(driver):
     run(driver, "flushed_by_another", ["flushed_by_another ok"])
+
+
+def test_blocks_freed_while_a_stream_records(driver):
+    run(driver, "given_while_capturing", ["given_while_capturing ok"])
