@@ -58,6 +58,7 @@ inline void ensure_rows(ScratchArena* ar, LevelBuf& b, uint64_t rows, uint32_t w
   if (b.cap >= rows && b.rows) return;
   uint64_t cap = std::max<uint64_t>(rows, 1024);
   if (b.cap) cap = std::max<uint64_t>(cap, b.cap + b.cap / 2);
+  b.cap = 0;  // until all arrays are there: an allocation may fail
   dev_alloc(ar, b.rows, cap * words);
   dev_alloc(ar, b.minlen, cap);
   dev_alloc(ar, b.minsel, cap);
@@ -68,6 +69,7 @@ inline void ensure_rows(ScratchArena* ar, LevelBuf& b, uint64_t rows, uint32_t w
 inline void ensure_rows_exact(ScratchArena* ar, LevelBuf& b, uint64_t rows, uint32_t words) {
   // like ensure_rows but never grows beyond `rows` (budget-bound levels)
   if (b.cap >= rows && b.rows) return;
+  b.cap = 0;
   dev_alloc(ar, b.rows, std::max<uint64_t>(rows, 1) * words);
   dev_alloc(ar, b.minlen, std::max<uint64_t>(rows, 1));
   dev_alloc(ar, b.minsel, std::max<uint64_t>(rows, 1));

@@ -94,11 +94,44 @@ static void given_while_capturing() {
   CHECK(d.used == 0);
 }
 
+// Memory runs out while a level grows: the level holds what it says, and the
+// next, smaller request gets all of its arrays.
+static void growth_that_fails() {
+  auto& d = fake::device();
+  pool_context(0, 1);
+  auto whole = [](const LevelBuf& b) { return b.rows && b.minlen && b.minsel && b.work_off && b.cbase; };
+  for (int exact = 0; exact < 2; ++exact) {
+    LevelBuf b;
+    auto ensure = [&](uint64_t n) { exact ? ensure_rows_exact(nullptr, b, n, 4) : ensure_rows(nullptr, b, n, 4); };
+    d.total = 1024 * MB;
+    ensure(MB);
+    CHECK(whole(b) && b.cap == MB);
+    for (uint64_t room = 0; room < 64; room += 3) {  // out of memory at each array in turn
+      d.total = d.used + room * MB;
+      bool failed = false;
+      try {
+        ensure(2 * MB);
+      } catch (const Error& e) {
+        failed = e.code == -5;
+      }
+      CHECK(failed ? b.cap == 0 || whole(b) : whole(b) && b.cap >= 2 * MB);
+      d.total = 1024 * MB;
+      ensure(MB / 2);
+      CHECK(whole(b) && b.cap >= MB / 2);
+      if (!failed) break;
+    }
+    for (void* p : {(void*)b.rows, (void*)b.minlen, (void*)b.minsel, (void*)b.work_off, (void*)b.cbase}) dev_free(p);
+  }
+  pool_context(0, -1);
+  CHECK(d.used == 0);
+}
+
 int main(int, char** argv) {
   const std::string what = argv[1];
   if (what == "end_of_process") end_of_process();
   else if (what == "flushed_by_another") flushed_by_another();
   else if (what == "given_while_capturing") given_while_capturing();
+  else if (what == "growth_that_fails") growth_that_fails();
   else return 3;
   std::printf("%s ok\n", argv[1]);
   return 0;

@@ -38,3 +38,7 @@ def test_allocation_that_fails_while_another_thread_flushes(driver):
 
 def test_blocks_freed_while_a_stream_records(driver):
     run(driver, "given_while_capturing", ["given_while_capturing ok"])
+
+
+def test_level_buffers_when_memory_runs_out(driver):
+    run(driver, "growth_that_fails", ["growth_that_fails ok"])
