@@ -533,22 +533,9 @@ __global__ __launch_bounds__(256) void k_mpnn_pack(const float* __restrict__ p, 
 }
 
 // ------------------------------------------------------------------ host
-namespace {
 template <typename T>
-T* malloc_dev(uint64_t n) {
-  void* p = nullptr;
-  if (device_malloc(&p, std::max<uint64_t>(n, 1) * sizeof(T)) != hipSuccess)
-    throw Error(-5, "mpnn: device allocation failed");
-  return (T*)p;
-}
-}  // namespace
-
-Mpnn::~Mpnn() {
-  if (ctx) (void)hipSetDevice(ctx->device);
-  for (void* q : {(void*)p, (void*)m, (void*)v, (void*)g, (void*)w, (void*)wt, (void*)part, (void*)loss,
-                  (void*)x, (void*)row, (void*)adj, (void*)meta, (void*)t, (void*)y})
-    if (q) (void)hipFree(q);
-  if (stage) (void)hipHostFree(stage);
+static T* malloc_dev(uint64_t n) {
+  return (T*)mpnn_malloc(n * sizeof(T));
 }
 
 void mpnn_init(Context& c, Mpnn& n, const float* params) {
@@ -602,17 +589,7 @@ struct Upload {
 // copies the padded samples as they are.
 static Upload upload(Mpnn& n, uint32_t cnt, const float* x, const uint16_t* adj, const uint32_t* meta, const float* t) {
   constexpr uint64_t kMost = 64ull << 20;
-  if (cnt > n.cap) {
-    for (void* q : {(void*)n.x, (void*)n.row, (void*)n.adj, (void*)n.meta, (void*)n.t, (void*)n.y})
-      if (q) (void)hipFree(q);
-    n.cap = std::max<uint32_t>(cnt, 1024);
-    n.x = malloc_dev<float>((uint64_t)n.cap * MAXN * FIN);
-    n.row = malloc_dev<uint32_t>(n.cap);
-    n.adj = malloc_dev<uint16_t>((uint64_t)n.cap * MAXN);
-    n.meta = malloc_dev<uint32_t>(n.cap);
-    n.t = malloc_dev<float>(n.cap);
-    n.y = malloc_dev<float>(n.cap);
-  }
+  mpnn_reserve(n, cnt);
   hipStream_t s = n.ctx->stream;
   Upload u(s, cnt);
   HIPCHECK(hipMemcpyAsync(n.adj, adj, (uint64_t)cnt * MAXN * 2, hipMemcpyHostToDevice, s));

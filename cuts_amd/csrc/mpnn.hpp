@@ -33,6 +33,10 @@ struct Mpnn {
   ~Mpnn();
 };
 
+// Device memory of the network's (pack.cpp); an error when there is none.
+void* mpnn_malloc(uint64_t bytes);
+// Makes room for cnt samples.
+void mpnn_reserve(Mpnn& n, uint32_t cnt);
 // The live rows of samples first .. last-1 (row: their first rows) to out.
 void pack_rows(const float* x, const uint32_t* meta, const uint32_t* row, uint32_t first, uint32_t last, float* out);
 

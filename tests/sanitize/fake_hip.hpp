@@ -76,6 +76,10 @@ hipError_t hipGetDevice(int* i) {
   return hipSuccess;
 }
 hipError_t hipSetDevice(int) { return hipSuccess; }
+hipError_t hipHostFree(void* p) {
+  std::free(p);
+  return hipSuccess;
+}
 hipError_t hipGetLastError() { return hipSuccess; }
 hipError_t hipDeviceSynchronize() {
   auto& d = fake::device();

@@ -8,6 +8,7 @@
 #include <vector>
 
 #include "../../cuts_amd/csrc/levels.hpp"
+#include "../../cuts_amd/csrc/mpnn.hpp"
 
 namespace cuts {
 void hip_check(hipError_t e, const char* what) {
@@ -126,12 +127,44 @@ static void growth_that_fails() {
   CHECK(d.used == 0);
 }
 
+// Memory runs out while a network's buffers grow: a later call finds them
+// whole, and no buffer is freed twice.
+static void network_that_does_not_fit() {
+  auto& d = fake::device();
+  const uint64_t per = kMpnnNodes * (kMpnnFeats * 4 + 2) + 4 * 4;
+  auto whole = [](const Mpnn& n) { return n.x && n.row && n.adj && n.meta && n.t && n.y; };
+  for (uint64_t room = 0; room <= 10000 * per; room += 50 * 1024) {
+    d.total = 1024 * MB;
+    Mpnn n;
+    mpnn_reserve(n, 5);
+    CHECK(whole(n) && n.cap == 1024);
+    const size_t first = d.used;
+    d.total = d.used + room;
+    bool failed = false;
+    try {
+      mpnn_reserve(n, 10000);
+    } catch (const Error& e) {
+      failed = e.code == -5;
+    }
+    CHECK(failed ? n.cap == 0 : whole(n) && n.cap == 10000);
+    if (failed) {
+      d.total = 1024 * MB;
+      mpnn_reserve(n, 1024);
+      CHECK(whole(n) && n.cap == 1024 && d.used >= first);
+      mpnn_reserve(n, 2000);
+      CHECK(whole(n) && n.cap == 2000);
+    }
+  }
+  CHECK(d.used == 0);
+}
+
 int main(int, char** argv) {
   const std::string what = argv[1];
   if (what == "end_of_process") end_of_process();
   else if (what == "flushed_by_another") flushed_by_another();
   else if (what == "given_while_capturing") given_while_capturing();
   else if (what == "growth_that_fails") growth_that_fails();
+  else if (what == "network_that_does_not_fit") network_that_does_not_fit();
   else return 3;
   std::printf("%s ok\n", argv[1]);
   return 0;

@@ -1,5 +1,5 @@
 """The library's host-side device-memory code (csrc/pool.cpp,
-csrc/levels.hpp) on the CPU, over
+csrc/levels.hpp, csrc/pack.cpp) on the CPU, over
 a fake device, under AddressSanitizer and UndefinedBehaviorSanitizer."""
 import os
 import shutil
@@ -42,3 +42,7 @@ def test_blocks_freed_while_a_stream_records(driver):
 
 def test_level_buffers_when_memory_runs_out(driver):
     run(driver, "growth_that_fails", ["growth_that_fails ok"])
+
+
+def test_network_buffers_when_memory_runs_out(driver):
+    run(driver, "network_that_does_not_fit", ["network_that_does_not_fit ok"])
