@@ -118,6 +118,7 @@ def lib():
             "cuts_plan_free": (None, [vp]),
             "cuts_context_create": (C.c_int, [C.c_int, pp]),
             "cuts_context_destroy": (None, [vp]),
+            "cuts_context_trim": (C.c_int, [vp, C.POINTER(C.c_uint64)]),
             "cuts_device_graph_upload": (C.c_int, [vp, vp, pp]),
             "cuts_device_graph_free": (None, [vp]),
             "cuts_device_graph_query": (C.c_int, [vp, C.POINTER(_DGInfo)]),
@@ -424,6 +425,14 @@ class Context:
         gbps = C.c_double()
         _check(lib().cuts_copy_probe(self._h, nbytes, iters, C.byref(gbps)))
         return gbps.value
+
+    def trim(self) -> int:
+        """Frees the device memory that released graphs and outgrown levels
+        left for the next ones (cuts_context_trim), for another allocator of
+        the process; returns its bytes."""
+        n = C.c_uint64()
+        _check(lib().cuts_context_trim(self._h, C.byref(n)))
+        return n.value
 
     def upload(self, g: Graph) -> DeviceGraph:
         h = C.c_void_p()

@@ -354,6 +354,16 @@ int cuts_context_create(int device, cuts_context** out) {
 
 void cuts_context_destroy(cuts_context* ctx) { delete ctx; }
 
+int cuts_context_trim(cuts_context* ctx, uint64_t* freed) {
+  return guard([&]() -> int {
+    if (!ctx) return fail(CUTS_E_ARG, "null argument");
+    cuts::hip_check(hipSetDevice(ctx->c.device), "hipSetDevice");
+    const uint64_t n = cuts::pool_trim(ctx->c.device);
+    if (freed) *freed = n;
+    return CUTS_OK;
+  });
+}
+
 int cuts_device_graph_upload(cuts_context* ctx, const cuts_graph* g, cuts_device_graph** out) {
   return guard([&]() -> int {
     if (!ctx || !g || !out) return fail(CUTS_E_ARG, "null argument");

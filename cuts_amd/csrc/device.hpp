@@ -33,12 +33,14 @@ void hip_check(hipError_t e, const char* what);
 // back once the device has finished with it, or, where that is not known
 // (idle false), freed.  device_idle: waits for the current device; false when
 // it could not.  pool_context: a context of the device begins (+1) or ends
-// (-1).  device_free_bytes: free memory, kept blocks included.
+// (-1).  pool_trim: frees the kept blocks, returns their bytes.
+// device_free_bytes: free memory, kept blocks included.
 hipError_t device_malloc(void** out, uint64_t bytes);
 void* pool_take(int device, uint64_t bytes);
 void pool_give(int device, void* b, bool idle = true);
 bool device_idle();
 void pool_context(int device, int change);
+uint64_t pool_trim(int device);
 uint64_t device_free_bytes(int device);
 
 // Plan in the form the kernels read: per position the list of constraints

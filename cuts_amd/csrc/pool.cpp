@@ -4,8 +4,8 @@
 // handed out once: uploads of a few milliseconds of kernels then waited 40 to
 // 85 ms for memory (R-MAT 18, 3.3 GB).  Freed blocks of at least kKeepMin
 // bytes stay here, up to 1/32 of the device's memory, while a context of the
-// device exists; an allocation takes one that is at most a quarter larger
-// than asked.  They count as free memory (device_free_bytes), and every
+// device exists and until pool_trim frees them; an allocation takes one that
+// is at most a quarter larger than asked.  They count as free memory (device_free_bytes), and every
 // allocation of the library that fails gives them back and tries again.
 #include <map>
 #include <mutex>
@@ -123,6 +123,14 @@ void pool_context(int device, int change) {
     size_t fr = 0, tot = 0;
     if (hipMemGetInfo(&fr, &tot) == hipSuccess) p.limit = tot / 32;
   }
+}
+
+uint64_t pool_trim(int device) {
+  Pool& p = pool_of(device);
+  std::lock_guard<std::mutex> lk(p.mu);
+  const uint64_t held = p.held;
+  release(p);
+  return held;
 }
 
 uint64_t device_free_bytes(int device) {

@@ -88,6 +88,13 @@ void cuts_plan_free(cuts_plan *p);
 /* ---- device ----------------------------------------------------------- */
 int cuts_context_create(int device, cuts_context **out);
 void cuts_context_destroy(cuts_context *ctx);
+/* Device memory of released graphs and outgrown trie levels is kept for the
+ * next ones, up to 1/32 of the device's memory, while a context of the device
+ * exists.  The library counts it as free and gives it back before an
+ * allocation of its own fails; another allocator of the process cannot.  This
+ * call frees it, for such an allocator (no reference counterpart).  freed, when
+ * not null, receives the bytes. */
+int cuts_context_trim(cuts_context *ctx, uint64_t *freed);
 /* Copies the CSR + signatures to HBM (src/gpu_memory_allocation.cu:26-36). */
 int cuts_device_graph_upload(cuts_context *ctx, const cuts_graph *g, cuts_device_graph **out);
 void cuts_device_graph_free(cuts_device_graph *dg);

@@ -158,6 +158,43 @@ static void network_that_does_not_fit() {
   CHECK(d.used == 0);
 }
 
+// Eight threads take and give blocks, give the kept ones back and run out of
+// memory now and then; nothing is kept beyond the limit or lost.
+static void threads() {
+  auto& d = fake::device();
+  d.total = 256 * MB;
+  pool_context(0, 1);
+  std::vector<std::thread> ts;
+  for (int t = 0; t < 8; ++t)
+    ts.emplace_back([t] {
+      unsigned seed = 7 + t;
+      std::vector<void*> mine;
+      for (int i = 0; i < 4000; ++i) {
+        const uint64_t n = (1 + rand_r(&seed) % 8) * MB + rand_r(&seed) % 1000;
+        if (void* p = pool_take(0, n)) mine.push_back(p);
+        while (mine.size() > 6 || (!mine.empty() && rand_r(&seed) % 2)) {
+          pool_give(0, mine.back(), rand_r(&seed) % 16 != 0);
+          mine.pop_back();
+        }
+        if (i % 64 == 0) pool_trim(0);
+        if (i % 97 == 0) {
+          pool_context(0, 1);
+          pool_context(0, -1);
+        }
+      }
+      for (void* p : mine) pool_give(0, p);
+    });
+  for (auto& t : ts) t.join();
+  CHECK(d.used <= d.total / 32);
+  CHECK(device_free_bytes(0) == d.total);
+  const uint64_t kept = d.used;
+  CHECK(pool_trim(0) == kept && d.used == 0 && pool_trim(0) == 0);
+  pool_give(0, pool_take(0, 2 * MB));
+  CHECK(d.used == 2 * MB);
+  pool_context(0, -1);
+  CHECK(d.used == 0);
+}
+
 int main(int, char** argv) {
   const std::string what = argv[1];
   if (what == "end_of_process") end_of_process();
@@ -165,6 +202,7 @@ int main(int, char** argv) {
   else if (what == "given_while_capturing") given_while_capturing();
   else if (what == "growth_that_fails") growth_that_fails();
   else if (what == "network_that_does_not_fit") network_that_does_not_fit();
+  else if (what == "threads") threads();
   else return 3;
   std::printf("%s ok\n", argv[1]);
   return 0;

@@ -1,6 +1,7 @@
 """The library's host-side device-memory code (csrc/pool.cpp,
 csrc/levels.hpp, csrc/pack.cpp) on the CPU, over
 a fake device, under AddressSanitizer and UndefinedBehaviorSanitizer."""
+import ctypes
 import os
 import shutil
 import subprocess
@@ -46,3 +47,34 @@ def test_level_buffers_when_memory_runs_out(driver):
 
 def test_network_buffers_when_memory_runs_out(driver):
     run(driver, "network_that_does_not_fit", ["network_that_does_not_fit ok"])
+
+
+def test_kept_memory_with_several_threads_and_given_back(driver):
+    run(driver, "threads", ["threads ok"])
+
+
+@pytest.mark.gpu
+def test_trim():
+    """The index of a released graph stays with the library until it is asked
+    for; the counts of later graphs do not depend on it."""
+    import cuts_amd as F
+    ctx = F.Context()
+    hip = ctypes.CDLL("libamdhip64.so")  # the runtime that the library has loaded
+
+    def free_bytes():
+        fr, tot = ctypes.c_size_t(), ctypes.c_size_t()
+        assert hip.hipMemGetInfo(ctypes.byref(fr), ctypes.byref(tot)) == 0
+        return fr.value
+
+    ctx.trim()
+    g = F.Graph.chung_lu(20000, 100000, 2.2, 900, 3)
+    p = F.Plan(F.Graph.from_edges(4, [(0, 1), (1, 2), (2, 0), (2, 3)]))
+    dg = ctx.upload(g)
+    want = ctx.match(dg, p).count
+    del dg
+    before = free_bytes()
+    freed = ctx.trim()
+    assert freed >= 1 << 20
+    assert free_bytes() - before >= freed // 2
+    assert ctx.trim() == 0
+    assert ctx.match(ctx.upload(g), p).count == want
