@@ -151,6 +151,8 @@ struct DeviceGraph {
   int32_t* h2_did = nullptr;
   uint16_t* h2_dense = nullptr;
   uint32_t h2_dense_rows = 0;
+  char* slab = nullptr;  // the small arrays (graph_alloc)
+  uint64_t slab_used = 0;
   double h2_build_s = 0;
   bool h2_on_gpu = false;  // built on the device (V <= 2^17) rather than on the host
   // per-arc common-neighbour counts (symmetric loop-free graphs): arc_cn[i]

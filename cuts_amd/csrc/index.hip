@@ -24,6 +24,7 @@
 #include <algorithm>
 
 #include "batch.hpp"
+#include "levels.hpp"
 
 namespace cuts {
 
@@ -240,16 +241,17 @@ __global__ __launch_bounds__(RB) void k_row_scan(uint32_t* __restrict__ tcnt, ui
   }
 }
 
-// A device buffer of this build, from the pool; the stream has drained when
-// it ends (each build synchronizes before it returns; an error may not have).
+// A device buffer of this build: a small one from the graph's slab, else from
+// the pool; the stream has drained when it ends (each build synchronizes before
+// it returns; an error may not have).
 template <typename T>
 struct Temp {
   Context& c;
-  T* p;
-  Temp(Context& ctx, uint64_t n) : c(ctx), p((T*)pool_take(ctx.device, std::max<uint64_t>(n, 1) * sizeof(T))) {
-    if (!p) throw Error(-5, "device allocation of " + std::to_string(n * sizeof(T)) + " bytes failed (index build)");
-  }
+  DeviceGraph& dg;
+  T* p = nullptr;
+  Temp(Context& ctx, DeviceGraph& g, uint64_t n) : c(ctx), dg(g) { graph_alloc(dg, p, n); }
   ~Temp() {
+    if (in_slab(dg, p)) return;
     pool_give(c.device, p, hipStreamSynchronize(c.stream) == hipSuccess);
   }
   Temp(const Temp&) = delete;
@@ -302,8 +304,8 @@ void build_hub_rows(Context& c, DeviceGraph& dg, const std::vector<uint32_t>& hu
   a.nrows = (uint32_t)hubs.size();
   a.out = dg.hr;
   const uint32_t at_once = groups_at_once((a.nrows + 63) / 64, a.V);
-  Temp<uint32_t> rowv(c, hubs.size());
-  Temp<unsigned long long> mask(c, (uint64_t)at_once * a.V);
+  Temp<uint32_t> rowv(c, dg, hubs.size());
+  Temp<unsigned long long> mask(c, dg, (uint64_t)at_once * a.V);
   HIPCHECK(hipMemcpy(rowv.p, hubs.data(), hubs.size() * 4, hipMemcpyHostToDevice));
   a.rowv = rowv.p;
   row_passes<HUB_ROWS>(c, a, mask.p, at_once, true);
@@ -315,8 +317,8 @@ void build_two_hop_device(Context& c, DeviceGraph& dg, std::vector<uint64_t>& of
   RowArgs a = row_args(dg);
   const uint32_t V = a.V, groups = (V + 63) / 64, at_once = groups_at_once(groups, V);
   a.nrows = V;
-  Temp<unsigned long long> mask(c, (uint64_t)at_once * V), total(c, V);
-  Temp<uint32_t> tcnt(c, (uint64_t)V * a.ntiles);
+  Temp<unsigned long long> mask(c, dg, (uint64_t)at_once * V), total(c, dg, V);
+  Temp<uint32_t> tcnt(c, dg, (uint64_t)V * a.ntiles);
   a.tcnt = tcnt.p;
   row_passes<H2_COUNT>(c, a, mask.p, at_once, true);
   hipLaunchKernelGGL(k_row_scan, dim3(std::min<uint32_t>((V + 3) / 4, 65535)), dim3(RB), 0, c.stream, tcnt.p, V,
@@ -328,20 +330,16 @@ void build_two_hop_device(Context& c, DeviceGraph& dg, std::vector<uint64_t>& of
   for (uint32_t u = 0; u < V; ++u) off[u + 1] = off[u] + t[u];
   dg.h2_entries = off[V];
   const std::vector<uint32_t> cand = dense_rows(off);
-  auto alloc = [&](auto*& p, uint64_t n) {
-    p = (std::remove_reference_t<decltype(p)>)pool_take(dg.device, std::max<uint64_t>(n, 1) * sizeof(*p));
-    if (!p) throw Error(-5, "device allocation of " + std::to_string(n * sizeof(*p)) + " bytes failed (two-hop index)");
-  };
-  alloc(dg.h2_off, (uint64_t)V + 1);
+  graph_alloc(dg, dg.h2_off, (uint64_t)V + 1);
   HIPCHECK(hipMemcpy(dg.h2_off, off.data(), ((uint64_t)V + 1) * 8, hipMemcpyHostToDevice));
-  alloc(dg.h2_v, off[V]);
-  alloc(dg.h2_c, off[V]);
+  graph_alloc(dg, dg.h2_v, off[V]);
+  graph_alloc(dg, dg.h2_c, off[V]);
   if (!cand.empty()) {
     std::vector<int32_t> did(V, -1);
     for (uint64_t r = 0; r < cand.size(); ++r) did[cand[r]] = (int32_t)r;
-    alloc(dg.h2_did, V);
+    graph_alloc(dg, dg.h2_did, V);
     HIPCHECK(hipMemcpy(dg.h2_did, did.data(), (uint64_t)V * 4, hipMemcpyHostToDevice));
-    alloc(dg.h2_dense, cand.size() * V);
+    graph_alloc(dg, dg.h2_dense, cand.size() * V);
     dg.h2_dense_rows = (uint32_t)cand.size();
   }
   a.h2_off = dg.h2_off;

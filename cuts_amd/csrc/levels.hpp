@@ -30,11 +30,28 @@ void dev_alloc(T*& p, uint64_t n) {
   if (!p) throw Error(-5, "device allocation of " + std::to_string(n * sizeof(T)) + " bytes failed");
 }
 
-// An array of the device graph's own, from the pool.
+// An array of the device graph's own: of up to kSlabMost bytes from the graph's
+// slab while that has room, else a block of its own.  Both come from the pool,
+// which keeps slabs but not blocks that small: with an allocation for each of
+// its 10 to 25 arrays a small graph's upload was mostly those.
+constexpr uint64_t kSlab = 1ull << 20, kSlabMost = 128ull << 10;
 template <typename T>
-void graph_alloc(const DeviceGraph& dg, T*& p, uint64_t n) {
-  p = (T*)pool_take(dg.device, std::max<uint64_t>(n, 1) * sizeof(T));
-  if (!p) throw Error(-5, "device allocation of " + std::to_string(n * sizeof(T)) + " bytes failed");
+void graph_alloc(DeviceGraph& dg, T*& p, uint64_t n) {
+  const uint64_t bytes = std::max<uint64_t>(n, 1) * sizeof(T);
+  if (bytes <= kSlabMost) {
+    if (!dg.slab) dg.slab = (char*)pool_take(dg.device, kSlab);
+    const uint64_t at = (dg.slab_used + 255) & ~255ull;
+    if (dg.slab && at + bytes <= kSlab) {
+      p = (T*)(dg.slab + at);
+      dg.slab_used = at + bytes;
+      return;
+    }
+  }
+  p = (T*)pool_take(dg.device, bytes);
+  if (!p) throw Error(-5, "device allocation of " + std::to_string(bytes) + " bytes failed");
+}
+inline bool in_slab(const DeviceGraph& dg, const void* p) {
+  return dg.slab && (const char*)p >= dg.slab && (const char*)p < dg.slab + kSlab;
 }
 
 // Device buffer of n elements: from the pool (the old one goes back to it), or

@@ -4238,9 +4238,10 @@ DeviceGraph::~DeviceGraph() {
                   (void*)nsig_in, (void*)hub_id, (void*)bits, (void*)hub_dir[0], (void*)hub_dir[1],
                   (void*)bits_dir[0], (void*)bits_dir[1], (void*)arc_cn, (void*)h2_off, (void*)h2_v, (void*)h2_c,
                   (void*)h2_did, (void*)h2_dense, (void*)hr_id, (void*)hr})
-    pool_give(device, p, idle);
+    if (!in_slab(*this, p)) pool_give(device, p, idle);
   for (auto& kv : cnt_tables) pool_give(device, kv.second, idle);
   for (auto& kv : chain_tables) pool_give(device, kv.second, idle);
+  pool_give(device, slab, idle);
   (void)hipSetDevice(prev);
 }
 
@@ -4303,9 +4304,27 @@ void upload_graph(Context& c, const Graph& g, DeviceGraph& dg) {
   dg.V = g.V;
   dg.A = g.arcs();
   dg.symmetric = g.symmetric;
+  // a small graph's arrays go out in one copy of the slab (flush); those put
+  // after it each in its own
+  std::vector<char> image;
+  bool flushed = false;
+  auto put = [&](void* d, const void* h, uint64_t bytes) {
+    if (!bytes) return;
+    if (flushed || !in_slab(dg, d)) {
+      HIPCHECK(hipMemcpy(d, h, bytes, hipMemcpyHostToDevice));
+      return;
+    }
+    image.reserve(kSlab);
+    image.resize(dg.slab_used);
+    std::memcpy(image.data() + ((char*)d - dg.slab), h, bytes);
+  };
+  auto flush = [&] {
+    if (!flushed && !image.empty()) HIPCHECK(hipMemcpy(dg.slab, image.data(), image.size(), hipMemcpyHostToDevice));
+    flushed = true;
+  };
   auto up = [&](uint32_t*& d, const std::vector<uint32_t>& h) {
     graph_alloc(dg, d, h.size());
-    HIPCHECK(hipMemcpy(d, h.data(), h.size() * 4, hipMemcpyHostToDevice));
+    put(d, h.data(), h.size() * 4);
   };
   up(dg.off_out, g.out_off);
   up(dg.adj_out, g.out_adj);
@@ -4317,53 +4336,44 @@ void upload_graph(Context& c, const Graph& g, DeviceGraph& dg) {
     up(dg.off_in, g.in_off);
     up(dg.adj_in, g.in_adj);
   }
-  auto entry_sigs = [&](uint2*& d, const uint32_t* adj, uint64_t A) {
-    graph_alloc(dg, d, A);
-    if (!A) return;
-    hipLaunchKernelGGL(k_entry_sigs, dim3(grid_for(A, 256, (uint32_t)c.cus * 32)), dim3(256), 0, c.stream, adj, A,
-                       (const uint2*)dg.sig, d);
-    HIPCHECK(hipGetLastError());
-  };
-  entry_sigs(dg.nsig_out, dg.adj_out, g.out_adj.size());
-  if (g.symmetric) dg.nsig_in = dg.nsig_out;
-  else entry_sigs(dg.nsig_in, dg.adj_in, g.in_adj.size());
-  // longest out-list, self-loops and wedges
-  unsigned long long *d_stats = nullptr, stats[3];
-  dev_alloc(d_stats, 3);
-  HIPCHECK(hipMemsetAsync(d_stats, 0, sizeof(stats), c.stream));
-  hipLaunchKernelGGL(k_list_stats, dim3(grid_for(g.V, 256, (uint32_t)c.cus * 8)), dim3(256), 0, c.stream, dg.off_out,
-                     dg.adj_out, g.V, d_stats);
-  HIPCHECK(hipGetLastError());
-  HIPCHECK(hipMemcpyAsync(stats, d_stats, sizeof(stats), hipMemcpyDeviceToHost, c.stream));
-  HIPCHECK(hipStreamSynchronize(c.stream));
-  dev_free(d_stats);
-  dg.max_deg = (uint32_t)stats[0];
-  dg.loops = stats[1];
-  const uint64_t wedges = stats[2];
   // Hub bitmaps: the lowest power-of-two degree threshold (>= 32) whose
   // bitmaps fit the budget (1/32 of free HBM, at most 4 GiB); a directed
   // graph's out-lists and in-lists have half of it each.
   if (g.V >= 64) {
-    const uint64_t fr = device_free_bytes(c.device);
-    uint64_t cap = std::min<uint64_t>(fr / 32, 4ull << 30);
-    // CUTS_HUB_BITMAP_MB replaces the cap (at most half of free HBM)
-    if (const char* e = std::getenv("CUTS_HUB_BITMAP_MB"))
-      cap = std::min<uint64_t>((uint64_t)std::strtoull(e, nullptr, 10) << 20, fr / 2);
+    const char* mb = std::getenv("CUTS_HUB_BITMAP_MB");
+    auto budget = [&] {
+      const uint64_t fr = device_free_bytes(c.device);
+      // CUTS_HUB_BITMAP_MB replaces the cap (at most half of free HBM)
+      const uint64_t cap = mb ? std::min<uint64_t>((uint64_t)std::strtoull(mb, nullptr, 10) << 20, fr / 2)
+                              : std::min<uint64_t>(fr / 32, 4ull << 30);
+      return g.symmetric ? cap : cap / 2;
+    };
     const uint32_t words = (g.V + 63) / 64;
     uint32_t tmin = 32;
     // CUTS_HUB_MIN_DEG raises the starting threshold (fewer, larger hubs:
     // a bitmap set small enough to stay in L2)
     if (const char* e = std::getenv("CUTS_HUB_MIN_DEG"))
       tmin = std::max<uint32_t>(tmin, (uint32_t)std::strtoul(e, nullptr, 10));
-    // the rows of one side's lists; returns their number, t the threshold
-    auto build = [&](const std::vector<uint32_t>& off, const uint32_t* d_off, const uint32_t* d_adj, uint64_t most,
-                     int32_t*& hub_id, uint64_t*& bits, uint32_t& t) {
+    // the rows of one side's lists; returns their number, t the threshold.
+    // Rows of at most kSlabMost bytes are set here and go out with the lists:
+    // a copy, a clear and a launch of their own took a small graph longer than
+    // all of its lists
+    auto build = [&](const std::vector<uint32_t>& off, const std::vector<uint32_t>& adj, const uint32_t* d_off,
+                     const uint32_t* d_adj, int32_t*& hub_id, uint64_t*& bits, uint32_t& t) {
       std::vector<uint32_t> deg(g.V);
       for (uint32_t v = 0; v < g.V; ++v) deg[v] = off[v + 1] - off[v];
-      for (t = tmin; t <= (1u << 30); t *= 2) {
-        uint64_t nh = 0;
+      uint64_t nh = 0;
+      auto count = [&] {
+        nh = 0;
         for (uint32_t d : deg) nh += d >= t;
-        if (nh * words * 8 <= most) break;
+      };
+      t = tmin;
+      count();
+      const bool here = !mb && (uint64_t)g.V * 4 <= kSlabMost && nh * words * 8 <= kSlabMost;
+      if (!here) {
+        const uint64_t most = budget();
+        for (; nh * words * 8 > most && t < (1u << 30); count()) t *= 2;
+        if (nh * words * 8 > most) t *= 2;
       }
       std::vector<uint32_t> hubs;
       std::vector<int32_t> hid(g.V, -1);
@@ -4374,29 +4384,40 @@ void upload_graph(Context& c, const Graph& g, DeviceGraph& dg) {
         }
       if (hubs.empty()) return (uint32_t)0;
       graph_alloc(dg, hub_id, g.V);
-      HIPCHECK(hipMemcpy(hub_id, hid.data(), g.V * 4, hipMemcpyHostToDevice));
+      put(hub_id, hid.data(), (uint64_t)g.V * 4);
       graph_alloc(dg, bits, (uint64_t)hubs.size() * words);
-      HIPCHECK(hipMemset(bits, 0, (uint64_t)hubs.size() * words * 8));
+      if (here) {
+        std::vector<uint64_t> b(hubs.size() * words);
+        for (uint64_t r = 0; r < hubs.size(); ++r)
+          for (uint32_t i = off[hubs[r]]; i < off[hubs[r] + 1]; ++i) b[r * words + (adj[i] >> 6)] |= 1ull << (adj[i] & 63);
+        put(bits, b.data(), b.size() * 8);
+        return (uint32_t)hubs.size();
+      }
+      flush();
+      HIPCHECK(hipMemsetAsync(bits, 0, (uint64_t)hubs.size() * words * 8, c.stream));
       uint32_t* dh = nullptr;
-      dev_alloc(dh, hubs.size());
+      if (hubs.size() * 4 <= kSlabMost) graph_alloc(dg, dh, hubs.size());
+      else dev_alloc(dh, hubs.size());
       HIPCHECK(hipMemcpy(dh, hubs.data(), hubs.size() * 4, hipMemcpyHostToDevice));
       hipLaunchKernelGGL(k_hub_bits, dim3((uint32_t)std::min<size_t>(hubs.size(), 65535)), dim3(256), 0, c.stream,
                          d_off, d_adj, dh, (uint32_t)hubs.size(), words, bits);
       HIPCHECK(hipGetLastError());
-      HIPCHECK(hipStreamSynchronize(c.stream));
-      dev_free(dh);
+      if (!in_slab(dg, dh)) {
+        HIPCHECK(hipStreamSynchronize(c.stream));
+        dev_free(dh);
+      }
       return (uint32_t)hubs.size();
     };
     uint32_t t = 0;
     if (g.symmetric) {
-      dg.hubs = build(g.out_off, dg.off_out, dg.adj_out, cap, dg.hub_id, dg.bits, t);
+      dg.hubs = build(g.out_off, g.out_adj, dg.off_out, dg.adj_out, dg.hub_id, dg.bits, t);
       if (dg.hubs) {
         dg.words = words;
         dg.hub_min_deg = t;
       }
     } else {
-      const uint32_t o = build(g.out_off, dg.off_out, dg.adj_out, cap / 2, dg.hub_dir[0], dg.bits_dir[0], t);
-      const uint32_t i = build(g.in_off, dg.off_in, dg.adj_in, cap / 2, dg.hub_dir[1], dg.bits_dir[1], t);
+      const uint32_t o = build(g.out_off, g.out_adj, dg.off_out, dg.adj_out, dg.hub_dir[0], dg.bits_dir[0], t);
+      const uint32_t i = build(g.in_off, g.in_adj, dg.off_in, dg.adj_in, dg.hub_dir[1], dg.bits_dir[1], t);
       dg.words = words;
       // the kernels ask for both sides or neither: a side without hubs has a
       // table of none (and no row that could be read)
@@ -4404,12 +4425,36 @@ void upload_graph(Context& c, const Graph& g, DeviceGraph& dg) {
         if ((o || i) && !(d ? i : o)) {
           const std::vector<int32_t> none(g.V, -1);
           graph_alloc(dg, dg.hub_dir[d], g.V);
-          HIPCHECK(hipMemcpy(dg.hub_dir[d], none.data(), (uint64_t)g.V * 4, hipMemcpyHostToDevice));
+          put(dg.hub_dir[d], none.data(), (uint64_t)g.V * 4);
+          const uint64_t zero = 0;
           graph_alloc(dg, dg.bits_dir[d], 1);
-          HIPCHECK(hipMemset(dg.bits_dir[d], 0, 8));
+          put(dg.bits_dir[d], &zero, 8);
         }
     }
   }
+  flush();
+  auto entry_sigs = [&](uint2*& d, const uint32_t* adj, uint64_t A) {
+    graph_alloc(dg, d, A);
+    if (!A) return;
+    hipLaunchKernelGGL(k_entry_sigs, dim3(grid_for(A, 256, (uint32_t)c.cus * 32)), dim3(256), 0, c.stream, adj, A,
+                       (const uint2*)dg.sig, d);
+    HIPCHECK(hipGetLastError());
+  };
+  entry_sigs(dg.nsig_out, dg.adj_out, g.out_adj.size());
+  if (g.symmetric) dg.nsig_in = dg.nsig_out;
+  else entry_sigs(dg.nsig_in, dg.adj_in, g.in_adj.size());
+  // longest out-list, self-loops and wedges, by way of the run's counters
+  unsigned long long* const d_stats = c.counters + kCounterWords;
+  volatile uint64_t* const stats = c.host_pinned;
+  HIPCHECK(hipMemsetAsync(d_stats, 0, 3 * sizeof(*d_stats), c.stream));
+  hipLaunchKernelGGL(k_list_stats, dim3(grid_for(g.V, 256, (uint32_t)c.cus * 8)), dim3(256), 0, c.stream, dg.off_out,
+                     dg.adj_out, g.V, d_stats);
+  HIPCHECK(hipGetLastError());
+  HIPCHECK(hipMemcpyAsync(c.host_pinned, d_stats, 3 * sizeof(*d_stats), hipMemcpyDeviceToHost, c.stream));
+  HIPCHECK(hipStreamSynchronize(c.stream));
+  dg.max_deg = (uint32_t)stats[0];
+  dg.loops = stats[1];
+  const uint64_t wedges = stats[2];
   // Per-arc common-neighbour counts (symmetric loop-free graphs): 4 bytes
   // per arc while they fit 1/16 of free HBM, filled below from the index or
   // the hub rows.
@@ -4527,6 +4572,8 @@ void upload_graph(Context& c, const Graph& g, DeviceGraph& dg) {
     HIPCHECK(hipGetLastError());
     HIPCHECK(hipStreamSynchronize(c.stream));
     dg.arc_cn_build_s = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
+  } else {
+    HIPCHECK(hipStreamSynchronize(c.stream));  // the graph is there for every stream
   }
 }
 
