@@ -4417,8 +4417,11 @@ void upload_graph(Context& c, const Graph& g, DeviceGraph& dg) {
       }
     } else {
       const uint32_t o = build(g.out_off, g.out_adj, dg.off_out, dg.adj_out, dg.hub_dir[0], dg.bits_dir[0], t);
+      const uint32_t to = t;
       const uint32_t i = build(g.in_off, g.in_adj, dg.off_in, dg.adj_in, dg.hub_dir[1], dg.bits_dir[1], t);
       dg.words = words;
+      dg.hubs = o + i;
+      if (dg.hubs) dg.hub_min_deg = !i || (o && to < t) ? to : t;
       // the kernels ask for both sides or neither: a side without hubs has a
       // table of none (and no row that could be read)
       for (int d = 0; d < 2; ++d)

@@ -104,7 +104,8 @@ typedef struct {
   uint64_t arcs;
   int symmetric;
   uint64_t self_loops;          /* vertices u with u in out(u) */
-  uint32_t hubs, hub_min_deg;   /* hub bitmap rows and their degree threshold */
+  uint32_t hubs, hub_min_deg;   /* hub bitmap rows and their degree threshold (directed
+                                   graphs: of out-lists and in-lists, the lower one) */
   uint64_t two_hop_entries;     /* 0: no two-hop index */
   uint32_t two_hop_dense_rows;
   int arc_common;               /* 1: per-arc common-neighbour counts present */
