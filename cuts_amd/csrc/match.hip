@@ -3864,9 +3864,8 @@ struct Matcher {
     // position k-3 (no rows of level k-3 are stored)
     chain_fused = chain && g.h2_off && kp.ch_ta <= 2;
     // a collapsing pair level is counted inside the expansion of position
-    // k-4 (no rows of level k-4 are stored); with a deadline, in the planner
-    // of level k-3 instead (the rolled-back counters are those of 0..2)
-    collapse_fused = pair && kp.pr_collapse && pair_cab_known() && k >= 5 && !(o.time_limit_ms > 0);
+    // k-4 (no rows of level k-4 are stored)
+    collapse_fused = pair && kp.pr_collapse && pair_cab_known() && k >= 5;
     // the fused chain with position k-3's candidates shared by siblings
     sib = chain_fused && kp.ch_sib && !(o.flags & 1024u);
     get_tables();
