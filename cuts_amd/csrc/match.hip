@@ -1223,7 +1223,10 @@ __global__ __launch_bounds__(BLOCK) void k_closed_form(GView g, KPlan P, const u
 
 // Degree-threshold table: tbl[u] = |{x in N(u) : deg(x) >= thr}|, one wave per
 // vertex.  Degrees from the list entries' signatures (of a symmetric graph),
-// read in order.
+// read in order.  R-MAT 20, 31 M entries: 0.47 ms, bound by each wave's chain
+// of loads and by the blocks that hold the hubs; 16 lanes per vertex a grid
+// apart and long lists by whole blocks took 0.31, not worth their code for a
+// table built once.
 static __global__ __launch_bounds__(BLOCK) void k_cnt_table(GView g, uint32_t thr, uint32_t* __restrict__ tbl) {
   const uint32_t lane = threadIdx.x & 63;
   const uint64_t nw = (uint64_t)gridDim.x * (BLOCK / 64);
@@ -1402,8 +1405,9 @@ __global__ __launch_bounds__(BLOCK, L <= 4 ? 5 : L <= 5 ? 4 : 1) void k_expand(G
   // rows of the first NJP constraints.  An item then takes its prefix from
   // LDS by 32-bit searches and reads instead of repeating the prefix's loads
   // and address arithmetic, which bound the kernel by instruction issue
-  // (a directed last level of 1.3e10 items: 111 -> 56.8 ms).  Tiles
-  // of more prefixes (short lists) keep the offsets alone, or nothing.
+  // (a directed last level of 1.3e10 items: 111 -> 79.6 ms; five waves per
+  // SIMD took it to 68.1, constraints of one direction together to 56.8).
+  // Tiles of more prefixes (short lists) keep the offsets alone, or nothing.
   constexpr uint32_t SP = 256, NJP = 3;
   constexpr uint32_t STAGE_WORDS = (SP + 1) + (L + 3 + NJP + (MODE == M_FUSED ? 1 : 0)) * SP;
   constexpr uint32_t RAW_WORDS = STAGE_WORDS > 2 * (LDS_OFF + 1) ? STAGE_WORDS : 2 * (LDS_OFF + 1);
@@ -2898,13 +2902,15 @@ struct Matcher {
     }
     return kp.pr_a == kp.pr_b || pair_cab_known();
   }
-  // a pair counted from whole prefixes whose intersection only the per-arc
-  // table holds (no two-hop index, owners adjacent in the query) is left to
-  // the expansion of position k-2.  Not for its speed: from whole prefixes
-  // the score order of the 5-cycle + chord + 2 tails query on R-MAT 20 takes
-  // 2.9 ms instead of 97 (the learned order 1.3), and the learned order is
-  // held to a tenth of the score order's time there
-  // (tests/test_learned.py, training on R-MAT 18 and judging on R-MAT 20)
+  // a pair on a graph without the two-hop index but with the per-arc table,
+  // its owners adjacent in the query, is left to the expansion of position
+  // k-2, whatever its thresholds.  Not for its speed: from whole prefixes the
+  // score order of the 5-cycle + chord + 2 tails query on R-MAT 20 takes 2.9 ms
+  // instead of 83 to 97 (the learned order 1.3), and the learned order is held
+  // to a tenth of the score order's time there (tests/test_learned.py,
+  // training on R-MAT 18 and judging on R-MAT 20).  CUTS_FLAG_NO_ARC_COMMON,
+  // and a graph whose per-arc table does not fit, thus open the route, over
+  // stored rows
   bool tail_left() const { return kp.tl_kind == 1 && kp.pr_a != kp.pr_b && !g.h2_off && g.arc_cn && kp.pr_adj; }
   // the tables of the whole-prefix tail are none or with the graph already
   bool tail_tables_held() const {

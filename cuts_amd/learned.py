@@ -236,7 +236,10 @@ def connected_subsets(k: int, adj: List[int]) -> List[int]:
 class Engine:
     """What the matcher counts in closed form for a given order
     (make_kplan and Matcher::run in cuts_amd/csrc/match.hip), so that an
-    order is costed by the levels the engine actually expands:
+    order is costed by the levels the engine expands.  The whole-prefix tails
+    (tl_kind, a leaf or a 2-edge tail on position k-3 itself or on an owner of
+    a doubly joined position k-2) are not in it: their orders are costed as if
+    position k-2 were expanded, so they are rated too dear:
 
     * symmetric data graph, last vertex with one earlier neighbour: the last
       level is counted in closed form inside the expansion of position k-2;
