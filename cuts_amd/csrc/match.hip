@@ -935,21 +935,23 @@ __device__ __forceinline__ void publish_rows(uint64_t* publish, uint64_t rows, u
 // alone changes: the other threads may index tiles that nothing then takes.
 // The work of a counting level beyond the cap is added all the same, as the
 // readback does, and that of the counting levels after it is not: the run has
-// ended there.  publish (a writing level): a level without tiles has no
+// ended there (from bit 2 of *status, the number of those levels).  publish (a writing level): a level without tiles has no
 // expansion block to publish its size; one withheld tells the host its work
-// (from bit 2 of the status word) and that of the levels before it (in place
-// of the rows), so that no readback follows.
+// (from bit 3 of the status word) and that of the levels before it (in place
+// of the rows), so that no readback follows.  Bit 2: a counting level of an
+// earlier trunk went beyond the cap (*ended, the status of counting levels).
 static __device__ __forceinline__ bool claim_work(bool fits, uint64_t W, uint64_t nt, unsigned long long* dyn,
                                            unsigned long long* status, unsigned long long* work, uint64_t work_cap,
                                            uint64_t* publish) {
   const unsigned long long before = *work;
+  const unsigned long long* const ended = work - 1;
   const bool over = W > work_cap || before > work_cap - W;
   const bool go = fits && !over;
   dyn[0] = go ? W : 0ull;
   dyn[1] = go ? nt : 0ull;
   if (go || (over && !publish && !(*status & 2ull))) *work = before + W;
-  if (!go) *status |= over ? 2ull : 1ull;
-  if (publish && !go) publish_rows(publish, before, (over ? 2ull : 1ull) | W << 2);
+  if (!go) *status = (*status | (over ? 2ull : 1ull)) + (over && !publish && (*status & 2ull) ? 4ull : 0ull);
+  if (publish && !go) publish_rows(publish, before, (over ? 2ull : 1ull) | (*ended & 2ull) << 1 | W << 3);
   else if (publish && W == 0) publish_rows(publish, 0u, 0ull);
   return go;
 }
@@ -2047,7 +2049,7 @@ __global__ __launch_bounds__(BLOCK, L <= 4 ? 5 : L <= 5 ? 4 : 1) void k_expand(G
 // and a candidate v adds, with inv = [v in N(u), deg v >= ta]:
 //   inv (-cnt_tb(v) + [deg u >= tb] + sum_{i in Dold} [r_i ~ v])
 //   + [deg v >= tb] sum_{j in inu_old} [v ~ r_j] - [deg v >= tb] |N(u) & N(v)|
-// (chain_sib_item); na = na_old - inv.  Stored per row: base (int64), na_old,
+// (k_chain_sib); na = na_old - inv.  Stored per row: base (int64), na_old,
 // and the masks (inu_old in bits 0..14, Dold in 15..29, [deg u >= tb] in 30)
 // in pb, the start of the parent's block in rstart, its length in minlen.
 template <int L>
@@ -3038,13 +3040,17 @@ struct Matcher {
   // point and CUTS_FLAG_SYNC_LEVELS.
   // A work cap is tested on the device too (claim_work), so a level beyond it
   // is never expanded: a writing level tells the host, which ends the run
-  // there; a counting level ends it too (capped_at_end).  All levels after one
-  // that the host counted are read back, and so are all of a run of several
-  // trunks.  A capped run that stays below its cap thus has the launches and
-  // readbacks of one without: a 6-vertex query of 4.1 M candidates on R-MAT
-  // 20, more than 0.185 ms with its levels read back, takes 0.142.
+  // there; a counting level ends it too, which the host sees at the end of the
+  // run (capped_at_end) or with the first writing level of the next trunk.  All
+  // levels after one that the host counted are read back.  A capped run that
+  // stays below its cap thus has the launches and readbacks of one without: a
+  // 6-vertex query of 4.1 M candidates on R-MAT 20, more than 0.185 ms with
+  // its levels read back, takes 0.142; a 4-clique on 4,096 vertices in 16
+  // trunks ends at caps of 2^9 and 2^12 in 66 and 91 us (repeated: 114, 138).
   bool no_spec = false;
   bool spec_overflow = false;
+  bool wrote_first = false;     // position 1 is a writing level
+  bool trunk_capped = false;    // ended by a counting level of the trunk before
   bool dev_work = false;        // candidates counted on the device and not yet in r.work
   uint64_t dev_taken = 0;       // of the device's count, what r.work holds
   uint64_t dev_before = ~0ull;  // the device's count before the level being read back, where it told
@@ -3070,7 +3076,7 @@ struct Matcher {
   }
   bool speculate() const {
     return !no_spec && !prof && !has_deadline && !arena && !(o.flags & 8192u) &&
-           !(o.max_work && (r.work || o.trunks > 1));
+           !(o.max_work && r.work);
   }
   // Word w of the coherent host words once the stream has drained: true
   // when a kernel published it (it holds ~0 until then).  Polling the word
@@ -3332,6 +3338,7 @@ struct Matcher {
                   uint64_t& W, const unsigned long long* dn = nullptr) {
     if (!small) scan_launch(in, n);
     dev_work = true;
+    if (L == 1 && mode == M_WRITE) wrote_first = true;
     LevelBuf& out = lv[L];
     uint64_t row_cap = ~0ull;
     const bool want_parent = (chain && !chain_fused && mode == M_WRITE && L == k - 3) ||
@@ -3436,10 +3443,13 @@ struct Matcher {
       if (dn && (got[1] & 3ull)) return true;
       if (got[1] & 3ull) {
         r.chunks--;
-        W = got[1] >> 2;
+        W = got[1] >> 3;
         if (got[1] & 2ull) {
-          // the work cap: the run ends as add_work ends it
-          r.work += W;
+          // the work cap: the run ends as add_work ends it, or has ended with
+          // the last level of the trunk before
+          trunk_capped = (got[1] & 4ull) != 0;
+          if (trunk_capped) r.chunks--;
+          else r.work += W;
           r.work_capped = 1;
           aborted = true;
           return true;
@@ -3944,6 +3954,8 @@ struct Matcher {
         has_deadline = true;
         deadline = t_start + std::chrono::microseconds((int64_t)(o.time_limit_ms * 1000.0));
       }
+      // where the last finished trunk began, and the level sizes before it
+      uint64_t last_level[kMaxQuery] = {0}, last_trunk = 0;
       for (uint64_t s = 0; s < n0; s += ts) {
         // snapshot so that a trunk interrupted by the deadline can be undone
         uint64_t snap_level[kMaxQuery];
@@ -3960,9 +3972,12 @@ struct Matcher {
             HIPCHECK(hipMemcpyAsync(ctr + kSlot0, ctr + kCounterWords + kSlot0, (kTile0 - kSlot0) * 8,
                                     hipMemcpyDeviceToDevice, c.stream));
           }
-          std::memcpy(r.level, snap_level, sizeof(snap_level));
+          std::memcpy(r.level, trunk_capped ? last_level : snap_level, sizeof(snap_level));
+          if (trunk_capped) r.roots_done = s - ts;
           break;
         }
+        std::memcpy(last_level, snap_level, sizeof(snap_level));
+        last_trunk = s;
         r.roots_done = std::min(n0, s + ts);
       }
       if (aborted || r.roots_done < n0) r.complete = 0;
@@ -3984,10 +3999,16 @@ struct Matcher {
       const bool host_work = r.work != 0;
       r.work += hp[13] - dev_taken;
       const bool void_counts = aborted && !has_deadline;  // ended by the work cap on the host
-      // a run stopped by its work cap at a counting level: one path down the
-      // levels, all of it counted on the device
-      const bool capped_at_end = hp[12] == 2ull && !host_work && !chained_mask && o.trunks <= 1;
-      spec_overflow = hp[12] != 0 && !capped_at_end;
+      // a run stopped by its work cap at a counting level of its last trunk: one
+      // path down the levels, all of it counted on the device (an earlier
+      // trunk's is seen by the writing level that begins the next one); or of
+      // any trunk, where each is one counting level: as many were withheld as
+      // trunks followed
+      const bool one_level = trunks > 1 && !wrote_first;
+      const bool capped_at_end = (hp[12] & 3ull) == 2ull && !aborted && !host_work && !chained_mask &&
+                                 (!one_level || r.chunks == (n0 + ts - 1) / ts);
+      const uint64_t after = one_level ? hp[12] >> 2 : 0;
+      spec_overflow = hp[12] != 0 && !capped_at_end && !trunk_capped;
       if (r.work_capped && chained_mask) spec_overflow = true;
       // sizes of the levels whose successor read them on the device (level
       // 0's: every root processed in one trunk)
@@ -4017,10 +4038,11 @@ struct Matcher {
         aborted = true;
         r.work_capped = 1;
         r.complete = 0;
-        r.roots_done = 0;
+        r.roots_done = last_trunk - after * ts;
         r.last_root = 0;
-        r.chunks--;
-        for (uint32_t l = 1; l < k; ++l) r.level[l] = 0;
+        last_root_read = false;
+        r.chunks -= (uint32_t)after + 1u;
+        for (uint32_t l = 1; l < k; ++l) r.level[l] = last_level[l];
       }
       if (r.work_capped) r.count = 0;
     }

@@ -63,3 +63,22 @@ def test_remembered_sizes_with_a_smaller_budget():
         want = outcome(dg.ctx.match(dg, plan, flags=flags | F.FLAG_SYNC_LEVELS))
         for budget in (0, 2048, 0, 2048):
             assert outcome(dg.ctx.match(dg, plan, flags=flags, budget=budget)) == want
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("flags", [0, F.FLAG_NO_PAIR | F.FLAG_NO_CHAIN])
+@pytest.mark.parametrize("name", SHAPES)
+def test_the_cap_in_every_trunk(name, flags):
+    """The cap a candidate below, at and above the work of each number of
+    trunks: the run ends at the last level of one trunk, or in the next."""
+    edges, order = SHAPES[name]
+    dg = F.Context().upload(graph(60, 300, seed=len(order)))
+    plan = F.Plan(F.Graph.from_edges(len(order), edges), order)
+    for trunks in (2, 5):
+        size = -(-60 // trunks)
+        ends = [dg.ctx.match(dg, plan, flags=flags | F.FLAG_SYNC_LEVELS, roots=(0, size * t, 1)).work
+                for t in range(1, trunks + 1)]
+        for cap in sorted({e + d for e in ends for d in (-1, 0, 1)} - {-1, 0}):
+            runs = [dg.ctx.match(dg, plan, flags=flags | f, max_work=cap, trunks=trunks) for f in (F.FLAG_SYNC_LEVELS, 0, 0)]
+            want, *got = [outcome(r) + (r.chunks,) for r in runs]
+            assert got == [want, want], (cap, ends, trunks)
