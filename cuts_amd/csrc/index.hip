@@ -258,11 +258,6 @@ struct Temp {
   Temp& operator=(const Temp&) = delete;
 };
 
-// Groups of 64 rows whose masks are held at once (512 MiB, at least one).
-uint32_t groups_at_once(uint32_t groups, uint32_t V) {
-  return (uint32_t)std::min<uint64_t>(groups, std::max<uint64_t>(1, (512ull << 20) / (8ull * V)));
-}
-
 // One launch of k_rows<MODE> per batch of groups.  fresh: build the masks
 // (false: a single batch's are still there).
 template <int MODE>
@@ -303,7 +298,7 @@ void build_hub_rows(Context& c, DeviceGraph& dg, const std::vector<uint32_t>& hu
   RowArgs a = row_args(dg);
   a.nrows = (uint32_t)hubs.size();
   a.out = dg.hr;
-  const uint32_t at_once = groups_at_once((a.nrows + 63) / 64, a.V);
+  const uint32_t at_once = mask_groups((a.nrows + 63) / 64, a.V, device_free_bytes(c.device));
   Temp<uint32_t> rowv(c, dg, hubs.size());
   Temp<unsigned long long> mask(c, dg, (uint64_t)at_once * a.V);
   HIPCHECK(hipMemcpy(rowv.p, hubs.data(), hubs.size() * 4, hipMemcpyHostToDevice));
@@ -315,7 +310,7 @@ void build_hub_rows(Context& c, DeviceGraph& dg, const std::vector<uint32_t>& hu
 void build_two_hop_device(Context& c, DeviceGraph& dg, std::vector<uint64_t>& off,
                           const std::function<std::vector<uint32_t>(const std::vector<uint64_t>&)>& dense_rows) {
   RowArgs a = row_args(dg);
-  const uint32_t V = a.V, groups = (V + 63) / 64, at_once = groups_at_once(groups, V);
+  const uint32_t V = a.V, groups = (V + 63) / 64, at_once = mask_groups(groups, V, device_free_bytes(c.device));
   a.nrows = V;
   Temp<unsigned long long> mask(c, dg, (uint64_t)at_once * V), total(c, dg, V);
   Temp<uint32_t> tcnt(c, dg, (uint64_t)V * a.ntiles);

@@ -69,6 +69,21 @@ void dev_alloc(ScratchArena* a, T*& p, uint64_t n) {
   p = (T*)a->carve(m * sizeof(T));
 }
 
+// The index builds' own memory beside what they build, of `free` bytes: the
+// masks of one group of 64 rows are 8V bytes, those of as many groups are held
+// at once as fit 512 MiB and a sixteenth of it (one at least; with fewer than
+// all, the write pass builds them again).
+inline uint32_t mask_groups(uint32_t groups, uint32_t V, uint64_t free) {
+  const uint64_t bytes = std::min<uint64_t>(512ull << 20, free / 16);
+  return (uint32_t)std::min<uint64_t>(groups, std::max<uint64_t>(1, bytes / (8ull * V)));
+}
+// The two-hop index is built on the device up to 2^17 vertices, where its
+// counts per row and tile of 256 columns (V^2/64 bytes, 256 MiB at most) fit
+// an eighth of the free memory; else on the host, which needs only the index.
+inline bool two_hop_on_device(uint32_t V, uint64_t free) {
+  return V <= (1u << 17) && (uint64_t)V * ((V + 255) / 256) * 4 <= free / 8;
+}
+
 // Makes sure level buffer `lv` can hold `rows` rows of `words` words plus
 // the planning arrays for them.
 inline void ensure_rows(ScratchArena* ar, LevelBuf& b, uint64_t rows, uint32_t words) {

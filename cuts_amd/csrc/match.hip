@@ -4492,7 +4492,7 @@ void upload_graph(Context& c, const Graph& g, DeviceGraph& dg) {
     const uint64_t fr = device_free_bytes(c.device);
     if (dg.A * 4 <= fr / 16) graph_alloc(dg, dg.arc_cn, dg.A);
   }
-  // Two-hop index: built on the host when the wedges (ordered neighbour
+  // Two-hop index (two_hop_on_device: where): built when the wedges (ordered neighbour
   // pairs of every vertex, an upper bound on the entries) fit 1/16 of free
   // HBM at 8 bytes each, at most 2^28 of them, on graphs of at most 2^25
   // vertices.
@@ -4530,7 +4530,7 @@ void upload_graph(Context& c, const Graph& g, DeviceGraph& dg) {
         return cand;
       };
       std::vector<uint64_t> off((size_t)V + 1, 0);
-      if (V <= (1u << 17)) {
+      if (two_hop_on_device(V, fr)) {
         dg.h2_on_gpu = true;
         build_two_hop_device(c, dg, off, dense_rows);
       } else {

@@ -5,8 +5,9 @@
 // 85 ms for memory (R-MAT 18, 3.3 GB).  Freed blocks of at least kKeepMin
 // bytes stay here, up to 1/32 of the device's memory, while a context of the
 // device exists and until pool_trim frees them; an allocation takes one that
-// is at most a quarter larger than asked.  They count as free memory (device_free_bytes), and every
-// allocation of the library that fails gives them back and tries again.
+// is at most a quarter larger than asked.  They count as free memory
+// (device_free_bytes), and every allocation of the library that fails gives
+// them back and tries again.
 #include <map>
 #include <mutex>
 #include <unordered_map>

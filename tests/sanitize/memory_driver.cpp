@@ -195,6 +195,22 @@ static void threads() {
   CHECK(d.used == 0);
 }
 
+// What an index build takes for itself, on devices with little and much free
+// memory: never more than the bounds that its comment gives, but one group.
+static void index_builds() {
+  for (uint64_t free : {0 * MB, 64 * MB, 600 * MB, 2048 * MB, 294912 * MB})
+    for (uint32_t V : {2u, 255u, 257u, 36692u, 65536u, 131072u, 131073u, 1u << 20, 1u << 25}) {
+      const uint32_t groups = (V + 63) / 64, at_once = mask_groups(groups, V, free);
+      CHECK(at_once >= 1 && at_once <= groups);
+      CHECK(at_once == 1 || 8ull * V * at_once <= std::min<uint64_t>(512 * MB, free / 16));
+      CHECK(at_once == groups || 8ull * V * (at_once + 1) > std::min<uint64_t>(512 * MB, free / 16));
+      const uint64_t counts = (uint64_t)V * ((V + 255) / 256) * 4;
+      CHECK(two_hop_on_device(V, free) == (V <= 131072 && counts <= free / 8));
+    }
+  CHECK(mask_groups(2048, 131072, 288ull << 30) == 512 && two_hop_on_device(131072, 288ull << 30));
+  CHECK(!two_hop_on_device(131072, 1024 * MB));
+}
+
 int main(int, char** argv) {
   const std::string what = argv[1];
   if (what == "end_of_process") end_of_process();
@@ -203,6 +219,7 @@ int main(int, char** argv) {
   else if (what == "growth_that_fails") growth_that_fails();
   else if (what == "network_that_does_not_fit") network_that_does_not_fit();
   else if (what == "threads") threads();
+  else if (what == "index_builds") index_builds();
   else return 3;
   std::printf("%s ok\n", argv[1]);
   return 0;

@@ -37,6 +37,10 @@ def test_allocation_that_fails_while_another_thread_flushes(driver):
     run(driver, "flushed_by_another", ["flushed_by_another ok"])
 
 
+def test_what_index_builds_take_of_little_memory(driver):
+    run(driver, "index_builds", ["index_builds ok"])
+
+
 def test_blocks_freed_while_a_stream_records(driver):
     run(driver, "given_while_capturing", ["given_while_capturing ok"])
 
